@@ -208,8 +208,8 @@ typedef struct yee2d_desc {
     int32_t pitch;           /* row stride in elements of every (nx, *) array: a multiple of 4, >= ny */
     int32_t polarization;    /* YEE_EZ or YEE_HZ */
     int32_t periodic_x, periodic_y;
-    int32_t rows_per_tile;   /* x rows marched by one wavefront tile (0: 4, balanced over nx) */
-    int32_t lane_columns;    /* y columns per lane: 2 or 4 (0: 2); a tile spans 64 * lane_columns columns */
+    int32_t rows_per_tile;   /* x rows marched by one wavefront tile of the one-step kernels (0: 8, balanced over nx) */
+    int32_t lane_columns;    /* their y columns per lane: 2 or 4 (0: 2); a tile spans 64 * lane_columns columns */
     float* field[2][3];      /* [set][component]: E_z (ez, hx, hy) or H_z (hz, ex, ey) */
     const uint16_t* material;
     const float* table;      /* (n_materials, 4) */
@@ -406,7 +406,9 @@ int32_t yee2d_create(const yee2d_desc* desc, yee_ctx** out);
 
 /*
  * Advance by n_steps steps on `stream` (hipStream_t; 0 = the null stream). Launches only: no allocation, no sync.
- * Whole chunks of graph_steps steps replay a cached HIP graph when graph_steps > 0.
+ * Whole chunks of graph_steps steps replay a cached HIP graph when graph_steps > 0. A single 2D instance whose features
+ * allow it (no poles, TFSF, walls, DFT regions or probes; no step limit) advances several steps per launch, chosen by
+ * the size of the grid and n_steps; the others one step per launch.
  * Replaces coupling/runner.py:174-204 (advance) -> EMPhysics.step (physics/em/__init__.py:163-168).
  */
 int32_t yee_step(yee_ctx* ctx, int64_t n_steps, void* stream);
@@ -433,6 +435,13 @@ int32_t yee_build_graph(yee_ctx* ctx);
 
 /* Replace the descriptor (new buffers or tables); drops cached graphs. */
 int32_t yee2d_update(yee_ctx* ctx, const yee2d_desc* desc);
+
+/*
+ * Performance hint: whether every material is lossless and not PEC (ca = 1 for every id, no magnetic loss, one mu_r).
+ * It chooses between launch shapes that give the same bits; the kernels look at the tables themselves. Default 0;
+ * yee2d_update keeps it. The reference has one kernel form (physics/em/solvers/fdtd_hz_2d_kernels.py:28-155).
+ */
+int32_t yee2d_set_lossless(yee_ctx* ctx, int32_t lossless);
 
 /* The descriptor a single 2D context steps, with the defaults it resolved (rows_per_tile, lane_columns). */
 int32_t yee2d_get_desc(const yee_ctx* ctx, yee2d_desc* out);

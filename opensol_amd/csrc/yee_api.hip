@@ -20,6 +20,8 @@ __global__ void yee2d_step_kernel(yee2d_desc d, yee2d_tile_sets sets, int32_t of
 template <int VEC, bool EDGE, bool LEFT>
 __global__ void yee2d_batch_kernel(const yee2d_desc* __restrict__ descs, const yee2d_tile_sets* __restrict__ sets,
                                    const int32_t* __restrict__ prefix, int32_t n_inst, int32_t offset);
+template <int POL, int VEC, int R, int TV, int TR, int NW>
+__global__ void yee2d_multi_kernel(yee2d_desc d, yee2d_multi_plan plan, int32_t offset, int32_t launch);
 template <int J, bool POLES>
 __global__ void yee3d_step_kernel(yee3d_desc d, int32_t tiles_j, int32_t tiles_k, int32_t tiles, int32_t offset);
 template <int J>
@@ -93,6 +95,8 @@ struct yee_ctx {
     int blocks = 0;        // blocks of the bulk kernel (4 tiles each)
     int edge_blocks = 0;   // blocks of the edge kernel (sets.edge_parts wavefronts per tile, 4 per block)
     yee2d_tile_sets sets{};
+    bool multi = false;    // several steps per launch (yee2d_multi.hip)
+    bool lossless = false; // yee2d_set_lossless
     // 3D
     yee3d_desc d3{};
     int32_t tiles_j3 = 0, tiles_k3 = 0;
@@ -442,8 +446,131 @@ yee2d_tile_sets tile_sets(const yee2d_desc& d, bool batch = false)
     return s;
 }
 
+bool has_walls(const yee2d_desc& d)
+{
+    return d.wall_sign[0] != 0 || d.wall_sign[1] != 0 || d.wall_sign[2] != 0 || d.wall_sign[3] != 0;
+}
+
+// Whether several steps of an instance can share a launch: no feature that reads or writes the state between steps
+// outside the multi-step kernel, and a coefficient table that fits its LDS.
+bool multi_ok(const yee2d_desc& d)
+{
+    const int ids = d.polarization == YEE_EZ ? kMultiIds : kMultiIds / 2;   // H_z keeps two entries an id
+    return d.n_poles == 0 && d.n_tfsf == 0 && !has_walls(d) && d.n_dft == 0 && d.probes.n_probes == 0 &&
+           d.n_materials < ids && d.step_limit == INT64_MAX;
+}
+
+typedef void (*MultiKernel)(yee2d_desc, yee2d_multi_plan, int32_t, int32_t);
+struct MultiShape {
+    int vec, r;             // general windows: 64 * vec columns, waves * r rows
+    int tall_vec, tall_r;   // lean windows of the interior, likewise (tall_r 0: none)
+    int waves;
+    int most;               // steps of a launch: past it the halo leaves too little of a window
+    // time of a launch of t steps (multi_time): fixed + step * t us while its windows fit the chip side by side, and
+    // window_fixed + window_step * t ns more for every further window (the first mostly its loads and stores)
+    float fixed, step, window_fixed, window_step;
+    MultiKernel kernel[2];  // by polarisation
+};
+template <int VEC, int R, int TV, int TR, int NW>
+MultiShape multi_shape(int most, float fixed, float step, float window_fixed, float window_step)
+{
+    return MultiShape{VEC, R, TV, TR, NW, most, fixed, step, window_fixed, window_step,
+                      {yee2d_multi_kernel<YEE_EZ, VEC, R, TV, TR, NW>, yee2d_multi_kernel<YEE_HZ, VEC, R, TV, TR, NW>}};
+}
+// Small windows step fastest while there are few of them, tall ones waste least on their halo. Measured (us a step, E_z,
+// graph replay) at 128^2 / 300^2 / 600^2 / 1200^2 / 4000^2 cells: 64 x 16 windows, 7 steps 1.35 / 2.24 / 5.7 / 18.6 / -;
+// 64 x 32, 7 steps 1.84 / 1.74 / 1.96 / 4.32 / 33.7, 10 steps 1.47 / 1.48 / 2.28 / 4.91 / -; 64 x 64 with a 128 x 64
+// interior, 10 steps - / 2.34 / - / 3.28 / 16.7, 14 steps 2.19 / 1.96 / 2.03 / 2.91 / -. 8192^2: 108 / 65 us
+// a step at 5 / 10 steps, 46 ns a window. The numbers of a shape are fitted to these times.
+const MultiShape kMultiShape[] = {multi_shape<1, 8, 2, 8, 8>(14, 11.0f, 1.25f, 35.0f, 1.1f),
+                                  multi_shape<1, 4, 1, 0, 8>(12, 6.7f, 0.8f, 11.0f, 0.25f),
+                                  multi_shape<1, 2, 1, 0, 8>(7, 4.5f, 0.7f, 7.5f, 0.2f)};
+constexpr int32_t kMultiSideBySide = 400;   // windows that run at once (two blocks of 8 wavefronts a CU, unevenly)
+
+void add_region(yee2d_multi_plan& p, int32_t i0, int32_t i1, int32_t j0, int32_t j1, int32_t rows, int32_t columns)
+{
+    if (i0 >= i1 || j0 >= j1) return;
+    yee2d_multi_region& g = p.region[p.n_regions++];
+    g = yee2d_multi_region{i0, i1, j0, j1, rows, columns, (j1 - j0 + columns - 1) / columns, p.blocks};
+    p.blocks += (i1 - i0 + rows - 1) / rows * g.tiles_j;
+}
+
+// The windows of a launch of `steps` steps: with `tall` the lean windows that fit, halo included, between the CPML
+// layers, and general windows on the frame around them; else general windows everywhere.
+yee2d_multi_plan multi_plan(const yee2d_desc& d, int32_t steps, const MultiShape& shape, bool tall)
+{
+    yee2d_multi_plan p{};
+    p.steps = steps;
+    const int32_t rows = yee2d_multi_rows(steps, shape.waves, shape.r), columns = yee2d_multi_columns(steps, shape.vec);
+    if (tall && shape.tall_r) {
+        const int32_t high = yee2d_multi_rows(steps, shape.waves, shape.tall_r);
+        const int32_t wide = yee2d_multi_columns(steps, shape.tall_vec);
+        const int32_t halo = yee2d_multi_halo(steps, shape.tall_vec);
+        const int32_t x0 = (std::max(d.layer_x_lo, 0) + steps + rows - 1) / rows * rows;
+        // a multiple of tall_vec, so that the lanes of the wide windows start at one
+        const int32_t y0 = yee2d_multi_halo((std::max(d.layer_y_lo, 0) + halo + columns - 1) / columns * columns,
+                                            shape.tall_vec);
+        // a window's last row and column, halo included, lies before the high layers and the grid's last row and column
+        const int32_t x_end = std::min(d.layer_x_hi, d.nx - 1) - steps;
+        const int32_t y_end = std::min(d.layer_y_hi, d.ny - 1) - (64 * shape.tall_vec - halo);
+        const int32_t n = x_end >= x0 ? (x_end - x0) / high : 0;
+        const int32_t m = y_end >= y0 ? (y_end - y0) / wide + 1 : 0;
+        if (n > 0 && m > 0) {
+            const int32_t x1 = x0 + n * high, y1 = y0 + m * wide;
+            p.interior = 1;
+            add_region(p, x0, x1, y0, y1, high, wide);
+            add_region(p, 0, x0, 0, d.ny, rows, columns);
+            add_region(p, x1, d.nx, 0, d.ny, rows, columns);
+            add_region(p, x0, x1, 0, y0, rows, columns);
+            add_region(p, x0, x1, y1, d.ny, rows, columns);
+            return p;
+        }
+    }
+    add_region(p, 0, d.nx, 0, d.ny, rows, columns);
+    return p;
+}
+
+// The estimated time of one launch, in us.
+float multi_time(const yee2d_multi_plan& p, const MultiShape& shape)
+{
+    const float further = 1e-3f * std::max(0, p.blocks - kMultiSideBySide);
+    return shape.fixed + shape.step * p.steps + further * (shape.window_fixed + shape.window_step * p.steps);
+}
+
+// Launches of at most `most` steps each that advance an instance by `count` steps: as few as possible, with the parity
+// of `count` (each launch flips the state set). Launch k of `launches` takes multi_steps(count, launches, k).
+int32_t multi_launches(int32_t count, int32_t most)
+{
+    const int32_t launches = (count + most - 1) / most;
+    return launches + ((launches ^ count) & 1);
+}
+
+int32_t multi_steps(int32_t count, int32_t launches, int32_t k) { return count / launches + (k < count % launches); }
+
+// Tall windows: not for H_z with lossy or PEC materials, whose four coefficients a cell do not fit the registers of a
+// 128 x 64 window (1200^2: 14.5 us a step with them, 4.8 without; lossless 3.6 with them, 4.6 without).
+bool tall_windows(const yee_ctx* ctx) { return ctx->d2.polarization == YEE_EZ || ctx->lossless; }
+
+// Shape and number of launches with the least estimated time for `count` steps.
+void choose_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, int32_t* launches)
+{
+    float best = 0.f;
+    *shape = nullptr;
+    for (const MultiShape& s : kMultiShape)
+        for (int32_t most = 1; most <= std::min(s.most, count); ++most) {
+            const int32_t n = multi_launches(count, most);
+            const float time = n * multi_time(multi_plan(ctx->d2, multi_steps(count, n, 0), s, tall_windows(ctx)), s);
+            if (!*shape || time < best) {
+                best = time;
+                *shape = &s;
+                *launches = n;
+            }
+        }
+}
+
 void set_geometry(yee_ctx* ctx)
 {
+    ctx->multi = multi_ok(ctx->d2);
     const yee2d_desc& d = ctx->d2;
     ctx->sets = tile_sets(d);
     const yee2d_tile_sets& s = ctx->sets;
@@ -545,11 +672,6 @@ BatchAux3D batch_aux_3d(const yee3d_desc* descs, int32_t n)
         a.probes = a.probes || d.probes.n_probes > 0;
     }
     return a;
-}
-
-bool has_walls(const yee2d_desc& d)
-{
-    return d.wall_sign[0] != 0 || d.wall_sign[1] != 0 || d.wall_sign[2] != 0 || d.wall_sign[3] != 0;
 }
 
 // The E_z copy launch (H_z walls act inside the H update).
@@ -672,6 +794,23 @@ int32_t ensure_side(yee_ctx* ctx)
 int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
 {
     if (count <= 0) return YEE_OK;
+    if (ctx->kind == kSingle2D && ctx->multi) {
+        const MultiShape* shape = nullptr;
+        int32_t launches = 0;
+        choose_multi(ctx, count, &shape, &launches);
+        for (int32_t k = 0, offset = 0; k < launches; ++k) {
+            const yee2d_multi_plan plan = multi_plan(ctx->d2, multi_steps(count, launches, k), *shape, tall_windows(ctx));
+            const int blocks = (plan.blocks + 7) / 8 * 8;   // a multiple of the XCDs
+            hipLaunchKernelGGL(shape->kernel[ctx->d2.polarization], dim3(blocks), dim3(64 * shape->waves), 0, stream,
+                               ctx->d2, plan, offset, k);
+            offset += plan.steps;
+        }
+        YEE_HIP(hipGetLastError());
+        hipLaunchKernelGGL(yee_clock_advance, dim3(1), dim3(64), 0, stream, ctx->d2.clock, (int64_t)count,
+                           ctx->d2.step_limit);
+        YEE_HIP(hipGetLastError());
+        return YEE_OK;
+    }
     if (ctx->kind == kSingle2D) {
         const StepKernel bulk = step_kernel(ctx->d2, false);
         const StepKernel edge = step_kernel(ctx->d2, true);
@@ -917,6 +1056,14 @@ int32_t yee2d_update(yee_ctx* ctx, const yee2d_desc* desc)
     drop_graph(ctx);
     ctx->d2 = d;
     set_geometry(ctx);
+    return YEE_OK;
+}
+
+int32_t yee2d_set_lossless(yee_ctx* ctx, int32_t lossless)
+{
+    if (!ctx || ctx->kind != kSingle2D) return fail(YEE_ESTATE, "not a single 2D context");
+    if (ctx->lossless != (lossless != 0)) drop_graph(ctx);
+    ctx->lossless = lossless != 0;
     return YEE_OK;
 }
 

@@ -49,3 +49,32 @@ typedef struct yee2d_tile_sets {
     int32_t rows[YEE_MAX_EDGE_LINES];
     int32_t cols[YEE_MAX_EDGE_LINES];
 } yee2d_tile_sets;
+
+// Several steps per launch (yee2d_multi.hip): a block of `waves` wavefronts holds a window of 64 * vec columns by
+// waves * r rows and owns what its halo of `steps` rows and columns on every side leaves.
+constexpr int kMultiWavesMax = 8;
+constexpr int kMultiIds = 1024;        // entries of the coefficient table in LDS, the zero entry included
+constexpr int kMultiRowsMax = 64;      // rows of a window
+constexpr int kMultiMax = 16;          // steps of a launch
+
+// Columns left of the owned ones: `steps`, rounded up so that a lane's columns start at a multiple of vec.
+constexpr int yee2d_multi_halo(int steps, int vec) { return (steps + vec - 1) / vec * vec; }
+constexpr int yee2d_multi_columns(int steps, int vec) { return (64 * vec - yee2d_multi_halo(steps, vec) - steps) / vec * vec; }
+constexpr int yee2d_multi_rows(int steps, int waves, int r) { return waves * r - 2 * steps; }
+
+// One rectangle of the grid cut into windows that own rows x columns cells each (window ti * tiles_j + tj of the region
+// is block `first` + that index).
+typedef struct yee2d_multi_region {
+    int32_t i0, i1, j0, j1;
+    int32_t rows, columns, tiles_j;
+    int32_t first;
+} yee2d_multi_region;
+
+// Regions of one launch: region 0 holds windows of the kernel's tall lean shape when `interior` is set; the last
+// region's `first` is followed by `blocks`.
+typedef struct yee2d_multi_plan {
+    yee2d_multi_region region[5];
+    int32_t n_regions, interior;
+    int32_t blocks;
+    int32_t steps;
+} yee2d_multi_plan;

@@ -734,6 +734,7 @@ class Engine2D:
             _lib.check(self.lib.yee2d_create(ctypes_byref(d), ctypes_byref(self._ctx)), 'yee2d_create')
         else:
             _lib.check(self.lib.yee2d_update(self._ctx, ctypes_byref(d)), 'yee2d_update')
+        _lib.check(self.lib.yee2d_set_lossless(self._ctx, int(self.model.materials.lossless())), 'yee2d_set_lossless')
 
     def launch_geometry(self):
         """(rows_per_tile, lane_columns) the library resolved for this instance."""

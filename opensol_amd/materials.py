@@ -145,6 +145,11 @@ class MaterialMap:
         """(n_materials, 6) float64 array of the float32 material values."""
         return np.array(self.materials, dtype=np.float64)
 
+    def lossless(self):
+        """Whether no entry is PEC or lossy and all share one mu_r (the library's launch-shape hint)."""
+        v = self.values()
+        return bool(np.all(v[:, 0] > 0) and not np.any(v[:, (3, 5)]) and np.all(v[:, 4] == v[0, 4]))
+
     def used(self):
         """Sorted unique ids present in the grid."""
         return np.unique(self.ids)

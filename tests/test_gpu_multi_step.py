@@ -1,0 +1,95 @@
+"""Several 2D steps in one launch against the same steps one launch each (step_timed): every field, psi array and
+accumulator equal bit for bit, at sizes around the window edges, across polarisations, boundaries, materials, sources,
+monitors and step counts, from random fields and psi."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+DX, NPML = 25e-9, 8
+
+
+def build(pol, nx, ny, boundaries, media, graph_steps=0):
+    from opensol_amd import Simulation
+    px, py = boundaries in ('periodic_x', 'periodic'), boundaries in ('periodic_y', 'periodic')
+    wx, wy = nx - (0 if px else 2 * NPML), ny - (0 if py else 2 * NPML)
+    sim = Simulation(wx * DX, wy * DX, DX, npml=NPML, boundaries=boundaries, polarization=pol, graph_steps=graph_steps)
+    assert sim.model.shape == (nx, ny)
+    rng = np.random.default_rng([nx, ny])
+    for _ in range(6):
+        x0, y0 = rng.uniform(0, 0.7 * wx * DX), rng.uniform(0, 0.7 * wy * DX)
+        sim.add_dielectric_rectangle(x0, y0, x0 + 0.3 * wx * DX, y0 + 0.3 * wy * DX, eps_r=rng.uniform(1, 12),
+                                     sigma_e=2e3 if media == 'lossy' else 0.0)
+    if media == 'pec':
+        sim.add_pec_rectangle(0.3 * wx * DX, 0.2 * wy * DX, 0.5 * wx * DX, 0.6 * wy * DX)
+    sim.add_line_source(axis='y', position=0.4 * wx * DX, wavelength=600e-9, bandwidth=0.8, waveform='ricker')
+    sim.add_line_source(axis='x', position=0.6 * wy * DX, wavelength=700e-9, bandwidth=0.8, waveform='ricker',
+                        span=(0.1 * wx * DX, 0.8 * wx * DX))
+    if pol == 'ez':
+        sim.add_point_source(0.5 * wx * DX, 0.5 * wy * DX, wavelength=600e-9, waveform='ricker')
+    else:
+        sim.add_magnetic_line_current(0.5 * wx * DX, 0.5 * wy * DX, wavelength=600e-9, waveform='ricker')
+        sim.add_electric_dipole(0.7 * wx * DX, 0.3 * wy * DX, wavelength=600e-9, orientation=30.0, waveform='ricker')
+    sim.add_flux_monitor(axis='y', position=0.7 * wx * DX, span=(0.0, wy * DX), wavelengths=[500e-9, 700e-9])
+    sim.add_flux_monitor(axis='x', position=0.2 * wy * DX, span=(0.2 * wx * DX, wx * DX), wavelengths=[600e-9])
+    sim.finalize()
+    torch = sim.engine.torch
+    generator = torch.Generator().manual_seed(nx * 1000 + ny)
+
+    def fill(t):   # the current set only, as a restored run has it; padding columns stay 0
+        t.copy_(torch.randn(t.shape, generator=generator))
+    fill(sim.engine.fields[0, :, :, :ny])
+    for axis in sim.engine.cpml.values():
+        if axis is not None:
+            fill(axis['psi_e'][0][..., :ny] if axis is sim.engine.cpml['x'] else axis['psi_e'][0])
+            fill(axis['psi_h'][0][..., :ny] if axis is sim.engine.cpml['x'] else axis['psi_h'][0])
+    # psi of a hi-face row past the grid's last one is never updated and holds 0 in a run
+    return sim
+
+
+def arrays(sim, n):
+    e = sim.engine
+    out = {'fields': e.fields[n & 1]}
+    for name, axis in e.cpml.items():
+        if axis is not None:
+            out[f'psi_e {name}'], out[f'psi_h {name}'] = axis['psi_e'][n & 1], axis['psi_h'][n & 1]
+    out.update({f'acc {k}': a for k, a in enumerate(e.accumulators)})
+    out['clock'] = e.clock
+    return out
+
+
+# sizes below, at and past one window (64 x 16, 64 x 32, 64 x 64 cells less their halos), odd columns, a few windows,
+# and grids with an interior of 128 x 64 windows
+SIZES = [(20, 19), (34, 64), (61, 37), (50, 108), (129, 130), (300, 257), (97, 700), (611, 523)]
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+@pytest.mark.parametrize('nx,ny', SIZES)
+@pytest.mark.parametrize('boundaries,media', [('pml', 'plain'), ('periodic_y', 'lossy'), ('periodic_x', 'pec'),
+                                              ('periodic', 'plain'), ('pml', 'lossy')])
+def test_multi_step_matches_single_steps(gpu, pol, nx, ny, boundaries, media):
+    multi, single = (build(pol, nx, ny, boundaries, media) for _ in range(2))
+    total = 0
+    for steps in (1, 2, 7, 20, 33):
+        multi.engine.step(steps)
+        single.engine.step_timed(steps)
+        total += steps
+        a, b = arrays(multi, total), arrays(single, total)
+        for name in a:
+            same = (a[name] == b[name]).all()
+            assert bool(same), (name, total, int((a[name] != b[name]).sum()))
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+def test_multi_step_graph_replays(gpu, pol):
+    """Graphs of an odd and an even number of steps, replayed several times with eager steps between."""
+    for graph_steps in (5, 12):
+        graphed, single = build(pol, 140, 171, 'pml', 'plain', graph_steps), build(pol, 140, 171, 'pml', 'plain')
+        total = 0
+        for steps in (2 * graph_steps, 3, graph_steps + 1, 3 * graph_steps):
+            graphed.engine.step(steps)
+            single.engine.step_timed(steps)
+            total += steps
+            a, b = arrays(graphed, total), arrays(single, total)
+            for name in a:
+                assert bool((a[name] == b[name]).all()), (name, graph_steps, total)
