@@ -22,6 +22,10 @@ __global__ void yee2d_batch_kernel(const yee2d_desc* __restrict__ descs, const y
                                    const int32_t* __restrict__ prefix, int32_t n_inst, int32_t offset);
 template <int POL, int VEC, int R, int TV, int TR, int NW>
 __global__ void yee2d_multi_kernel(yee2d_desc d, yee2d_multi_plan plan, int32_t offset, int32_t launch);
+template <int VEC, int R, int TV, int TR, int NW>
+__global__ void yee2d_multi_batch_kernel(const yee2d_desc* __restrict__ descs, const yee2d_multi_plan* __restrict__ plans,
+                                         const int32_t* __restrict__ prefix, int32_t n_inst, int32_t offset,
+                                         int32_t launch, int32_t steps, int32_t previous);
 template <int J, bool POLES>
 __global__ void yee3d_step_kernel(yee3d_desc d, int32_t tiles_j, int32_t tiles_k, int32_t tiles, int32_t offset);
 template <int J>
@@ -75,6 +79,17 @@ enum CtxKind { kSingle2D = 1, kBatch2D = 2, kSingle3D = 3, kBatch3D = 4 };
 constexpr int kRows3D = yee3idx::kRows;    // y rows per 3D wavefront tile (yee3d_index.h)
 constexpr int kOwned3D = yee3idx::kOwned;  // z cells a 3D wavefront tile owns (yee3d_index.h)
 constexpr int kAutoPlanes = 4;     // default x planes per 3D tile
+constexpr int32_t kStepChunk = 4096;   // steps enqueued between clock advances
+
+struct MultiShape;
+
+// What a 2D batch launches: tiles of the two one-step kernels, and, when every member allows it, the shape, steps and
+// windows of the multi-step one (shape null: one step a launch).
+struct Batch2DWork {
+    int64_t bulk_tiles = 0, edge_tiles = 0, windows = 0;
+    const MultiShape* shape = nullptr;
+    int32_t steps = 0;
+};
 
 }  // namespace
 
@@ -84,12 +99,8 @@ struct yee_ctx {
     // batch
     std::vector<yee2d_desc> descs;
     yee2d_desc* descs_dev = nullptr;
-    int32_t* prefix_dev = nullptr;
     int32_t n_inst = 0;
-    // 2D batch: member tile sets and the bulk / general tile prefixes in the device buffer, and the tile counts
-    yee2d_tile_sets* sets_dev = nullptr;
-    int32_t* general_prefix_dev = nullptr;
-    int64_t general_tiles = 0;
+    Batch2DWork batch;
     // launch geometry
     int64_t tiles = 0;
     int blocks = 0;        // blocks of the bulk kernel (4 tiles each)
@@ -452,15 +463,17 @@ bool has_walls(const yee2d_desc& d)
 }
 
 // Whether several steps of an instance can share a launch: no feature that reads or writes the state between steps
-// outside the multi-step kernel, and a coefficient table that fits its LDS.
+// outside the multi-step kernel, and a coefficient table that fits its LDS. (A step limit is for batches only.)
 bool multi_ok(const yee2d_desc& d)
 {
     const int ids = d.polarization == YEE_EZ ? kMultiIds : kMultiIds / 2;   // H_z keeps two entries an id
     return d.n_poles == 0 && d.n_tfsf == 0 && !has_walls(d) && d.n_dft == 0 && d.probes.n_probes == 0 &&
-           d.n_materials < ids && d.step_limit == INT64_MAX;
+           d.n_materials < ids;
 }
 
 typedef void (*MultiKernel)(yee2d_desc, yee2d_multi_plan, int32_t, int32_t);
+typedef void (*MultiBatchKernel)(const yee2d_desc* __restrict__, const yee2d_multi_plan* __restrict__,
+                                 const int32_t* __restrict__, int32_t, int32_t, int32_t, int32_t, int32_t);
 struct MultiShape {
     int vec, r;             // general windows: 64 * vec columns, waves * r rows
     int tall_vec, tall_r;   // lean windows of the interior, likewise (tall_r 0: none)
@@ -470,21 +483,26 @@ struct MultiShape {
     // window_fixed + window_step * t ns more for every further window (the first mostly its loads and stores)
     float fixed, step, window_fixed, window_step;
     MultiKernel kernel[2];  // by polarisation
+    MultiBatchKernel batch; // for batches (null: a shape for few windows only)
 };
 template <int VEC, int R, int TV, int TR, int NW>
-MultiShape multi_shape(int most, float fixed, float step, float window_fixed, float window_step)
+MultiShape multi_shape(int most, float fixed, float step, float window_fixed, float window_step,
+                       MultiBatchKernel batch)
 {
     return MultiShape{VEC, R, TV, TR, NW, most, fixed, step, window_fixed, window_step,
-                      {yee2d_multi_kernel<YEE_EZ, VEC, R, TV, TR, NW>, yee2d_multi_kernel<YEE_HZ, VEC, R, TV, TR, NW>}};
+                      {yee2d_multi_kernel<YEE_EZ, VEC, R, TV, TR, NW>, yee2d_multi_kernel<YEE_HZ, VEC, R, TV, TR, NW>},
+                      batch};
 }
 // Small windows step fastest while there are few of them, tall ones waste least on their halo. Measured (us a step, E_z,
 // graph replay) at 128^2 / 300^2 / 600^2 / 1200^2 / 4000^2 cells: 64 x 16 windows, 7 steps 1.35 / 2.24 / 5.7 / 18.6 / -;
 // 64 x 32, 7 steps 1.84 / 1.74 / 1.96 / 4.32 / 33.7, 10 steps 1.47 / 1.48 / 2.28 / 4.91 / -; 64 x 64 with a 128 x 64
 // interior, 10 steps - / 2.34 / - / 3.28 / 16.7, 14 steps 2.19 / 1.96 / 2.03 / 2.91 / -. 8192^2: 108 / 65 us
 // a step at 5 / 10 steps, 46 ns a window. The numbers of a shape are fitted to these times.
-const MultiShape kMultiShape[] = {multi_shape<1, 8, 2, 8, 8>(14, 11.0f, 1.25f, 35.0f, 1.1f),
-                                  multi_shape<1, 4, 1, 0, 8>(12, 6.7f, 0.8f, 11.0f, 0.25f),
-                                  multi_shape<1, 2, 1, 0, 8>(7, 4.5f, 0.7f, 7.5f, 0.2f)};
+const MultiShape kMultiShape[] = {multi_shape<1, 8, 2, 8, 8>(14, 11.0f, 1.25f, 35.0f, 1.1f,
+                                                             yee2d_multi_batch_kernel<1, 8, 2, 8, 8>),
+                                  multi_shape<1, 4, 1, 0, 8>(12, 6.7f, 0.8f, 11.0f, 0.25f,
+                                                             yee2d_multi_batch_kernel<1, 4, 1, 0, 8>),
+                                  multi_shape<1, 2, 1, 0, 8>(7, 4.5f, 0.7f, 7.5f, 0.2f, nullptr)};
 constexpr int32_t kMultiSideBySide = 400;   // windows that run at once (two blocks of 8 wavefronts a CU, unevenly)
 
 void add_region(yee2d_multi_plan& p, int32_t i0, int32_t i1, int32_t j0, int32_t j1, int32_t rows, int32_t columns)
@@ -530,11 +548,11 @@ yee2d_multi_plan multi_plan(const yee2d_desc& d, int32_t steps, const MultiShape
     return p;
 }
 
-// The estimated time of one launch, in us.
-float multi_time(const yee2d_multi_plan& p, const MultiShape& shape)
+// The estimated time of one launch of `windows` windows, in us.
+float multi_time(int64_t windows, int32_t steps, const MultiShape& shape)
 {
-    const float further = 1e-3f * std::max(0, p.blocks - kMultiSideBySide);
-    return shape.fixed + shape.step * p.steps + further * (shape.window_fixed + shape.window_step * p.steps);
+    const float further = 1e-3f * (float)std::max<int64_t>(0, windows - kMultiSideBySide);
+    return shape.fixed + shape.step * steps + further * (shape.window_fixed + shape.window_step * steps);
 }
 
 // Launches of at most `most` steps each that advance an instance by `count` steps: as few as possible, with the parity
@@ -559,7 +577,8 @@ void choose_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, i
     for (const MultiShape& s : kMultiShape)
         for (int32_t most = 1; most <= std::min(s.most, count); ++most) {
             const int32_t n = multi_launches(count, most);
-            const float time = n * multi_time(multi_plan(ctx->d2, multi_steps(count, n, 0), s, tall_windows(ctx)), s);
+            const int32_t steps = multi_steps(count, n, 0);
+            const float time = n * multi_time(multi_plan(ctx->d2, steps, s, tall_windows(ctx)).blocks, steps, s);
             if (!*shape || time < best) {
                 best = time;
                 *shape = &s;
@@ -570,7 +589,7 @@ void choose_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, i
 
 void set_geometry(yee_ctx* ctx)
 {
-    ctx->multi = multi_ok(ctx->d2);
+    ctx->multi = multi_ok(ctx->d2) && ctx->d2.step_limit == INT64_MAX;
     const yee2d_desc& d = ctx->d2;
     ctx->sets = tile_sets(d);
     const yee2d_tile_sets& s = ctx->sets;
@@ -683,18 +702,19 @@ bool has_ez_walls(const yee2d_desc& d)
 // One lane per column (x faces) and per row (y faces).
 int wall_blocks(const yee2d_desc& d) { return (int)(((int64_t)d.nx + d.ny + 255) / 256); }
 
-// Device buffer of a 2D batch: the member descriptors, their tile sets, then the bulk and the edge tile prefixes
-// (tile counts of members 0..k-1, n + 1 entries each).
+// Device buffer of a 2D batch: the member descriptors, their tile sets and multi-step plans, then the bulk and the edge
+// tile prefixes and the window prefix (counts of members 0..k-1, n + 1 entries each).
 struct Batch2DLayout {
-    size_t sets, bulk_prefix, edge_prefix, bytes;
+    size_t sets, plans, bulk_prefix, edge_prefix, window_prefix, bytes;
 };
 
 constexpr Batch2DLayout batch2d_layout(int32_t n)
 {
     const size_t sets = sizeof(yee2d_desc) * (size_t)n;
-    const size_t bulk = sets + sizeof(yee2d_tile_sets) * (size_t)n;
-    const size_t edge = bulk + sizeof(int32_t) * (size_t)(n + 1);
-    return Batch2DLayout{sets, bulk, edge, edge + sizeof(int32_t) * (size_t)(n + 1)};
+    const size_t plans = sets + sizeof(yee2d_tile_sets) * (size_t)n;
+    const size_t bulk = plans + sizeof(yee2d_multi_plan) * (size_t)n;
+    const size_t prefix = sizeof(int32_t) * (size_t)(n + 1);
+    return Batch2DLayout{sets, plans, bulk, bulk + prefix, bulk + 2 * prefix, bulk + 3 * prefix};
 }
 
 // The launches a 2D batch's members need after each step, over all members at once: E_z walls (blocks along x of the
@@ -722,30 +742,57 @@ BatchAux2D batch_aux_2d(const yee2d_desc* descs, int32_t n)
     return a;
 }
 
-// A 2D batch on the device: where its arrays are, how many tiles of each class it has and its after-step launches.
+// A 2D batch on the device: where its arrays are, what it launches and its after-step launches.
 struct Batch2DArgs {
     const yee2d_desc* descs;
     const yee2d_tile_sets* sets;
+    const yee2d_multi_plan* plans;
     const int32_t* bulk_prefix;
     const int32_t* edge_prefix;
+    const int32_t* window_prefix;
     int32_t n;
-    int64_t bulk_tiles, edge_tiles;
     int32_t lane_columns;
+    Batch2DWork work;
     BatchAux2D aux;
 };
 
-Batch2DArgs batch2d_args(void* base, int32_t n, int64_t bulk_tiles, int64_t edge_tiles, int32_t lane_columns,
-                         const BatchAux2D& aux)
+Batch2DArgs batch2d_args(void* base, int32_t n, const Batch2DWork& work, int32_t lane_columns, const BatchAux2D& aux)
 {
     const Batch2DLayout l = batch2d_layout(n);
     char* b = static_cast<char*>(base);
-    return Batch2DArgs{reinterpret_cast<const yee2d_desc*>(b), reinterpret_cast<const yee2d_tile_sets*>(b + l.sets),
+    return Batch2DArgs{reinterpret_cast<const yee2d_desc*>(b),
+                       reinterpret_cast<const yee2d_tile_sets*>(b + l.sets),
+                       reinterpret_cast<const yee2d_multi_plan*>(b + l.plans),
                        reinterpret_cast<const int32_t*>(b + l.bulk_prefix),
-                       reinterpret_cast<const int32_t*>(b + l.edge_prefix), n, bulk_tiles, edge_tiles, lane_columns,
-                       aux};
+                       reinterpret_cast<const int32_t*>(b + l.edge_prefix),
+                       reinterpret_cast<const int32_t*>(b + l.window_prefix),
+                       n, lane_columns, work, aux};
 }
 
-// count launches of the batched bulk-tile kernel (the lean loops) and of the batched edge-tile kernel (the general
+// Calls of fewer steps than this step one at a time: a batch's windows are laid out once, for the steps of its full
+// launches, and their halos would cost more than the launches they save.
+constexpr int32_t kMultiBatchLeast = 4;
+
+// `count` steps of a batch whose members all share launches of up to work.steps steps, and one launch more for members
+// that end with the wrong parity (yee2d_multi_batch_kernel).
+int32_t launch_multi_batch_2d(const Batch2DArgs& b, int32_t count, hipStream_t stream)
+{
+    const MultiShape& shape = *b.work.shape;
+    const int32_t launches = multi_launches(count, b.work.steps);
+    const int blocks = (int)((b.work.windows + 7) / 8 * 8);   // a multiple of the XCDs
+    int32_t offset = 0, previous = 0;
+    for (int32_t k = 0; k <= launches; ++k) {
+        const int32_t steps = k < launches ? multi_steps(count, launches, k) : 0;
+        hipLaunchKernelGGL(shape.batch, dim3(blocks), dim3(64 * shape.waves), 0, stream, b.descs, b.plans,
+                           b.window_prefix, b.n, offset, k, steps, previous);
+        offset += steps;
+        previous = steps;
+    }
+    YEE_HIP(hipGetLastError());
+    return YEE_OK;
+}
+
+// count steps: several a launch when the members allow it; else count launches of the batched bulk-tile kernel (the lean loops) and of the batched edge-tile kernel (the general
 // loops, one wavefront per tile: the many members keep the device busy), each step followed by the members' E_z
 // walls, DFT regions and probes in the single-instance order, then the clocks.
 int32_t launch_batch_2d(const Batch2DArgs& b, int32_t count, hipStream_t stream)
@@ -754,10 +801,15 @@ int32_t launch_batch_2d(const Batch2DArgs& b, int32_t count, hipStream_t stream)
     auto edge = b.lane_columns == 2
                     ? (b.aux.left ? yee2d_batch_kernel<2, true, true> : yee2d_batch_kernel<2, true, false>)
                     : (b.aux.left ? yee2d_batch_kernel<4, true, true> : yee2d_batch_kernel<4, true, false>);
-    const int bulk_blocks = (int)((b.bulk_tiles + 3) / 4);
-    const int edge_blocks = (int)((b.edge_tiles + 3) / 4);
+    const int bulk_blocks = (int)((b.work.bulk_tiles + 3) / 4);
+    const int edge_blocks = (int)((b.work.edge_tiles + 3) / 4);
     const BatchAux2D& a = b.aux;
-    for (int32_t k = 0; k < count; ++k) {
+    const bool multi = b.work.shape && count >= kMultiBatchLeast;
+    if (multi) {
+        const int32_t status = launch_multi_batch_2d(b, count, stream);
+        if (status != YEE_OK) return status;
+    }
+    for (int32_t k = 0; k < count && !multi; ++k) {
         if (bulk_blocks > 0)
             hipLaunchKernelGGL(bulk, dim3(bulk_blocks), dim3(256), 0, stream, b.descs, b.sets, b.bulk_prefix, b.n, k);
         if (edge_blocks > 0)
@@ -901,8 +953,8 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
         return YEE_OK;
     }
     if (ctx->kind == kBatch2D)
-        return launch_batch_2d(batch2d_args(ctx->descs_dev, ctx->n_inst, ctx->tiles, ctx->general_tiles,
-                                            ctx->descs[0].lane_columns, batch_aux_2d(ctx->descs.data(), ctx->n_inst)),
+        return launch_batch_2d(batch2d_args(ctx->descs_dev, ctx->n_inst, ctx->batch, ctx->descs[0].lane_columns,
+                                            batch_aux_2d(ctx->descs.data(), ctx->n_inst)),
                                count, stream);
     return fail(YEE_ESTATE, "context has no instances");
 }
@@ -941,15 +993,46 @@ int32_t check_batch_member_2d(const yee2d_desc& d, int32_t lane_columns, int32_t
     return YEE_OK;
 }
 
+// The plan of a batch member: tall windows for E_z only (a batch carries no word of its members' materials).
+yee2d_multi_plan batch_plan(const yee2d_desc& d, int32_t steps, const MultiShape& shape)
+{
+    return multi_plan(d, steps, shape, d.polarization == YEE_EZ);
+}
+
+// Shape and steps per launch with the least estimated time per step over all members, for calls of up to `count` steps;
+// none when a member's features need one step a launch.
+void choose_multi_batch(const yee2d_desc* descs, int32_t n, int32_t count, Batch2DWork* work)
+{
+    if (count < kMultiBatchLeast) return;
+    for (int32_t k = 0; k < n; ++k)
+        if (!multi_ok(descs[k])) return;
+    float best = 0.f;
+    for (const MultiShape& s : kMultiShape) {
+        for (int32_t steps = kMultiBatchLeast; s.batch && steps <= std::min(s.most, count); ++steps) {
+            int64_t windows = 0;
+            for (int32_t k = 0; k < n; ++k) windows += batch_plan(descs[k], steps, s).blocks;
+            const float time = multi_time(windows, steps, s) / (float)steps;
+            if (windows > INT32_MAX / 16 || (work->shape && time >= best)) continue;
+            best = time;
+            work->shape = &s;
+            work->steps = steps;
+            work->windows = windows;
+        }
+    }
+}
+
 // The device image of a 2D batch (batch2d_layout(n).bytes bytes at `image`) from member descriptors whose defaults
-// are resolved: checks every member, then writes the descriptors, their tile sets and the two tile prefixes.
-int32_t stage_batch_2d(const yee2d_desc* descs, int32_t n, char* image, int64_t* bulk_tiles, int64_t* edge_tiles)
+// are resolved: checks every member, then writes the descriptors, their tile sets, plans (for calls of up to `count`
+// steps) and prefixes.
+int32_t stage_batch_2d(const yee2d_desc* descs, int32_t n, int32_t count, char* image, Batch2DWork* work)
 {
     const Batch2DLayout l = batch2d_layout(n);
     auto* sets = reinterpret_cast<yee2d_tile_sets*>(image + l.sets);
+    auto* plans = reinterpret_cast<yee2d_multi_plan*>(image + l.plans);
     auto* bulk = reinterpret_cast<int32_t*>(image + l.bulk_prefix);
     auto* edge = reinterpret_cast<int32_t*>(image + l.edge_prefix);
-    bulk[0] = edge[0] = 0;
+    auto* window = reinterpret_cast<int32_t*>(image + l.window_prefix);
+    bulk[0] = edge[0] = window[0] = 0;
     for (int32_t k = 0; k < n; ++k) {
         int32_t status = check_batch_member_2d(descs[k], descs[0].lane_columns, k);
         if (status != YEE_OK) return status;
@@ -964,8 +1047,13 @@ int32_t stage_batch_2d(const yee2d_desc* descs, int32_t n, char* image, int64_t*
         bulk[k + 1] = (int32_t)next_bulk;
         edge[k + 1] = (int32_t)next_edge;
     }
-    *bulk_tiles = bulk[n];
-    *edge_tiles = edge[n];
+    work->bulk_tiles = bulk[n];
+    work->edge_tiles = edge[n];
+    choose_multi_batch(descs, n, count, work);
+    for (int32_t k = 0; k < n; ++k) {
+        plans[k] = work->shape ? batch_plan(descs[k], work->steps, *work->shape) : yee2d_multi_plan{};
+        window[k + 1] = window[k] + plans[k].blocks;
+    }
     return YEE_OK;
 }
 
@@ -1079,8 +1167,8 @@ int32_t yee2d_batch_create(const yee2d_desc* descs, int32_t n, void* descs_dev, 
     }
     const Batch2DLayout l = batch2d_layout(n);
     std::vector<char> image(l.bytes);
-    int64_t bulk_tiles = 0, edge_tiles = 0;
-    int32_t status = stage_batch_2d(host.data(), n, image.data(), &bulk_tiles, &edge_tiles);
+    Batch2DWork work;
+    int32_t status = stage_batch_2d(host.data(), n, INT32_MAX, image.data(), &work);
     if (status != YEE_OK) return status;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     YEE_HIP(hipMemcpyAsync(descs_dev, image.data(), l.bytes, hipMemcpyHostToDevice, s));
@@ -1090,9 +1178,7 @@ int32_t yee2d_batch_create(const yee2d_desc* descs, int32_t n, void* descs_dev, 
     ctx->descs = std::move(host);
     ctx->descs_dev = reinterpret_cast<yee2d_desc*>(descs_dev);
     ctx->n_inst = n;
-    ctx->tiles = bulk_tiles;
-    ctx->general_tiles = edge_tiles;
-    ctx->blocks = (int)((bulk_tiles + 3) / 4);
+    ctx->batch = work;
     *out = ctx;
     return YEE_OK;
 }
@@ -1116,20 +1202,19 @@ int32_t yee2d_batch_step_static(const yee2d_desc* descs, int32_t n, int64_t n_st
     int32_t status = scratch_address(&base);
     if (status != YEE_OK) return status;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    int64_t bulk_tiles = 0, edge_tiles = 0;
+    Batch2DWork work;
     {
         std::lock_guard<std::mutex> lock(g_scratch_mutex);
-        status = stage_batch_2d(descs, n, g_static_image, &bulk_tiles, &edge_tiles);
+        status = stage_batch_2d(descs, n, (int32_t)std::min<int64_t>(n_steps, kStepChunk), g_static_image, &work);
         if (status != YEE_OK) return status;
         // stream-ordered after this stream's earlier work (an earlier call's launches read the same array); the
         // host image is reused by the next call, so the copy completes before the lock is released
         YEE_HIP(hipMemcpyAsync(base, g_static_image, batch2d_layout(n).bytes, hipMemcpyHostToDevice, s));
         YEE_HIP(hipStreamSynchronize(s));
     }
-    const Batch2DArgs args = batch2d_args(base, n, bulk_tiles, edge_tiles, descs[0].lane_columns,
-                                          batch_aux_2d(descs, n));
+    const Batch2DArgs args = batch2d_args(base, n, work, descs[0].lane_columns, batch_aux_2d(descs, n));
     for (int64_t remaining = n_steps; remaining > 0;) {
-        const int32_t chunk = remaining > 4096 ? 4096 : (int32_t)remaining;
+        const int32_t chunk = (int32_t)std::min<int64_t>(remaining, kStepChunk);
         status = launch_batch_2d(args, chunk, s);
         if (status != YEE_OK) return status;
         remaining -= chunk;
@@ -1311,7 +1396,7 @@ int32_t yee_step(yee_ctx* ctx, int64_t n_steps, void* stream)
         }
     }
     while (remaining > 0) {
-        const int32_t chunk = remaining > 4096 ? 4096 : (int32_t)remaining;
+        const int32_t chunk = (int32_t)std::min<int64_t>(remaining, kStepChunk);
         int32_t status = launch_steps(ctx, chunk, s);
         if (status != YEE_OK) return status;
         remaining -= chunk;

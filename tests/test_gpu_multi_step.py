@@ -93,3 +93,31 @@ def test_multi_step_graph_replays(gpu, pol):
             a, b = arrays(graphed, total), arrays(single, total)
             for name in a:
                 assert bool((a[name] == b[name]).all()), (name, graph_steps, total)
+
+
+# (polarisation, nx, ny, boundaries, media): grids with and without a lean interior, of both polarisations
+MEMBERS = [('ez', 61, 37, 'pml', 'plain'), ('hz', 129, 130, 'pml', 'lossy'), ('ez', 611, 523, 'periodic_y', 'lossy'),
+           ('hz', 34, 64, 'periodic', 'plain'), ('ez', 300, 257, 'pml', 'pec'), ('hz', 97, 300, 'periodic_x', 'pec'),
+           ('ez', 20, 19, 'periodic', 'plain')]
+
+
+@pytest.mark.parametrize('graph_steps', [0, 9])
+@pytest.mark.parametrize('large', [False, True])
+def test_multi_step_batch_members(gpu, graph_steps, large):
+    """Members that stop within, at the end of and between launches, after odd and even counts, over several calls."""
+    from opensol_amd.batch import Batch2D
+    chosen = [m for m in MEMBERS if large or m[1] * m[2] < 100_000] * (4 if large else 1)
+    members, singles = ([build(*m) for m in chosen] for _ in range(2))
+    batch = Batch2D(members, graph_steps=graph_steps)
+    totals = [0] * len(chosen)
+    for call in ([29, 14, 1, 22, 28, 0, 15], [3, 2, 1, 0, 3, 2, 1], [12, 11, 10, 9, 4, 12, 0], [40] * 7):
+        counts = [call[k % 7] for k in range(len(chosen))]
+        batch.run(counts)
+        for k, (a, b, n) in enumerate(zip(members, singles, counts)):
+            if n:
+                b.engine.step_timed(n)
+            totals[k] += n
+            got, expected = arrays(a, totals[k]), arrays(b, totals[k])
+            for name in got:
+                assert bool((got[name] == expected[name]).all()), (k, name, call)
+    batch.close()
