@@ -2,22 +2,25 @@
 // axis, E update with its CPML, point dipole injection); a second, small launch takes the FP64 Kahan DFT samples of
 // the flux planes on sample steps.
 //
-// Work decomposition. Arrays are (nx, ny, nz) with z contiguous. A wavefront tile spans 64 consecutive z cells, one
-// per lane, of which lanes 1..62 own their cell: lane 0 holds the cell below (its H feeds the E of lane 1) and lane 63
-// the cell above (its E feeds the H of lane 62), so every z neighbour is a wave shuffle and no lane runs extra code.
-// A lane carries J rows along y in registers (rows j0..j0+J-1 owned, plus the halo row j0-1 whose H_x, H_z feed the
-// E of row j0, plus row j0+J whose E feeds the H of row j0+J-1), and the tile marches planes i0..i1-1 along x with the
-// new H of the previous plane kept in registers (the plane i0-1 is recomputed once at the start). Halo values are
-// recomputed from the previous state, which is race-free because the fields and the H CPML psi are double-buffered
-// (step n reads set n & 1 and writes set (n & 1) ^ 1); E psi is read and written only by the owner of its cell.
-// Every copy of an H value goes through the same update helper (the library is built with -ffp-contract=on), so a
-// recomputed halo equals its owner's value bit for bit.
+// It takes instances and batches from kFused3D cells (yee_api.hip) on; smaller ones step in two launches (yee3d_split.hip).
+//
+// Work decomposition. Arrays are (nx, ny, nz) with z contiguous. A block of 16 wavefronts marches a tile of 64 z cells (one a
+// lane) x 14 rows (one a wavefront) along planes_per_tile planes of x. The new H of the plane before stays in registers; a
+// row's new H goes to the row above, and the E it loads to the row below, through LDS, so that a plane costs each wavefront
+// seven loads and six stores. The H of the row below the tile and of the cells below its first z cell is formed again, by
+// two further wavefronts; halo values come from the previous state, which is race-free because the fields and the H CPML psi
+// are double-buffered (step n reads set n & 1 and writes set (n & 1) ^ 1); E psi is read and written only by the owner of its
+// cell. A plane's loads are in flight during the step of the plane before it.
 //
 // Boundaries: a periodic axis wraps its indices; on a non-periodic axis indices are clamped to the grid, which makes
 // the hi neighbour of the last row the row itself (face partner = the cell itself, and inv_h[n-1] = 0 cancels the
 // curl term), and the lo neighbour of row 0 is forced to 0.
 //
-// HBM traffic per cell-update: read six fields (24 B) + uint16 material id (2 B), write six fields (24 B) = 50 B.
+// What bounds it: memory, 26 B read and 24 B written a cell and step; 512^3 takes 1.64 ms (4.1 TB/s of these; a kernel that
+// copies the same arrays takes 1.27). A wavefront's 256 B must be whole cache lines: tiles of 62 cells, as a wavefront with
+// its own z halo owns, take 1.9 ms even to copy, since the lines that two blocks share are written in parts. Measured at
+// 512^3 on the way here: 62-cell tiles without LDS 2.00 ms (10.6 GB moved), rows through LDS 2.02, 64-cell tiles 1.90 (the
+// columns beside the tile cost a line a lane: 2.8 times the reads of L2), without the loads that another wavefront makes 1.64.
 //
 // Reference semantics (file:line of the reference package open_sol/):
 //   H update + CPML    physics/em3d/kernels3d.py:335-400 (update_h_3d), :44-56 (edge_coefficients)
@@ -26,34 +29,47 @@
 //   dipole             physics/em3d/sources3d.py:41-75
 //   plane flux         physics/em3d/monitors3d.py:90-101; physics/em/monitors.py:22-34, 92-96
 //   step order         physics/em3d/engine3d.py:497-554
-#include "yee_device.h"
+#include "yee3d_cells.h"
 #include "yee3d_index.h"
 
 namespace yee3 {
 
 constexpr int LANES = yee3idx::kLanes;
-constexpr int OWNED = yee3idx::kOwned;   // z cells a wavefront tile owns (lanes 1..62)
+constexpr int OWNED = yee3idx::kOwned;
+constexpr int ROWS = yee3idx::kRows;
+constexpr int WAVES = ROWS + 2;    // a block's wavefronts: the halo row, the owned rows, the halo column
 constexpr int LDS_IDS = 512;       // ids whose table is staged in LDS: (da, db, ca, cb) + (eps_r, sigma_e), 12 KiB
-constexpr float EPS0F = 8.8541878128e-12f;
 
 __shared__ float4 lds3_coef[LDS_IDS];
 __shared__ float2 lds3_mat[LDS_IDS];
+// What a plane's step hands on within the block, two planes in turn so that one barrier a plane is enough: the new (H_x,
+// H_z) of a row for the row above it; (E_x, E_z) and the id of the next plane of a row for the row below it; the new (H_x,
+// H_y) of the cell below a row's first one along z; (E_x, E_y) of the next plane of a row's first cell, and (E_x, E_y, id)
+// of the next plane of the cell above its last one.
+__shared__ float2 lds3_h[2][ROWS + 1][LANES], lds3_e[2][ROWS + 1][LANES];
+__shared__ int lds3_id[2][ROWS + 1][LANES];
+__shared__ float2 lds3_below[2][ROWS + 1], lds3_first[2][ROWS + 1];
+__shared__ float4 lds3_above[2][ROWS + 1];
+
+// Orders the block's LDS accesses; global loads and stores stay in flight (no thread reads what another one stores).
+__device__ __forceinline__ void barrier_lds()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
-// Stage the table of one instance in LDS (whole block; every thread reaches the barrier).
-__device__ __forceinline__ bool stage_tables(const yee3d_desc& d)
+// Stage the table of one instance in LDS (whole block; the barrier is the caller's).
+__device__ __forceinline__ void stage_tables(const yee3d_desc& d)
 {
-    const bool use = d.n_materials <= LDS_IDS;
-    if (use) {
-        for (int k = threadIdx.x; k < d.n_materials; k += blockDim.x) {
-            const float* t = d.table + 8 * k;
-            lds3_coef[k] = make_float4(t[0], t[1], t[2], t[3]);
-            lds3_mat[k] = make_float2(t[4], t[5]);
-        }
+    if (d.n_materials > LDS_IDS) return;
+    for (int k = threadIdx.x; k < d.n_materials; k += blockDim.x) {
+        const float* t = d.table + 8 * k;
+        lds3_coef[k] = make_float4(t[0], t[1], t[2], t[3]);
+        lds3_mat[k] = make_float2(t[4], t[5]);
     }
-    __syncthreads();
-    return use;
 }
 
 template <bool LDS>
@@ -70,535 +86,464 @@ __device__ __forceinline__ float2 mat(const yee3d_desc& d, int id)
     else return *reinterpret_cast<const float2*>(d.table + 8 * id + 4);
 }
 
-// (ca, cb) of an E face between cells of ids a and b: the id's own entry when they agree, else the coefficients of the
-// float32 mean eps_r and sigma_e (shares 1/2; kernels3d.py:61-85). With k = sigma dt / (2 eps):
-// ca = (1 - k) / (1 + k) = (eps - sigma dt/2) / (eps + sigma dt/2) and cb = (dt / eps) / (1 + k) = dt / (eps + sigma
-// dt/2), formed with one reciprocal (within 2 ulp of the reference's float32 divisions).
-// PEC ids carry eps_r = -1 and (ca, cb) = (0, 0): a face between two PEC cells is pinned by the id's own entry, and a
-// face between a PEC cell and another cell takes the other cell's values (kernels3d.py:61-85), i.e. its own entry.
+// The face coefficients between cells of ids a (whose entry is `own`) and b.
 template <bool LDS>
-__device__ __forceinline__ float2 face(const yee3d_desc& d, int a, int b)
+__device__ __forceinline__ float2 face(const yee3d_desc& d, int a, int b, const float4& own)
 {
-    if (a == b) {
-        const float4 c = coef<LDS>(d, a);
-        return make_float2(c.z, c.w);
-    }
+    if (a == b) return make_float2(own.z, own.w);
     const float2 ma = mat<LDS>(d, a), mb = mat<LDS>(d, b);
     if (ma.x < 0.f || mb.x < 0.f) {
-        const float4 c = coef<LDS>(d, ma.x < 0.f ? b : a);
+        const float4 c = ma.x < 0.f ? coef<LDS>(d, b) : own;
         return make_float2(c.z, c.w);
     }
-    const float eps = (0.5f * ma.x + 0.5f * mb.x) * EPS0F;
-    const float loss = (0.5f * ma.y + 0.5f * mb.y) * (0.5f * d.dt);
-    const float inv = __builtin_amdgcn_rcpf(eps + loss);
-    return make_float2((eps - loss) * inv, d.dt * inv);
+    return mixed_face(d.dt, ma, mb);
 }
-
-__device__ __forceinline__ float from_next(float v) { return __shfl_down(v, 1, LANES); }
-__device__ __forceinline__ float from_prev(float v) { return __shfl_up(v, 1, LANES); }
-__device__ __forceinline__ int from_next_i(int v) { return __shfl_down(v, 1, LANES); }
 
 using yee3idx::fold;
 
-// psi recursion of one layer cell: b psi + g dF.
-__device__ __forceinline__ float psi_next(float b, float psi, float g, float difference) { return b * psi + g * difference; }
-
-// ---- H components (shared by owners and halo copies) ----
-// H_x: -db (dEz/dy - dEy/dz); CPML y first (-), z first (+).
-__device__ __forceinline__ float hx_yee(float da, float db, float hx, float dez_y, float ihy, float dey_z, float ihz)
-{
-    return da * hx - db * (dez_y * ihy - dey_z * ihz);
-}
-// H_y: -db (dEx/dz - dEz/dx); CPML x first (+), z second (-).
-__device__ __forceinline__ float hy_yee(float da, float db, float hy, float dex_z, float ihz, float dez_x, float ihx)
-{
-    return da * hy - db * (dex_z * ihz - dez_x * ihx);
-}
-// H_z: -db (dEy/dx - dEx/dy); CPML x second (-), y second (+).
-__device__ __forceinline__ float hz_yee(float da, float db, float hz, float dey_x, float ihx, float dex_y, float ihy)
-{
-    return da * hz - db * (dey_x * ihx - dex_y * ihy);
-}
-
-// CPML row of one axis at one index: psi row (-1 outside the layers), b, gain.
-struct Row {
-    int r;
-    float b, g;
+// What the step of one plane reads, loaded a plane ahead: E and the id of the next plane (also of the row above the tile, by
+// its last row), the old H, and the psi of the layers that the cell lies in.
+struct Plane {
+    float ex, ey, ez, exu, ezu, hx, hy, hz;
+    int id, idu;
+    float hp[6];   // x, y, z layers, two each
 };
 
-// The per-index record of an axis read at a wave-uniform index: through the constant address space, so it is a scalar
-// load (counted apart from the vector loads of the field rows, which it would otherwise wait behind).
-__device__ __forceinline__ yee3d_axis_row uniform_row(const yee3d_axis_row* rows, int index)
+// The value of the lane above (lane 63: 0) and below (lane 0: 0).
+__device__ __forceinline__ int lane_above(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true); }
+__device__ __forceinline__ float lane_above(float v) { return __int_as_float(lane_above(__float_as_int(v))); }
+__device__ __forceinline__ float lane_below(float v)
 {
-    typedef const __attribute__((address_space(4))) float ConstF;
-    typedef const __attribute__((address_space(4))) int32_t ConstI;
-    ConstF* f = (ConstF*)(rows) + 8 * index;
-    ConstI* n = (ConstI*)(rows) + 8 * index;
-    yee3d_axis_row out;
-    out.inv_h = f[0];
-    out.inv_e = f[1];
-    out.psi_row_h = n[2];
-    out.b_h = f[3];
-    out.g_h = f[4];
-    out.psi_row_e = n[5];
-    out.b_e = f[6];
-    out.g_e = f[7];
-    return out;
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
 }
 
-__device__ __forceinline__ Row h_row(const yee3d_axis_row& a) { return Row{a.psi_row_h, a.b_h, a.g_h}; }
-__device__ __forceinline__ Row e_row(const yee3d_axis_row& a) { return Row{a.psi_row_e, a.b_e, a.g_e}; }
-
-__device__ __forceinline__ int64_t psi_x(const yee3d_desc& d, int r, int j, int k)
-{
-    return ((int64_t)r * d.ny + j) * d.nz + k;
-}
-__device__ __forceinline__ int64_t psi_y(const yee3d_desc& d, int i, int r, int k)
-{
-    return ((int64_t)i * d.cpml[1].n_rows + r) * d.nz + k;
-}
-__device__ __forceinline__ int64_t psi_z(const yee3d_desc& d, int i, int j, int r)
-{
-    return ((int64_t)i * d.ny + j) * d.cpml[2].n_rows + r;
-}
-
-// Values of one cell column the H update needs from the current plane.
-struct Cell {
-    float ex, ey, ez;
-    int id;
-};
-
-// New H of one cell.
-struct HNew {
-    float hx, hy, hz;
-};
-
-// H update of one cell at (i, j, k) from E at the cell (ex, ey, ez), at j+1 (ez_yp, ex_yp), at k+1 (ey_zp, ex_zp) and
-// at i+1 (ey_xp, ez_xp), with the psi of every layer the cell lies in (read from set `par`; the owner, store = true,
-// writes the new psi to set par ^ 1).
-__device__ __forceinline__ HNew h_cell(const yee3d_desc& d, int par, bool store, float da, float db, float hx,
-                                       float hy, float hz, float ex, float ey, float ez, float ez_yp, float ex_yp,
-                                       float ey_zp, float ex_zp, float ey_xp, float ez_xp, float ihx, float ihy,
-                                       float ihz, const Row& rx, const Row& ry, const Row& rz, int i, int j, int k)
-{
-    const float dez_y = ez_yp - ez, dey_z = ey_zp - ey;
-    const float dex_z = ex_zp - ex, dez_x = ez_xp - ez;
-    const float dey_x = ey_xp - ey, dex_y = ex_yp - ex;
-    float vx = hx_yee(da, db, hx, dez_y, ihy, dey_z, ihz);
-    float vy = hy_yee(da, db, hy, dex_z, ihz, dez_x, ihx);
-    float vz = hz_yee(da, db, hz, dey_x, ihx, dex_y, ihy);
-    const int out = par ^ 1;
-    if (rx.r >= 0) {   // x layers: H_y from E_z (+), H_z from E_y (-)
-        const int64_t p = psi_x(d, rx.r, j, k);
-        const float a = psi_next(rx.b, d.cpml[0].psi_h[par][0][p], rx.g, dez_x);
-        const float b = psi_next(rx.b, d.cpml[0].psi_h[par][1][p], rx.g, dey_x);
-        if (store) {
-            d.cpml[0].psi_h[out][0][p] = a;
-            d.cpml[0].psi_h[out][1][p] = b;
-        }
-        vy += db * a;
-        vz -= db * b;
-    }
-    if (ry.r >= 0) {   // y layers: H_x from E_z (-), H_z from E_x (+)
-        const int64_t p = psi_y(d, i, ry.r, k);
-        const float a = psi_next(ry.b, d.cpml[1].psi_h[par][0][p], ry.g, dez_y);
-        const float b = psi_next(ry.b, d.cpml[1].psi_h[par][1][p], ry.g, dex_y);
-        if (store) {
-            d.cpml[1].psi_h[out][0][p] = a;
-            d.cpml[1].psi_h[out][1][p] = b;
-        }
-        vx -= db * a;
-        vz += db * b;
-    }
-    if (rz.r >= 0) {   // z layers: H_x from E_y (+), H_y from E_x (-)
-        const int64_t p = psi_z(d, i, j, rz.r);
-        const float a = psi_next(rz.b, d.cpml[2].psi_h[par][0][p], rz.g, dey_z);
-        const float b = psi_next(rz.b, d.cpml[2].psi_h[par][1][p], rz.g, dex_z);
-        if (store) {
-            d.cpml[2].psi_h[out][0][p] = a;
-            d.cpml[2].psi_h[out][1][p] = b;
-        }
-        vx += db * a;
-        vy -= db * b;
-    }
-    if (d.mirror[0] | d.mirror[1] | d.mirror[2] | d.mirror[3] | d.mirror[4] | d.mirror[5]) {
-        // symmetric mirror planes (the hi face of cell 0 / n - 2): tangential H = 0 (engine3d.py:513-518)
-        if ((d.mirror[0] == YEE_MIRROR_SYMMETRIC && i == 0) || (d.mirror[1] == YEE_MIRROR_SYMMETRIC && i == d.nx - 2))
-            vy = vz = 0.f;
-        if ((d.mirror[2] == YEE_MIRROR_SYMMETRIC && j == 0) || (d.mirror[3] == YEE_MIRROR_SYMMETRIC && j == d.ny - 2))
-            vx = vz = 0.f;
-        if ((d.mirror[4] == YEE_MIRROR_SYMMETRIC && k == 0) || (d.mirror[5] == YEE_MIRROR_SYMMETRIC && k == d.nz - 2))
-            vx = vy = 0.f;
-    }
-    return HNew{vx, vy, vz};
-}
-
-// Pole records on cell (i, j, k): each record whose box holds the cell updates its state from E^n of its component
-// and corrects the updated value with that face's cb (physics/em3d/engine3d.py:508-530).
-__device__ __forceinline__ void apply_poles_3d(const yee3d_desc& d, int i, int j, int k, const float e_old[3],
-                                               const float cb[3], float e_new[3])
-{
-    for (int p = 0; p < d.n_poles; ++p) {
-        const yee3d_pole& pl = d.pole[p];
-        if (i < pl.i0 || i >= pl.i1 || j < pl.j0 || j >= pl.j1 || k < pl.k0 || k >= pl.k1) continue;
-        const int64_t q = ((int64_t)(i - pl.i0) * (pl.j1 - pl.j0) + (j - pl.j0)) * (pl.k1 - pl.k0) + (k - pl.k0);
-        const int c = pl.component;
-        const float drive = pl.drive[q];
-        if (pl.kind == YEE_DRUDE) {
-            float jc = pl.state[0][q];
-            jc += pl.damping * jc + drive * e_old[c];
-            pl.state[0][q] = jc;
-            e_new[c] -= cb[c] * jc;
-        } else {
-            const float pc = pl.state[0][q];
-            float dpc = pl.state[1][q];
-            dpc += pl.damping * dpc - pl.restoring * pc + drive * e_old[c];
-            pl.state[0][q] = pc + dpc;
-            pl.state[1][q] = dpc;
-            e_new[c] -= cb[c] * pl.inv_dt * dpc;
-        }
-    }
-}
-
-// E update of one owned cell with its CPML (psi in place), dispersive poles (POLES) and point sources.
-template <bool LDS, bool POLES>
-__device__ __forceinline__ void e_cell(const yee3d_desc& d, int64_t n, float& ex, float& ey, float& ez, float2 fx,
-                                       float2 fy, float2 fz, float dhz_y, float dhy_z, float dhx_z, float dhz_x,
-                                       float dhy_x, float dhx_y, float iex, float iey, float iez, const Row& rx,
-                                       const Row& ry, const Row& rz, int i, int j, int k)
-{
-    float vx = fx.x * ex + fx.y * (dhz_y * iey - dhy_z * iez);
-    float vy = fy.x * ey + fy.y * (dhx_z * iez - dhz_x * iex);
-    float vz = fz.x * ez + fz.y * (dhy_x * iex - dhx_y * iey);
-    if (rx.r >= 0) {   // x layers: E_y from H_z (-), E_z from H_y (+)
-        const int64_t p = psi_x(d, rx.r, j, k);
-        float* pf = d.cpml[0].psi_e[0];
-        float* ps = d.cpml[0].psi_e[1];
-        const float a = psi_next(rx.b, pf[p], rx.g, dhz_x);
-        const float b = psi_next(rx.b, ps[p], rx.g, dhy_x);
-        pf[p] = a;
-        ps[p] = b;
-        vy -= fy.y * a;
-        vz += fz.y * b;
-    }
-    if (ry.r >= 0) {   // y layers: E_x from H_z (+), E_z from H_x (-)
-        const int64_t p = psi_y(d, i, ry.r, k);
-        float* pf = d.cpml[1].psi_e[0];
-        float* ps = d.cpml[1].psi_e[1];
-        const float a = psi_next(ry.b, pf[p], ry.g, dhz_y);
-        const float b = psi_next(ry.b, ps[p], ry.g, dhx_y);
-        pf[p] = a;
-        ps[p] = b;
-        vx += fx.y * a;
-        vz -= fz.y * b;
-    }
-    if (rz.r >= 0) {   // z layers: E_x from H_y (-), E_y from H_x (+)
-        const int64_t p = psi_z(d, i, j, rz.r);
-        float* pf = d.cpml[2].psi_e[0];
-        float* ps = d.cpml[2].psi_e[1];
-        const float a = psi_next(rz.b, pf[p], rz.g, dhy_z);
-        const float b = psi_next(rz.b, ps[p], rz.g, dhx_z);
-        pf[p] = a;
-        ps[p] = b;
-        vx -= fx.y * a;
-        vy += fy.y * b;
-    }
-    if constexpr (POLES) {
-        const float e_old[3] = {ex, ey, ez};
-        const float cb[3] = {fx.y, fy.y, fz.y};
-        float e_new[3] = {vx, vy, vz};
-        apply_poles_3d(d, i, j, k, e_old, cb, e_new);
-        vx = e_new[0];
-        vy = e_new[1];
-        vz = e_new[2];
-    }
-    for (int s = 0; s < d.n_sources; ++s) {
-        const yee_point_source& src = d.source[s];
-        if (src.i == i && src.j == j && src.k == k && n < src.wave_len) {
-            const float add = __fmul_rn(src.weight, src.wave[n]);
-            if (src.component == 0) vx += add;
-            else if (src.component == 1) vy += add;
-            else vz += add;
-        }
-    }
-    ex = vx;
-    ey = vy;
-    ez = vz;
-}
-
-// Raw buffer access to one x plane of an array: the plane's base and size sit in a buffer resource (scalar
-// registers), the row offset in a scalar register and the lane's z offset in a vector register, so a load or store
-// needs no vector address arithmetic; an access outside the plane reads 0 and writes nothing.
+// Raw buffer access to one plane of an array: its base and size sit in a buffer resource (scalar registers), the lane's
+// byte offset in a vector register. An access past the plane reads 0 and writes nothing, so a lane that takes no part has
+// the offset OFF instead of a branch around it. (Branches cost more than the accesses here: where paths with and without a
+// store join, the wait for an older load has to assume that there was none, and waits for the stores as well.)
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 constexpr int RSRC_DWORD3 = 0x00020000;   // 32-bit data format, no swizzle (gfx9 buffer resource word 3)
+constexpr uint32_t OFF = 0xfffffffeu;     // past any plane, also halved (ids)
 
 __device__ __forceinline__ Rsrc plane_rsrc(const void* base, uint32_t bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, RSRC_DWORD3);
 }
-__device__ __forceinline__ float ldf(Rsrc r, uint32_t lane_bytes, uint32_t row_bytes)
+__device__ __forceinline__ float ldf(Rsrc r, uint32_t bytes, uint32_t plane = 0)
 {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)lane_bytes, (int)row_bytes, 0));
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)bytes, (int)plane, 0));
 }
-__device__ __forceinline__ int ldid(Rsrc r, uint32_t lane_bytes, uint32_t row_bytes)
+__device__ __forceinline__ int ldid(Rsrc r, uint32_t bytes, uint32_t plane = 0)
 {
-    return (int)__builtin_amdgcn_raw_buffer_load_b16(r, (int)lane_bytes, (int)row_bytes, 0);
+    return (int)__builtin_amdgcn_raw_buffer_load_b16(r, (int)bytes, (int)plane, 0);
 }
-// Default cache policy: non-temporal stores (nt) measured 2.240 against 2.085 ms per 512^3 step, while the 2D stores
-// gain from nt. (Unlike the 2D rows, a 62-cell z row writes partial 64 B segments at both ends; that difference is
-// the likely reason, not a measured one.)
-__device__ __forceinline__ void stf(Rsrc r, uint32_t lane_bytes, uint32_t row_bytes, float v)
+__device__ __forceinline__ void stf(Rsrc r, uint32_t bytes, uint32_t plane, float v)
 {
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)lane_bytes, (int)row_bytes, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)bytes, (int)plane, 0);
 }
 
-// One wavefront tile: planes [i0, i1), rows j0..j0+J-1, z cells tk*OWNED .. +OWNED-1.
-template <int J, bool LDS, bool POLES>
-__device__ void tile3d(const yee3d_desc& d, int64_t n, int i0, int i1, int tj, int tk)
+typedef const __attribute__((address_space(4))) yee3d_desc ConstDesc;
+
+// One block tile: planes [i0, i1), rows tj * ROWS .. + ROWS - 1 (wavefronts 1..ROWS, one row each), z cells tk * OWNED ..
+// + OWNED - 1 (one a lane). Wavefront 0 holds the halo row below. The last wavefront holds the columns beside the tile, 16
+// lanes each: the cells below the first z cell (rows 1..ROWS + 1; their H_x and H_y) and above the last one (rows 0..ROWS;
+// their E_x, E_y). Each of its loads costs a cache line per lane, so it loads no more than that. Every wavefront reaches every barrier.
+// EDGE: any tile. Else no cell of it, halo included, lies in a layer, on a mirror plane, beside a wrap or under a source, and
+// the planes i0 - 1..i1 follow each other: each array is one buffer resource for the whole tile, a plane an offset in it.
+template <bool LDS, bool POLES, bool EDGE>
+__device__ __forceinline__ void tile3d(ConstDesc* desc, int64_t n, int i0, int i1, int tj, int tk)
 {
-    static_assert(J == yee3idx::kRows, "the row index math assumes kRows rows per lane");
-    const int lane = threadIdx.x & (LANES - 1);
+    const yee3d_desc& d = *(const yee3d_desc*)desc;
+    const int lane = threadIdx.x & (LANES - 1), wave = wave_index();
     const int nx = d.nx, ny = d.ny, nz = d.nz;
     const bool px = d.periodic[0] != 0, py = d.periodic[1] != 0, pz = d.periodic[2] != 0;
     const int64_t sx = (int64_t)ny * nz;
-    const uint32_t plane_bytes = (uint32_t)(sx * 4), plane_id_bytes = (uint32_t)(sx * 2);
+    const uint32_t plane_bytes = (uint32_t)sx * 4u;
     const int par = (int)(n & 1);
 
-    // z of this lane: byte offsets within a row
-    const int kraw = yee3idx::lane_z(tk, lane);
-    const int k = fold(kraw, nz, pz);
-    const uint32_t vk4 = (uint32_t)k * 4u, vk2 = (uint32_t)k * 2u;
-    const bool k_zero = !pz && kraw < 0;                      // lo neighbour of cell 0: H reads 0
-    const bool k_own = yee3idx::lane_owns(lane, kraw, nz);
-    const yee3d_axis_row az = d.axis_rows[2][k];
-    const float ihz = az.inv_h, iez = az.inv_e;
-    const Row rz_h = h_row(az), rz_e = e_row(az);
+    const bool column = wave == WAVES - 1, last_row = wave == ROWS;
+    const int side = lane >> 4;   // of the columns: 0 below, 1 above, 2 and 3 none
+    const int kraw = yee3idx::lane_z(tk, !column ? lane : side == 0 ? -1 : LANES);
+    const int jraw = yee3idx::row_y(tj, !column ? wave : side == 1 ? lane & 15 : 1 + min(lane & 15, ROWS));
+    const int k = fold(kraw, nz, pz), j = fold(jraw, ny, py), ju = fold(jraw + 1, ny, py);
+    const bool lone = column || lane == LANES - 1;   // the cell above along z is no other lane's
+    const bool k_zero = !pz && kraw < 0, row_zero = !py && jraw < 0;   // below cell 0 of a non-periodic axis: H reads 0
+    const bool own = wave > 0 && !column && jraw < ny && yee3idx::lane_owns(lane, kraw, nz);
+    const yee3d_axis_row az = d.axis_rows[2][k], ay = d.axis_rows[1][j];
+    const Row rz_h = h_row(az), rz_e = e_row(az), ry_h = h_row(ay), ry_e = e_row(ay);
+    const float ihy = ay.inv_h, iey = ay.inv_e, ihz = az.inv_h, iez = az.inv_e;
+    const uint32_t own_bytes = column && (side > 1 || (lane & 15) > ROWS) ? OFF : (uint32_t)(j * nz + k) * 4u;
+    const uint32_t ez_bytes = column && side == 1 ? OFF : own_bytes;
+    const uint32_t h_bytes = column && (side == 1 || lane >= ROWS) ? OFF : own_bytes, hz_bytes = column ? OFF : own_bytes;
+    const uint32_t up_bytes = (uint32_t)(ju * nz + k) * 4u, store_bytes = own ? own_bytes : OFF;
+    // offsets in a plane of the psi arrays of the y and z layers (used in the layers only)
+    const uint32_t y_bytes_h = (uint32_t)(ry_h.r * nz + k) * 4u, y_bytes_e = (uint32_t)(ry_e.r * nz + k) * 4u;
+    const uint32_t z_bytes_h = (uint32_t)(j * d.cpml[2].n_rows + rz_h.r) * 4u;
+    const uint32_t z_bytes_e = (uint32_t)(j * d.cpml[2].n_rows + rz_e.r) * 4u;
+    const bool layers = EDGE && __ballot(ry_h.r >= 0 || ry_e.r >= 0 || rz_h.r >= 0 || rz_e.r >= 0) != 0;
+    const bool mirrored = EDGE && (d.mirror[0] | d.mirror[1] | d.mirror[2] | d.mirror[3] | d.mirror[4] | d.mirror[5]) != 0;
+    bool sources = false;   // whether a source lies in this wavefront's row
+    for (int s = 0; EDGE && s < d.n_sources; ++s)
+        sources = sources || __ballot(own && d.source[s].j == j && d.source[s].k == k) != 0;
 
-    // rows: 0 = halo j0-1, 1..J owned, J+1 = the row above (E only)
-    int jr[J + 2];
-    uint32_t roff[J + 2];   // row byte offsets j * nz * 4 within a field plane (wave-uniform)
-    float ihy[J + 2], iey[J + 2];
-    bool own[J + 2];
-#pragma unroll
-    for (int r = 0; r < J + 2; ++r) {
-        const int jraw = yee3idx::row_y(tj, r);
-        jr[r] = fold(jraw, ny, py);
-        roff[r] = (uint32_t)jr[r] * (uint32_t)nz * 4u;
-        own[r] = r >= 1 && r <= J && jraw < ny;
-        const yee3d_axis_row ay = uniform_row(d.axis_rows[1], jr[r]);
-        ihy[r] = ay.inv_h;
-        iey[r] = ay.inv_e;
-    }
-    const bool row0_zero = !py && tj == 0;   // the halo row below j = 0 of a non-periodic y axis: its H reads 0
+    const float *fex = d.field[par][0], *fey = d.field[par][1], *fez = d.field[par][2], *fhx = d.field[par][3],
+                *fhy = d.field[par][4], *fhz = d.field[par][5];
+    float *oex = d.field[par ^ 1][0], *oey = d.field[par ^ 1][1], *oez = d.field[par ^ 1][2], *ohx = d.field[par ^ 1][3],
+          *ohy = d.field[par ^ 1][4], *ohz = d.field[par ^ 1][5];
+    const uint16_t* ids = d.material;
+    const yee3d_axis_row* rows_x = d.axis_rows[0];
+    // the resource that holds plane i of an array, and the plane's offset in it
+    const int64_t base = EDGE ? 0 : (int64_t)(i0 - 1) * sx;
+    const uint32_t span = EDGE ? plane_bytes : (uint32_t)(i1 - i0 + 2) * plane_bytes;
+    auto res = [&](const float* a, int i) { return plane_rsrc(a + (EDGE ? (int64_t)i * sx : base), span); };
+    auto res_id = [&](int i) { return plane_rsrc(ids + (EDGE ? (int64_t)i * sx : base), span >> 1); };
+    auto at = [&](int i) { return EDGE ? 0u : (uint32_t)(i - i0 + 1) * plane_bytes; };
 
-    // E (and ids) of plane i, rows 0..J+1 (the row above needs only E_x, E_z)
-    auto load_plane = [&](int i, Cell (&c)[J + 2]) {
-        const int64_t po = (int64_t)i * sx;
-        const Rsrc rx = plane_rsrc(d.field[par][0] + po, plane_bytes);
-        const Rsrc ry = plane_rsrc(d.field[par][1] + po, plane_bytes);
-        const Rsrc rz = plane_rsrc(d.field[par][2] + po, plane_bytes);
-        const Rsrc rid = plane_rsrc(d.material + po, plane_id_bytes);
-#pragma unroll
-        for (int r = 0; r < J + 2; ++r) {
-            c[r].ex = ldf(rx, vk4, roff[r]);
-            c[r].ey = r <= J ? ldf(ry, vk4, roff[r]) : 0.f;
-            c[r].ez = ldf(rz, vk4, roff[r]);
-            c[r].id = ldid(rid, vk2, roff[r] >> 1);
+    // E and the id of plane i
+    auto load_e = [&](int i, float& x, float& y, float& z, int& m, float& xu, float& zu, int& mu) {
+        if (last_row) {   // before the others: the wait for those does not have to assume it away
+            xu = ldf(res(fex, i), up_bytes, at(i));
+            zu = ldf(res(fez, i), up_bytes, at(i));
+            mu = ldid(res_id(i), up_bytes >> 1, at(i) >> 1);
+        }
+        x = ldf(res(fex, i), own_bytes, at(i));
+        y = ldf(res(fey, i), own_bytes, at(i));
+        z = ldf(res(fez, i), ez_bytes, at(i));
+        m = ldid(res_id(i), own_bytes >> 1, at(i) >> 1);
+    };
+    // the loads of plane i's step
+    auto load = [&](int i, int next, const yee3d_axis_row& ax, Plane& p) {
+        load_e(next, p.ex, p.ey, p.ez, p.id, p.exu, p.ezu, p.idu);
+        p.hx = ldf(res(fhx, i), h_bytes, at(i));
+        p.hy = ldf(res(fhy, i), h_bytes, at(i));
+        p.hz = ldf(res(fhz, i), hz_bytes, at(i));
+        if (!EDGE || (ax.psi_row_h < 0 && !layers)) return;
+        ConstDesc* fresh = desc;   // pointers of the layers are read where they are used: with the others they do not fit
+        asm volatile("" : "+s"(fresh));
+        const yee3d_desc& e = *(const yee3d_desc*)fresh;
+        if (ax.psi_row_h >= 0 && own_bytes != OFF) {
+            const int64_t q = (int64_t)ax.psi_row_h * sx;
+            p.hp[0] = ldp(e.cpml[0].psi_h[par][0] + q, own_bytes);
+            p.hp[1] = ldp(e.cpml[0].psi_h[par][1] + q, own_bytes);
+        }
+        if (ry_h.r >= 0) {
+            const int64_t q = (int64_t)i * e.cpml[1].n_rows * nz;
+            p.hp[2] = ldp(e.cpml[1].psi_h[par][0] + q, y_bytes_h);
+            p.hp[3] = ldp(e.cpml[1].psi_h[par][1] + q, y_bytes_h);
+        }
+        if (rz_h.r >= 0) {
+            const int64_t q = (int64_t)i * ny * e.cpml[2].n_rows;
+            p.hp[4] = ldp(e.cpml[2].psi_h[par][0] + q, z_bytes_h);
+            p.hp[5] = ldp(e.cpml[2].psi_h[par][1] + q, z_bytes_h);
         }
     };
 
-    // old H of plane i, rows r_lo..J (the halo row feeds E through H_x and H_z only)
-    auto load_hold = [&](int i, float (&hold)[J + 1][3], int r_lo) {
-        const int64_t po = (int64_t)i * sx;
-        const Rsrc rx = plane_rsrc(d.field[par][3] + po, plane_bytes);
-        const Rsrc ry = plane_rsrc(d.field[par][4] + po, plane_bytes);
-        const Rsrc rz = plane_rsrc(d.field[par][5] + po, plane_bytes);
-#pragma unroll
-        for (int r = 0; r < J + 1; ++r) {
-            if (r < r_lo) continue;
-            hold[r][0] = ldf(rx, vk4, roff[r]);
-            hold[r][1] = r > 0 ? ldf(ry, vk4, roff[r]) : 0.f;
-            hold[r][2] = ldf(rz, vk4, roff[r]);
+    float ex, ey, ez;                       // E of the current plane
+    int id;
+    float exu, ezu, exa, eya;               // and of the row above, and (lone) of the cell above along z
+    int idu, ida;
+    float hy_prev = 0.f, hz_prev = 0.f;     // new H_y, H_z of the plane before
+    int turn = 0;
+
+    // Hands on E of a plane: written before the barrier, read after it.
+    auto give = [&](float x, float y, float z, int m) {
+        if (!column) {
+            lds3_e[turn][wave][lane] = make_float2(x, z);
+            lds3_id[turn][wave][lane] = m;
+            if (lane == 0) lds3_first[turn][wave] = make_float2(x, y);
+        } else if (side == 1 && (lane & 15) <= ROWS) {
+            lds3_above[turn][lane & 15] = make_float4(x, y, __int_as_float(m), 0.f);
         }
     };
-
-    // new H of plane i (cur) from E of plane i+1 (nxt), rows r_lo..J
-    auto h_plane = [&](int i, const Cell (&cur)[J + 2], const Cell (&nxt)[J + 2], HNew (&out)[J + 1],
-                       const float (&hold)[J + 1][3], int r_lo, bool store) {
-        const yee3d_axis_row ax = uniform_row(d.axis_rows[0], i);
-        const Row rx = h_row(ax);
-#pragma unroll
-        for (int r = 0; r < J + 1; ++r) {
-            if (r < r_lo) continue;
-            const Row ry = h_row(uniform_row(d.axis_rows[1], jr[r]));
-            const float ey_zp = from_next(cur[r].ey);
-            const float ex_zp = from_next(cur[r].ex);
-            const float4 c = coef<LDS>(d, cur[r].id);
-            out[r] = h_cell(d, par, store && own[r] && k_own, c.x, c.y, hold[r][0], hold[r][1], hold[r][2], cur[r].ex,
-                            cur[r].ey, cur[r].ez, cur[r + 1].ez, cur[r + 1].ex, ey_zp, ex_zp, nxt[r].ey, nxt[r].ez,
-                            ax.inv_h, ihy[r], ihz, rx, ry, rz_h, i, jr[r], k);
-        }
+    auto take = [&](float xu, float zu, int mu) {
+        const float2 up = lds3_e[turn][min(wave + 1, ROWS)][lane];
+        const int up_id = lds3_id[turn][min(wave + 1, ROWS)][lane];
+        const float4 above = lds3_above[turn][min(wave, ROWS)];
+        exu = last_row ? xu : up.x;
+        ezu = last_row ? zu : up.y;
+        idu = last_row ? mu : up_id;
+        const float2 next = lds3_first[turn][min(lane + 1, ROWS)];   // of the columns: the cell above along z is the row's first
+        exa = column ? next.x : above.x;
+        eya = column ? next.y : above.y;
+        ida = __float_as_int(above.z);
     };
 
-    Cell cur[J + 2], nxt[J + 2];
-    float hold[J + 1][3];
-    HNew hn[J + 1];
-    float hy_prev[J + 1], hz_prev[J + 1];   // new H_y, H_z of plane i-1, rows 1..J
-
-    // prologue: new H of plane i0 - 1 (rows 1..J), or 0 below cell 0 of a non-periodic x axis
-    load_plane(i0, cur);
-    if (i0 > 0 || px) {
-        const int im = i0 > 0 ? i0 - 1 : nx - 1;
-        Cell prev[J + 2];
-        load_plane(im, prev);
-        load_hold(im, hold, 1);
-        h_plane(im, prev, cur, hn, hold, 1, false);
-#pragma unroll
-        for (int r = 1; r < J + 1; ++r) {
-            hy_prev[r] = hn[r].hy;
-            hz_prev[r] = hn[r].hz;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < J + 1; ++r) hy_prev[r] = hz_prev[r] = 0.f;
-    }
-
-    for (int i = i0; i < i1; ++i) {
-        const int ip = fold(i + 1, nx, px);
-        load_plane(ip, nxt);
-        load_hold(i, hold, 0);
-        h_plane(i, cur, nxt, hn, hold, 0, true);
-        // zero the H that stands for "below cell 0" on non-periodic axes
-        if (row0_zero) { hn[0].hx = 0.f; hn[0].hz = 0.f; }
-        if (k_zero) {
-#pragma unroll
-            for (int r = 0; r < J + 1; ++r) { hn[r].hx = 0.f; hn[r].hy = 0.f; }
-        }
-        const yee3d_axis_row ax = uniform_row(d.axis_rows[0], i);
-        const Row rx_e = e_row(ax);
-        const int64_t po = (int64_t)i * sx;
-        const Rsrc wex = plane_rsrc(d.field[par ^ 1][0] + po, plane_bytes);
-        const Rsrc wey = plane_rsrc(d.field[par ^ 1][1] + po, plane_bytes);
-        const Rsrc wez = plane_rsrc(d.field[par ^ 1][2] + po, plane_bytes);
-        const Rsrc whx = plane_rsrc(d.field[par ^ 1][3] + po, plane_bytes);
-        const Rsrc why = plane_rsrc(d.field[par ^ 1][4] + po, plane_bytes);
-        const Rsrc whz = plane_rsrc(d.field[par ^ 1][5] + po, plane_bytes);
-#pragma unroll
-        for (int r = 1; r < J + 1; ++r) {
-            const float hx_km = from_prev(hn[r].hx);
-            const float hy_km = from_prev(hn[r].hy);
-            const int id_zp = from_next_i(cur[r].id);
-            const float dhz_y = hn[r].hz - hn[r - 1].hz;
-            const float dhy_z = hn[r].hy - hy_km;
-            const float dhx_z = hn[r].hx - hx_km;
-            const float dhz_x = hn[r].hz - hz_prev[r];
-            const float dhy_x = hn[r].hy - hy_prev[r];
-            const float dhx_y = hn[r].hx - hn[r - 1].hx;
-            if (own[r] && k_own) {
-                const int id = cur[r].id;
-                const float2 fx = face<LDS>(d, id, nxt[r].id);
-                const float2 fy = face<LDS>(d, id, cur[r + 1].id);
-                const float2 fz = face<LDS>(d, id, id_zp);
-                const Row ry_e = e_row(uniform_row(d.axis_rows[1], jr[r]));
-                float ex = cur[r].ex, ey = cur[r].ey, ez = cur[r].ez;
-                e_cell<LDS, POLES>(d, n, ex, ey, ez, fx, fy, fz, dhz_y, dhy_z, dhx_z, dhz_x, dhy_x, dhx_y, ax.inv_e,
-                                   iey[r],
-                            iez, rx_e, ry_e, rz_e, i, jr[r], k);
-                stf(wex, vk4, roff[r], ex);
-                stf(wey, vk4, roff[r], ey);
-                stf(wez, vk4, roff[r], ez);
-                stf(whx, vk4, roff[r], hn[r].hx);
-                stf(why, vk4, roff[r], hn[r].hy);
-                stf(whz, vk4, roff[r], hn[r].hz);
+    // New H of plane i; the owners write it, and E of the plane (whole; i >= i0).
+    auto step = [&](int i, bool whole, const yee3d_axis_row& ax, const Plane& p) {
+        ConstDesc* fresh = desc;
+        asm volatile("" : "+s"(fresh));
+        const yee3d_desc& e = *(const yee3d_desc*)fresh;
+        const int out = par ^ 1;
+        float ep[6];   // psi of the E update, in flight during the H update
+        if (EDGE && whole && (layers || ax.psi_row_e >= 0)) {
+            if (own && ax.psi_row_e >= 0) {
+                const int64_t q = (int64_t)ax.psi_row_e * sx;
+                ep[0] = ldp(e.cpml[0].psi_e[0] + q, own_bytes);
+                ep[1] = ldp(e.cpml[0].psi_e[1] + q, own_bytes);
             }
-            hy_prev[r] = hn[r].hy;
-            hz_prev[r] = hn[r].hz;
+            if (own && ry_e.r >= 0) {
+                const int64_t q = (int64_t)i * e.cpml[1].n_rows * nz;
+                ep[2] = ldp(e.cpml[1].psi_e[0] + q, y_bytes_e);
+                ep[3] = ldp(e.cpml[1].psi_e[1] + q, y_bytes_e);
+            }
+            if (own && rz_e.r >= 0) {
+                const int64_t q = (int64_t)i * ny * e.cpml[2].n_rows;
+                ep[4] = ldp(e.cpml[2].psi_e[0] + q, z_bytes_e);
+                ep[5] = ldp(e.cpml[2].psi_e[1] + q, z_bytes_e);
+            }
         }
-#pragma unroll
-        for (int r = 0; r < J + 2; ++r) cur[r] = nxt[r];
+        const bool store = whole && own;
+        const float4 c = coef<LDS>(d, id);
+        const float da = c.x, db = c.y, ihx = ax.inv_h;
+        const float above_x = lane_above(ex), above_y = lane_above(ey), above_z = lane_above(ez);
+        const float ex_zp = lone ? exa : above_x, ey_zp = lone ? eya : above_y, ez_yp = column ? above_z : ezu;
+        const float dez_y = ez_yp - ez, dey_z = ey_zp - ey;
+        const float dex_z = ex_zp - ex, dez_x = p.ez - ez;
+        const float dey_x = p.ey - ey, dex_y = exu - ex;
+        float vx = hx_yee(da, db, p.hx, dez_y, ihy, dey_z, ihz);
+        float vy = hy_yee(da, db, p.hy, dex_z, ihz, dez_x, ihx);
+        float vz = hz_yee(da, db, p.hz, dey_x, ihx, dex_y, ihy);
+        if (EDGE && ax.psi_row_h >= 0) {   // x layers: H_y from E_z (+), H_z from E_y (-)
+            const float a = psi_next(ax.b_h, p.hp[0], ax.g_h, dez_x);
+            const float b = psi_next(ax.b_h, p.hp[1], ax.g_h, dey_x);
+            if (store) {
+                const int64_t q = (int64_t)ax.psi_row_h * sx;
+                stp(e.cpml[0].psi_h[out][0] + q, own_bytes, a);
+                stp(e.cpml[0].psi_h[out][1] + q, own_bytes, b);
+            }
+            vy += db * a;
+            vz -= db * b;
+        }
+        if (EDGE && ry_h.r >= 0) {   // y layers: H_x from E_z (-), H_z from E_x (+)
+            const float a = psi_next(ry_h.b, p.hp[2], ry_h.g, dez_y);
+            const float b = psi_next(ry_h.b, p.hp[3], ry_h.g, dex_y);
+            if (store) {
+                const int64_t q = (int64_t)i * e.cpml[1].n_rows * nz;
+                stp(e.cpml[1].psi_h[out][0] + q, y_bytes_h, a);
+                stp(e.cpml[1].psi_h[out][1] + q, y_bytes_h, b);
+            }
+            vx -= db * a;
+            vz += db * b;
+        }
+        if (EDGE && rz_h.r >= 0) {   // z layers: H_x from E_y (+), H_y from E_x (-)
+            const float a = psi_next(rz_h.b, p.hp[4], rz_h.g, dey_z);
+            const float b = psi_next(rz_h.b, p.hp[5], rz_h.g, dex_z);
+            if (store) {
+                const int64_t q = (int64_t)i * ny * e.cpml[2].n_rows;
+                stp(e.cpml[2].psi_h[out][0] + q, z_bytes_h, a);
+                stp(e.cpml[2].psi_h[out][1] + q, z_bytes_h, b);
+            }
+            vx += db * a;
+            vy -= db * b;
+        }
+        if (EDGE && mirrored) mirror_h(e, i, j, k, vx, vy, vz);
+        if (whole) {
+            stf(res(ohx, i), store_bytes, at(i), vx);
+            stf(res(ohy, i), store_bytes, at(i), vy);
+            stf(res(ohz, i), store_bytes, at(i), vz);
+            if (!column)
+                lds3_h[turn][wave][lane] = EDGE && row_zero ? make_float2(0.f, 0.f) : make_float2(vx, vz);
+            else if (side == 0 && lane < ROWS)
+                lds3_below[turn][lane + 1] = EDGE && k_zero ? make_float2(0.f, 0.f) : make_float2(vx, vy);
+        }
+        give(p.ex, p.ey, p.ez, p.id);
+        const int id_up = idu, id_far = ida;
+        barrier_lds();
+        take(p.exu, p.ezu, p.idu);
+        if (whole) {
+            const float2 row = lds3_h[turn][min(max(wave - 1, 0), ROWS)][lane], first = lds3_below[turn][min(wave, ROWS)];
+            const float below_x = lane_below(vx), below_y = lane_below(vy);
+            const float hx_km = lane == 0 ? first.x : below_x, hy_km = lane == 0 ? first.y : below_y;
+            const int id_above = lane_above(id), id_zp = lone ? id_far : id_above;
+            const float dhz_y = vz - row.y, dhy_z = vy - hy_km;
+            const float dhx_z = vx - hx_km, dhz_x = vz - hz_prev;
+            const float dhy_x = vy - hy_prev, dhx_y = vx - row.x;
+            const float iex = ax.inv_e;
+            float2 fx = make_float2(c.z, c.w), fy = fx, fz = fx;
+            if (__ballot((id != p.id) | (id != id_up) | (id != id_zp)) != 0) {
+                fx = face<LDS>(d, id, p.id, c);
+                fy = face<LDS>(d, id, id_up, c);
+                fz = face<LDS>(d, id, id_zp, c);
+            }
+            float wx = fx.x * ex + fx.y * (dhz_y * iey - dhy_z * iez);
+            float wy = fy.x * ey + fy.y * (dhx_z * iez - dhz_x * iex);
+            float wz = fz.x * ez + fz.y * (dhy_x * iex - dhx_y * iey);
+            if (EDGE && own && ax.psi_row_e >= 0) {   // x layers: E_y from H_z (-), E_z from H_y (+)
+                const int64_t q = (int64_t)ax.psi_row_e * sx;
+                const float a = psi_next(ax.b_e, ep[0], ax.g_e, dhz_x);
+                const float b = psi_next(ax.b_e, ep[1], ax.g_e, dhy_x);
+                stp(e.cpml[0].psi_e[0] + q, own_bytes, a);
+                stp(e.cpml[0].psi_e[1] + q, own_bytes, b);
+                wy -= fy.y * a;
+                wz += fz.y * b;
+            }
+            if (EDGE && own && ry_e.r >= 0) {   // y layers: E_x from H_z (+), E_z from H_x (-)
+                const int64_t q = (int64_t)i * e.cpml[1].n_rows * nz;
+                const float a = psi_next(ry_e.b, ep[2], ry_e.g, dhz_y);
+                const float b = psi_next(ry_e.b, ep[3], ry_e.g, dhx_y);
+                stp(e.cpml[1].psi_e[0] + q, y_bytes_e, a);
+                stp(e.cpml[1].psi_e[1] + q, y_bytes_e, b);
+                wx += fx.y * a;
+                wz -= fz.y * b;
+            }
+            if (EDGE && own && rz_e.r >= 0) {   // z layers: E_x from H_y (-), E_y from H_x (+)
+                const int64_t q = (int64_t)i * ny * e.cpml[2].n_rows;
+                const float a = psi_next(rz_e.b, ep[4], rz_e.g, dhy_z);
+                const float b = psi_next(rz_e.b, ep[5], rz_e.g, dhx_z);
+                stp(e.cpml[2].psi_e[0] + q, z_bytes_e, a);
+                stp(e.cpml[2].psi_e[1] + q, z_bytes_e, b);
+                wx -= fx.y * a;
+                wy += fy.y * b;
+            }
+            if constexpr (POLES) {
+                const float e_old[3] = {ex, ey, ez};
+                const float cb[3] = {fx.y, fy.y, fz.y};
+                float e_new[3] = {wx, wy, wz};
+                if (own) apply_poles_3d(e, i, j, k, e_old, cb, e_new);
+                wx = e_new[0];
+                wy = e_new[1];
+                wz = e_new[2];
+            }
+            if (EDGE && sources && own) add_sources_3d(e, n, i, j, k, wx, wy, wz);
+            stf(res(oex, i), store_bytes, at(i), wx);
+            stf(res(oey, i), store_bytes, at(i), wy);
+            stf(res(oez, i), store_bytes, at(i), wz);
+        }
+        hy_prev = vy;
+        hz_prev = vz;
+        ex = p.ex;
+        ey = p.ey;
+        ez = p.ez;
+        id = p.id;
+        turn ^= 1;
+    };
+
+    // the first plane whose H is formed here: i0 - 1 for H_y, H_z of the plane before (0 below a non-periodic cell 0)
+    const bool before = !EDGE || i0 > 0 || px;
+    const int first = before ? (i0 > 0 ? i0 - 1 : nx - 1) : i0;
+    auto after = [&](int i) { return i + 1 < nx ? i + 1 : (px ? 0 : nx - 1); };
+    Plane a, b;
+    yee3d_axis_row ax = uniform_row(rows_x, first), ax_next = uniform_row(rows_x, before ? i0 : after(i0));
+    load_e(first, ex, ey, ez, id, b.exu, b.ezu, b.idu);
+    load(first, before ? i0 : after(i0), ax, a);
+    give(ex, ey, ez, id);
+    barrier_lds();
+    take(b.exu, b.ezu, b.idu);
+    turn ^= 1;
+    int i = i0;
+    if (before) {
+        load(i0, after(i0), ax_next, b);
+        step(first, false, ax, a);
+        a = b;
+        ax = ax_next;
+        ax_next = uniform_row(rows_x, after(i0));
     }
+    // The next plane's loads are in flight during a plane's step; the last plane has nothing left to load.
+    while (i + 1 < i1) {
+        const yee3d_axis_row ax_far = uniform_row(rows_x, min(i + 2, nx - 1));
+        load(i + 1, after(i + 1), ax_next, b);
+        step(i, true, ax, a);
+        a = b;
+        ++i;
+        ax = ax_next;
+        ax_next = ax_far;
+    }
+    step(i, true, ax, a);
 }
 
-}  // namespace yee3
-
-namespace yee3 {
-
-// The tiles of one block of one instance: tile t = (i chunk, j tile, k tile), k fastest, one per wavefront. Every
-// thread of the block reaches the table barrier before a wave without a tile leaves.
-template <int J, bool POLES>
-__device__ __forceinline__ void step_block(const yee3d_desc& d, int64_t n, int tile, int tiles, int tiles_j,
-                                           int tiles_k)
+// Whether a block tile is an inner one (inner_tile3d). Stages the tables; ends in a barrier of the whole block.
+__device__ __forceinline__ bool inner_block(const yee3d_desc& d, int i0, int i1, int tj, int tk)
 {
-    const bool mine = tile < tiles;
-    if (!__syncthreads_or(mine)) return;
-    const bool lds = stage_tables(d);
-    if (!mine) return;
-    const yee3idx::TileCoords c = yee3idx::tile_coords(tile, tiles_j, tiles_k);
-    const int tk = c.tk, tj = c.tj, ic = c.ic;
-    const int i0 = ic * d.planes_per_tile;
+    stage_tables(d);
+    const int j0 = yee3idx::row_y(tj, 0), j1 = min(d.ny, yee3idx::row_y(tj, ROWS + 1) + 1);
+    const int k0 = yee3idx::lane_z(tk, -1), k1 = min(d.nz, yee3idx::lane_z(tk, OWNED) + 1);
+    bool edge = i0 < 1 || i1 >= d.nx || j0 < 0 || j1 >= d.ny || k0 < 0 || k1 >= d.nz ||
+                (int64_t)d.ny * d.nz * 4 * (i1 - i0 + 2) >= OFF;
+    if (!edge) {
+        auto layer = [&](int axis, int i) {
+            const yee3d_axis_row& r = d.axis_rows[axis][i];
+            return r.psi_row_h >= 0 || r.psi_row_e >= 0;
+        };
+        const int t = threadIdx.x;
+        for (int i = i0 - 1 + t; i <= i1; i += blockDim.x) edge = edge || layer(0, i);
+        if (j0 + t < j1) edge = edge || layer(1, j0 + t);
+        if (k0 + t < k1) edge = edge || layer(2, k0 + t);
+        if (t < d.n_sources) {
+            const yee_point_source& s = d.source[t];
+            edge = edge || (s.i >= i0 && s.i < i1 && s.j >= j0 && s.j < j1 && s.k >= k0 && s.k < k1);
+        }
+        // symmetric mirror planes: the hi face of cell 0 / n - 2
+        edge = edge || (d.mirror[0] && i0 < 2) || (d.mirror[1] && i1 > d.nx - 2) || (d.mirror[2] && j0 < 1) ||
+               (d.mirror[3] && j1 > d.ny - 2) || (d.mirror[4] && k0 < 1) || (d.mirror[5] && k1 > d.nz - 2);
+    }
+    return !__syncthreads_or(edge);
+}
+
+// The tile of block `block` of one instance: z tile fastest, then y tile, then x chunk.
+template <bool POLES>
+__device__ __forceinline__ void step_block(ConstDesc* desc, int64_t n, int block)
+{
+    const yee3d_desc& d = *(const yee3d_desc*)desc;
+    const int tiles_j = yee3idx::tiles_along(d.ny, yee3idx::kRows), tiles_k = yee3idx::tiles_along(d.nz, OWNED);
+    const yee3idx::TileCoords c = yee3idx::tile_coords(block, tiles_j, tiles_k);
+    const int i0 = c.ic * d.planes_per_tile;
     const int i1 = min(d.nx, i0 + d.planes_per_tile);
-    if (lds)
-        tile3d<J, true, POLES>(d, n, i0, i1, tj, tk);
+    const bool inner = inner_block(d, i0, i1, c.tj, c.tk) && !POLES;   // and the barrier that the tables need
+    const bool lds = d.n_materials <= LDS_IDS;
+    if (inner && lds)
+        tile3d<true, false, false>(desc, n, i0, i1, c.tj, c.tk);
+    else if (lds)
+        tile3d<true, POLES, true>(desc, n, i0, i1, c.tj, c.tk);
     else
-        tile3d<J, false, POLES>(d, n, i0, i1, tj, tk);
+        tile3d<false, POLES, true>(desc, n, i0, i1, c.tj, c.tk);
 }
+
+// Consecutive workgroups go to the 8 XCDs in turn: block b of a grid of a multiple of 8 takes part b % 8 of the tiles, so
+// that tiles side by side share an L2.
+__device__ __forceinline__ int xcd_block() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
 
 }  // namespace yee3
 
-// One 3D instance, four tiles per block. POLES: the E update carries the dispersive-pole records; that instantiation
-// reads the descriptor in place at the kernel-argument pointer (constant address space), since the records are
-// indexed at run time.
-template <int J, bool POLES>
-__global__ void __launch_bounds__(256) yee3d_step_kernel(yee3d_desc desc, int32_t tiles_j, int32_t tiles_k,
-                                                        int32_t tiles, int32_t offset)
+// One 3D instance, one tile per block. The descriptor is read in place at the kernel-argument pointer.
+template <bool POLES>
+__global__ void __launch_bounds__(64 * yee3::WAVES) yee3d_step_kernel(yee3d_desc desc, int32_t blocks, int32_t offset)
 {
-    if constexpr (POLES) {
-        typedef const __attribute__((address_space(4))) yee3d_desc ConstDesc;
-        const yee3d_desc& d = *(const yee3d_desc*)(ConstDesc*)__builtin_amdgcn_kernarg_segment_ptr();
-        if (d.clock != desc.clock) return;
-        const int64_t n = *d.clock + offset;
-        if (n >= d.step_limit) return;
-        yee3::step_block<J, true>(d, n, blockIdx.x * 4 + yee3::wave_index(), tiles, tiles_j, tiles_k);
-    } else {
-        const int64_t n = *desc.clock + offset;
-        if (n >= desc.step_limit) return;
-        yee3::step_block<J, false>(desc, n, blockIdx.x * 4 + yee3::wave_index(), tiles, tiles_j, tiles_k);
-    }
+    yee3::ConstDesc* d = (yee3::ConstDesc*)__builtin_amdgcn_kernarg_segment_ptr();
+    if (d->clock != desc.clock) return;
+    const int block = yee3::xcd_block();
+    if (block >= blocks) return;
+    const int64_t n = *d->clock + offset;
+    if (n >= d->step_limit) return;
+    yee3::step_block<POLES>(d, n, block);
 }
 
 // Many 3D instances of uneven sizes in one launch: block b belongs to the instance whose block range
 // [prefix[k], prefix[k+1]) holds it, so a block stages one instance's table. Each instance runs on its own clock
 // and stops at its own step limit; members with dispersive poles take the E update that carries them.
-template <int J>
-__global__ void __launch_bounds__(256) yee3d_batch_kernel(const yee3d_desc* __restrict__ descs,
-                                                         const int32_t* __restrict__ prefix, int32_t n_inst,
-                                                         int32_t offset)
+__global__ void __launch_bounds__(64 * yee3::WAVES) yee3d_batch_kernel(const yee3d_desc* __restrict__ descs,
+                                                          const int32_t* __restrict__ prefix, int32_t n_inst,
+                                                          int32_t offset)
 {
-    const int block = blockIdx.x;
+    const int block = yee3::xcd_block();
+    if (block >= prefix[n_inst]) return;
     int lo = 0, hi = n_inst;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         if (prefix[mid] <= block) lo = mid; else hi = mid;
     }
     // Read the descriptor through the constant address space: its fields become scalar loads, as a kernel argument's.
-    typedef const __attribute__((address_space(4))) yee3d_desc ConstDesc;
-    const yee3d_desc& d = *(const yee3d_desc*)((ConstDesc*)descs + lo);
-    const int64_t n = *d.clock + offset;
-    if (n >= d.step_limit) return;
-    const int tiles_j = (d.ny + J - 1) / J;
-    const int tiles_k = (d.nz + yee3::OWNED - 1) / yee3::OWNED;
-    const int tiles = ((d.nx + d.planes_per_tile - 1) / d.planes_per_tile) * tiles_j * tiles_k;
-    const int tile = (block - prefix[lo]) * 4 + yee3::wave_index();
-    if (d.n_poles > 0)   // the E update with the member's dispersive-pole records (block-uniform: one member per block)
-        yee3::step_block<J, true>(d, n, tile, tiles, tiles_j, tiles_k);
+    yee3::ConstDesc* d = (yee3::ConstDesc*)descs + lo;
+    const int64_t n = *d->clock + offset;
+    if (n >= d->step_limit) return;
+    const int own = block - prefix[lo];
+    if (d->n_poles > 0)   // the E update with the member's dispersive-pole records (block-uniform: one member per block)
+        yee3::step_block<true>(d, n, own);
     else
-        yee3::step_block<J, false>(d, n, tile, tiles, tiles_j, tiles_k);
+        yee3::step_block<false>(d, n, own);
 }
 
-template __global__ void yee3d_step_kernel<4, false>(yee3d_desc, int32_t, int32_t, int32_t, int32_t);
-template __global__ void yee3d_step_kernel<4, true>(yee3d_desc, int32_t, int32_t, int32_t, int32_t);
-template __global__ void yee3d_batch_kernel<4>(const yee3d_desc* __restrict__, const int32_t* __restrict__, int32_t,
-                                               int32_t);
+template __global__ void yee3d_step_kernel<false>(yee3d_desc, int32_t, int32_t);
+template __global__ void yee3d_step_kernel<true>(yee3d_desc, int32_t, int32_t);
 
 // FP64 Kahan DFT samples of the flux planes after step n (when (n + 1) % m == 0): one thread per plane cell and pair;
 // E = mean of the layers edge - 1 and edge along the normal, H on layer edge - 1 (monitors3d.py:90-101).

@@ -5,8 +5,8 @@
 namespace yee3idx {
 
 constexpr int kLanes = 64;
-constexpr int kOwned = 62;   // z cells a wavefront tile owns (lanes 1..62; lane 0 and lane 63 hold the z halo)
-constexpr int kRows = 4;     // y rows a lane owns
+constexpr int kOwned = 64;   // z cells of a tile, one a lane
+constexpr int kRows = 14;    // y rows of a tile, one a wavefront
 
 // Wrapped (periodic) or clamped index along an axis of n cells. A tile can span several periods of a short periodic
 // axis (64 lanes over nz = 5), so the wrap is a full modulo.
@@ -21,16 +21,16 @@ constexpr int fold(int v, int n, bool periodic)
 
 constexpr int tiles_along(int n, int per_tile) { return (n + per_tile - 1) / per_tile; }
 
-// z of lane `lane` of z tile tk before folding (the tile's first owned cell is tk * kOwned)
-constexpr int lane_z(int tk, int lane) { return tk * kOwned - 1 + lane; }
+// z of lane `lane` of z tile tk before folding (lane -1: the halo column below the tile, lane 64: the one above)
+constexpr int lane_z(int tk, int lane) { return tk * kOwned + lane; }
 
-// y of register row r (0: the halo row below, 1..kRows: owned, kRows + 1: the row above) of y tile tj before folding
+// y of row r (0: the halo row below, 1..kRows: owned, kRows + 1: the row above) of y tile tj before folding
 constexpr int row_y(int tj, int r) { return tj * kRows - 1 + r; }
 
 // whether lane `lane` owns its cell (z before folding: kz)
-constexpr bool lane_owns(int lane, int kz, int nz) { return lane >= 1 && lane <= kOwned && kz < nz; }
+constexpr bool lane_owns(int lane, int kz, int nz) { return lane >= 0 && lane < kOwned && kz < nz; }
 
-// The tile of wave slot `slot` of one instance: z tile fastest, then y tile, then x chunk.
+// The tile of block `slot` of one instance: z tile fastest, then y tile, then x chunk.
 struct TileCoords {
     int ic, tj, tk;
 };

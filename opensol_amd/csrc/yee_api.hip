@@ -26,9 +26,14 @@ template <int VEC, int R, int TV, int TR, int NW>
 __global__ void yee2d_multi_batch_kernel(const yee2d_desc* __restrict__ descs, const yee2d_multi_plan* __restrict__ plans,
                                          const int32_t* __restrict__ prefix, int32_t n_inst, int32_t offset,
                                          int32_t launch, int32_t steps, int32_t previous);
-template <int J, bool POLES>
-__global__ void yee3d_step_kernel(yee3d_desc d, int32_t tiles_j, int32_t tiles_k, int32_t tiles, int32_t offset);
-template <int J>
+__global__ void yee3d_h_kernel(yee3d_desc desc, int32_t offset);
+template <bool POLES>
+__global__ void yee3d_e_kernel(yee3d_desc desc, int32_t offset);
+template <bool E>
+__global__ void yee3d_batch_half_kernel(const yee3d_desc* __restrict__ descs, const int32_t* __restrict__ prefix,
+                                        int32_t n_inst, int32_t offset);
+template <bool POLES>
+__global__ void yee3d_step_kernel(yee3d_desc desc, int32_t blocks, int32_t offset);
 __global__ void yee3d_batch_kernel(const yee3d_desc* __restrict__ descs, const int32_t* __restrict__ prefix,
                                    int32_t n_inst, int32_t offset);
 __global__ void yee3d_sample_kernel(yee3d_desc d, int64_t cells_total, int32_t offset);
@@ -76,9 +81,7 @@ constexpr int kAutoRows = 8;
 
 enum CtxKind { kSingle2D = 1, kBatch2D = 2, kSingle3D = 3, kBatch3D = 4 };
 
-constexpr int kRows3D = yee3idx::kRows;    // y rows per 3D wavefront tile (yee3d_index.h)
-constexpr int kOwned3D = yee3idx::kOwned;  // z cells a 3D wavefront tile owns (yee3d_index.h)
-constexpr int kAutoPlanes = 4;     // default x planes per 3D tile
+constexpr int kRows3D = 4;         // the one accepted rows_per_tile of a 3D descriptor
 constexpr int32_t kStepChunk = 4096;   // steps enqueued between clock advances
 
 struct MultiShape;
@@ -107,10 +110,10 @@ struct yee_ctx {
     int edge_blocks = 0;   // blocks of the edge kernel (sets.edge_parts wavefronts per tile, 4 per block)
     yee2d_tile_sets sets{};
     bool multi = false;    // several steps per launch (yee2d_multi.hip)
+    bool fused = false;    // 3D: one launch a step (yee3d.hip), else two (yee3d_split.hip)
     bool lossless = false; // yee2d_set_lossless
     // 3D
     yee3d_desc d3{};
-    int32_t tiles_j3 = 0, tiles_k3 = 0;
     int64_t sample_cells = 0;   // plane cells x pairs of the sample launch
     // 3D batch: descriptors, block prefix and plane-cell prefix in the caller's device buffer
     std::vector<yee3d_desc> descs3;
@@ -350,15 +353,6 @@ int64_t tiles_2d(const yee2d_desc& d)
 }
 
 using StepKernel = void (*)(yee2d_desc, yee2d_tile_sets, int32_t);
-
-// Bulk-tile (edge = false) or edge-tile kernel of a descriptor.
-// The 3D step kernel of an instance: the one with the pole update only when it has poles (its registers and its
-// descriptor reads differ).
-typedef void (*StepKernel3D)(yee3d_desc, int32_t, int32_t, int32_t, int32_t);
-StepKernel3D step_kernel_3d(const yee3d_desc& d)
-{
-    return d.n_poles > 0 ? yee3d_step_kernel<kRows3D, true> : yee3d_step_kernel<kRows3D, false>;
-}
 
 // An H_z instance whose y_hi copy wall (pec or mirror) column ny - 1 is the first column of a tile: its edge tiles
 // run the general loop with lane 0's recompute of column ny - 2.
@@ -601,24 +595,46 @@ void set_geometry(yee_ctx* ctx)
     ctx->edge_blocks = (int)((edge * ctx->sets.edge_parts + 3) / 4);
 }
 
-// Defaults of a 3D descriptor: 4 rows per tile and kAutoPlanes x planes per tile (balanced over the x extent).
-// Short tiles re-read one extra E plane per kAutoPlanes planes but keep more tiles in flight; 4 measured fastest on
-// 512^3 (2.05 ms per step against 2.15 ms at 8 and slower beyond).
-void apply_defaults_3d(yee3d_desc& d)
+// Instances and batches of at least this many cells step in one fused launch (yee3d.hip), smaller ones in an H and an E
+// launch (yee3d_split.hip). Measured, us a step, fused / split at the planes per tile below: 140 x 130 x 120 (2.2M cells)
+// 53 / 37, 256^3 (16.8M) 265 / 293, 512^3 1640 / 2120.
+constexpr int64_t kFused3D = (int64_t)1 << 23;
+
+int64_t cells_3d(const yee3d_desc& d) { return (int64_t)d.nx * d.ny * d.nz; }
+
+// Default x planes per tile, balanced over the x extent. Split: few, to fill the chip (us a step at 1 / 2 / 4 planes: 64^3
+// 10.7 / 11.8 / 15.0, 97 x 88 x 75 20.0 / 18.3 / 20.9, 140 x 130 x 120 40.2 / 37.2 / 40.7, 256^3 343 / 307 / 293). Fused: a
+// tile forms the H of one plane more than it owns, so long tiles while there are enough of them (8 / 16 / 32 planes: 256^3
+// 283 / 265 / 297, 512^3 1887 / 1716 / 1639).
+int64_t default_planes(const yee3d_desc& d, bool fused)
+{
+    const int64_t cells = cells_3d(d);
+    if (fused) return cells >= (int64_t)1 << 26 ? 32 : 16;
+    return cells < 400000 ? 1 : cells < (int64_t)4 << 20 ? 2 : 4;
+}
+
+// Blocks of a 3D instance's launch: x chunks x y tiles x z tiles, or x chunks x runs of 256 plane cells in 8 equal parts.
+int64_t blocks_3d(const yee3d_desc& d, bool fused)
+{
+    const int64_t chunks = (d.nx + (int64_t)d.planes_per_tile - 1) / d.planes_per_tile;
+    if (fused) return chunks * yee3idx::tiles_along(d.ny, yee3idx::kRows) * yee3idx::tiles_along(d.nz, yee3idx::kOwned);
+    return chunks * ((((int64_t)d.ny * d.nz + 255) / 256 + 7) / 8 * 8);
+}
+constexpr int kThreads3D = 64 * (yee3idx::kRows + 2);
+int grid_3d(int64_t blocks) { return (int)((blocks + 7) / 8 * 8); }   // a multiple of the XCDs
+
+// Defaults of a 3D descriptor.
+void apply_defaults_3d(yee3d_desc& d, bool fused)
 {
     if (d.rows_per_tile == 0) d.rows_per_tile = kRows3D;
     if (d.planes_per_tile == 0 && d.nx > 0) {
-        const int64_t planes = std::min<int64_t>(kAutoPlanes, d.nx);
+        const int64_t planes = std::min<int64_t>(default_planes(d, fused), d.nx);
         const int64_t chunks = (d.nx + planes - 1) / planes;
         d.planes_per_tile = (int32_t)((d.nx + chunks - 1) / chunks);
     }
-}
-
-// Wavefront tiles of a 3D instance: x chunks x y tiles x z tiles.
-int64_t tiles_3d(const yee3d_desc& d)
-{
-    const int64_t chunks = (d.nx + d.planes_per_tile - 1) / d.planes_per_tile;
-    return chunks * ((d.ny + kRows3D - 1) / kRows3D) * ((d.nz + kOwned3D - 1) / kOwned3D);
+    // a launch holds at most 2^32 threads
+    while (fused && d.planes_per_tile > 0 && d.planes_per_tile < d.nx && blocks_3d(d, fused) >= (int64_t)1 << 22)
+        d.planes_per_tile *= 2;
 }
 
 // Plane cells x pairs sampled by the sample launch of a 3D instance.
@@ -634,11 +650,24 @@ int64_t sample_cells_3d(const yee3d_desc& d)
 void set_geometry_3d(yee_ctx* ctx)
 {
     const yee3d_desc& d = ctx->d3;
-    ctx->tiles_j3 = (d.ny + kRows3D - 1) / kRows3D;
-    ctx->tiles_k3 = (d.nz + kOwned3D - 1) / kOwned3D;
-    ctx->tiles = tiles_3d(d);
-    ctx->blocks = (int)((ctx->tiles + 3) / 4);
+    ctx->fused = cells_3d(d) >= kFused3D;
+    ctx->tiles = blocks_3d(d, ctx->fused);
+    ctx->blocks = grid_3d(ctx->tiles);
     ctx->sample_cells = sample_cells_3d(d);
+}
+
+// The launches of step *clock + offset of a single 3D instance up to its mirror planes.
+void launch_step_3d(const yee_ctx* ctx, int32_t offset, hipStream_t stream)
+{
+    const yee3d_desc& d = ctx->d3;
+    if (ctx->fused) {
+        hipLaunchKernelGGL(d.n_poles > 0 ? yee3d_step_kernel<true> : yee3d_step_kernel<false>, dim3(ctx->blocks),
+                           dim3(kThreads3D), 0, stream, d, (int32_t)ctx->tiles, offset);
+        return;
+    }
+    hipLaunchKernelGGL(yee3d_h_kernel, dim3(ctx->blocks), dim3(256), 0, stream, d, offset);
+    hipLaunchKernelGGL(d.n_poles > 0 ? yee3d_e_kernel<true> : yee3d_e_kernel<false>, dim3(ctx->blocks), dim3(256), 0, stream,
+                       d, offset);
 }
 
 void drop_graph(yee_ctx* ctx)
@@ -904,8 +933,7 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
     if (ctx->kind == kSingle3D) {
         const int sample_blocks = (int)((ctx->sample_cells + 255) / 256);
         for (int32_t k = 0; k < count; ++k) {
-            hipLaunchKernelGGL(step_kernel_3d(ctx->d3), dim3(ctx->blocks), dim3(256), 0, stream, ctx->d3,
-                               ctx->tiles_j3, ctx->tiles_k3, (int32_t)ctx->tiles, k);
+            launch_step_3d(ctx, k, stream);
             launch_mirrors_3d(ctx->d3, k, stream);
             if (sample_blocks > 0)
                 hipLaunchKernelGGL(yee3d_sample_kernel, dim3(sample_blocks), dim3(256), 0, stream, ctx->d3,
@@ -926,8 +954,15 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
         const int sample_blocks = (int)((ctx->sample_cells + 255) / 256);
         const BatchAux3D a = batch_aux_3d(ctx->descs3.data(), ctx->n_inst);
         for (int32_t k = 0; k < count; ++k) {
-            hipLaunchKernelGGL(yee3d_batch_kernel<kRows3D>, dim3(ctx->blocks), dim3(256), 0, stream, ctx->descs3_dev,
-                               ctx->block_prefix_dev, ctx->n_inst, k);
+            if (ctx->fused) {
+                hipLaunchKernelGGL(yee3d_batch_kernel, dim3(ctx->blocks), dim3(kThreads3D), 0, stream, ctx->descs3_dev,
+                                   ctx->block_prefix_dev, ctx->n_inst, k);
+            } else {
+                hipLaunchKernelGGL(yee3d_batch_half_kernel<false>, dim3(ctx->blocks), dim3(256), 0, stream,
+                                   ctx->descs3_dev, ctx->block_prefix_dev, ctx->n_inst, k);
+                hipLaunchKernelGGL(yee3d_batch_half_kernel<true>, dim3(ctx->blocks), dim3(256), 0, stream,
+                                   ctx->descs3_dev, ctx->block_prefix_dev, ctx->n_inst, k);
+            }
             // mirror faces as a single instance orders them: every symmetric face, then the antisymmetric ones
             for (int kind = 0; kind < 2; ++kind)
                 for (int face = 0; face < 6; ++face)
@@ -1287,8 +1322,7 @@ int32_t step_timed_3d(yee_ctx* ctx, int64_t n_steps, hipStream_t s, double* kern
     int32_t status = YEE_OK;
     for (int64_t k = 0; k < n_steps && status == YEE_OK; ++k) {
         (void)hipEventRecord(ev[0], s);
-        hipLaunchKernelGGL(step_kernel_3d(ctx->d3), dim3(ctx->blocks), dim3(256), 0, s, d, ctx->tiles_j3,
-                           ctx->tiles_k3, (int32_t)ctx->tiles, 0);
+        launch_step_3d(ctx, 0, s);
         (void)hipEventRecord(ev[1], s);
         launch_mirrors_3d(d, 0, s);
         if (sample_blocks > 0)
@@ -1409,7 +1443,7 @@ int32_t yee3d_create(const yee3d_desc* desc, yee_ctx** out)
     if (!out) return fail(YEE_EINVAL, "null output pointer");
     *out = nullptr;
     yee3d_desc d = desc ? *desc : yee3d_desc{};
-    if (desc) apply_defaults_3d(d);
+    if (desc) apply_defaults_3d(d, cells_3d(d) >= kFused3D);
     int32_t status = check_3d(desc ? &d : nullptr);
     if (status != YEE_OK) return status;
     yee_ctx* ctx = new yee_ctx();
@@ -1424,7 +1458,7 @@ int32_t yee3d_update(yee_ctx* ctx, const yee3d_desc* desc)
 {
     if (!ctx || ctx->kind != kSingle3D) return fail(YEE_ESTATE, "not a 3D context");
     yee3d_desc d = desc ? *desc : yee3d_desc{};
-    if (desc) apply_defaults_3d(d);
+    if (desc) apply_defaults_3d(d, cells_3d(d) >= kFused3D);
     int32_t status = check_3d(desc ? &d : nullptr);
     if (status != YEE_OK) return status;
     drop_graph(ctx);
@@ -1441,12 +1475,15 @@ int32_t yee3d_batch_create(const yee3d_desc* descs, int32_t n, void* descs_dev, 
     std::vector<yee3d_desc> host(descs, descs + n);
     std::vector<int64_t> sample_prefix(n + 1, 0);
     std::vector<int32_t> block_prefix(n + 1, 0);
+    int64_t cells = 0;
+    for (const yee3d_desc& d : host) cells += cells_3d(d);
+    const bool fused = cells >= kFused3D;
     for (int32_t k = 0; k < n; ++k) {
-        apply_defaults_3d(host[k]);
+        apply_defaults_3d(host[k], fused);
         const int32_t status = check_3d(&host[k]);
         if (status != YEE_OK) return fail(status, "instance " + std::to_string(k) + ": " + g_last_error);
         if (host[k].rows_per_tile != kRows3D) return fail(YEE_EINVAL, "batched 3D instances use 4 rows per tile");
-        const int64_t next = block_prefix[k] + (tiles_3d(host[k]) + 3) / 4;
+        const int64_t next = block_prefix[k] + blocks_3d(host[k], fused);
         if (next > INT32_MAX / 2) return fail(YEE_EINVAL, "batch has too many tiles");
         block_prefix[k + 1] = (int32_t)next;
         sample_prefix[k + 1] = sample_prefix[k] + sample_cells_3d(host[k]);
@@ -1467,8 +1504,9 @@ int32_t yee3d_batch_create(const yee3d_desc* descs, int32_t n, void* descs_dev, 
     ctx->sample_prefix_dev = dev_samples;
     ctx->block_prefix_dev = dev_blocks;
     ctx->n_inst = n;
-    ctx->blocks = block_prefix[n];
-    ctx->tiles = (int64_t)block_prefix[n] * 4;
+    ctx->fused = fused;
+    ctx->blocks = grid_3d(block_prefix[n]);
+    ctx->tiles = block_prefix[n];
     ctx->sample_cells = sample_prefix[n];
     *out = ctx;
     return YEE_OK;
