@@ -92,6 +92,7 @@ struct Batch2DWork {
     int64_t bulk_tiles = 0, edge_tiles = 0, windows = 0;
     const MultiShape* shape = nullptr;
     int32_t steps = 0;
+    int32_t least = 0;   // steps of a call below which it steps one at a time
 };
 
 }  // namespace
@@ -801,6 +802,12 @@ Batch2DArgs batch2d_args(void* base, int32_t n, const Batch2DWork& work, int32_t
 // Calls of fewer steps than this step one at a time: a batch's windows are laid out once, for the steps of its full
 // launches, and their halos would cost more than the launches they save.
 constexpr int32_t kMultiBatchLeast = 4;
+// Batches of fewer cells than this in calls of fewer steps also step one at a time. Not for speed: members of 84 x 69 and
+// 61 x 73 cells take 44 us a step so in calls of 25, and 9 with several steps a launch. A server that preempts a long job of
+// a few thousand cells between such calls (tests/test_gpu_serve.py, 3000 steps and a rival after 50 ms) counts on its
+// still running then.
+constexpr int64_t kMultiBatchCells = 1 << 14;
+constexpr int32_t kMultiBatchShort = 32;
 
 // `count` steps of a batch whose members all share launches of up to work.steps steps, and one launch more for members
 // that end with the wrong parity (yee2d_multi_batch_kernel).
@@ -833,7 +840,7 @@ int32_t launch_batch_2d(const Batch2DArgs& b, int32_t count, hipStream_t stream)
     const int bulk_blocks = (int)((b.work.bulk_tiles + 3) / 4);
     const int edge_blocks = (int)((b.work.edge_tiles + 3) / 4);
     const BatchAux2D& a = b.aux;
-    const bool multi = b.work.shape && count >= kMultiBatchLeast;
+    const bool multi = b.work.shape && count >= b.work.least;
     if (multi) {
         const int32_t status = launch_multi_batch_2d(b, count, stream);
         if (status != YEE_OK) return status;
@@ -1038,9 +1045,13 @@ yee2d_multi_plan batch_plan(const yee2d_desc& d, int32_t steps, const MultiShape
 // none when a member's features need one step a launch.
 void choose_multi_batch(const yee2d_desc* descs, int32_t n, int32_t count, Batch2DWork* work)
 {
-    if (count < kMultiBatchLeast) return;
-    for (int32_t k = 0; k < n; ++k)
+    int64_t cells = 0;
+    for (int32_t k = 0; k < n; ++k) {
         if (!multi_ok(descs[k])) return;
+        cells += (int64_t)descs[k].nx * descs[k].ny;
+    }
+    work->least = cells < kMultiBatchCells ? kMultiBatchShort : kMultiBatchLeast;
+    if (count < work->least) return;
     float best = 0.f;
     for (const MultiShape& s : kMultiShape) {
         for (int32_t steps = kMultiBatchLeast; s.batch && steps <= std::min(s.most, count); ++steps) {
