@@ -407,8 +407,9 @@ int32_t yee2d_create(const yee2d_desc* desc, yee_ctx** out);
 /*
  * Advance by n_steps steps on `stream` (hipStream_t; 0 = the null stream). Launches only: no allocation, no sync.
  * Whole chunks of graph_steps steps replay a cached HIP graph when graph_steps > 0. A single 2D instance whose features
- * allow it (no poles, TFSF, walls, DFT regions or probes; no step limit) advances several steps per launch, chosen by
- * the size of the grid and n_steps; the others one step per launch.
+ * allow it (no TFSF or walls, at most 64 probes, no pole but one Drude pole of an E_z instance with a work array, DFT
+ * regions of cell values or of face means along the face's normal; no step limit) advances several steps per launch,
+ * chosen by the size of the grid and n_steps; the others one step per launch.
  * Replaces coupling/runner.py:174-204 (advance) -> EMPhysics.step (physics/em/__init__.py:163-168).
  */
 int32_t yee_step(yee_ctx* ctx, int64_t n_steps, void* stream);
@@ -442,6 +443,16 @@ int32_t yee2d_update(yee_ctx* ctx, const yee2d_desc* desc);
  * yee2d_update keeps it. The reference has one kernel form (physics/em/solvers/fdtd_hz_2d_kernels.py:28-155).
  */
 int32_t yee2d_set_lossless(yee_ctx* ctx, int32_t lossless);
+
+/*
+ * Work array of an instance with a single Drude pole, and no other: (i1 - i0) * (j1 - j0) device floats of any content, held
+ * by the caller until the context is destroyed, the descriptor replaced (yee2d_update forgets it) or another one set
+ * (NULL: none). With it an E_z instance can advance several steps per launch, which pass the pole's current through
+ * state[0] and this array in turn; between calls the current is in state[0], as without it. Same bits either way. Drops
+ * cached graphs. The reference updates the current in place, one step at a time
+ * (physics/em/solvers/fdtd_ez_2d.py:262-358).
+ */
+int32_t yee2d_set_pole_work(yee_ctx* ctx, float* work);
 
 /* The descriptor a single 2D context steps, with the defaults it resolved (rows_per_tile, lane_columns). */
 int32_t yee2d_get_desc(const yee_ctx* ctx, yee2d_desc* out);

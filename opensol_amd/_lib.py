@@ -129,6 +129,7 @@ SIGNATURES = (
     ('yee_build_graph', c_i32, (c_ptr,)),
     ('yee2d_update', c_i32, (c_ptr, ctypes.POINTER(Desc2DC))),
     ('yee2d_set_lossless', c_i32, (c_ptr, c_i32)),
+    ('yee2d_set_pole_work', c_i32, (c_ptr, c_ptr)),
     ('yee2d_get_desc', c_i32, (c_ptr, ctypes.POINTER(Desc2DC))),
     ('yee3d_create', c_i32, (ctypes.POINTER(Desc3DC), ctypes.POINTER(c_ptr))),
     ('yee3d_update', c_i32, (c_ptr, ctypes.POINTER(Desc3DC))),

@@ -24,6 +24,11 @@
 // Two forms of a window: the lean one lies, halo included, inside the grid and outside every CPML layer; the general
 // one takes grid edges, periodic wraps and CPML. Cells outside the grid take a table entry of zeros, so they stay 0
 // without selects. Sheet sources and flux lines are applied in both.
+//
+// EXTRA windows also take the DFT regions, the field probes and a Drude pole of an E_z instance, which one-step launches
+// serve with two kernels more a step: a sampled cell or probe is taken from the registers of the window that owns it, the
+// pole's current lives in registers beside E_z (its drive in LDS) and passes from launch to launch through two arrays in
+// turn. They are instantiations of their own: the current costs the registers of half a field.
 #pragma once
 
 #include "yee2d_cells.h"
@@ -37,6 +42,7 @@ __shared__ float lds_profile[YEE_MAX_SOURCES * 128];      // source profiles alo
 __shared__ float lds_up[kMultiWavesMax * 128];            // the row each wavefront hands down (its lowest)
 __shared__ float lds_down[kMultiWavesMax * 128];          // the row each wavefront hands up (its highest)
 __shared__ float lds_sigma[kMultiIds / 2];                // H_z: sigma_e per id
+__shared__ float lds_drive[kMultiCells];                  // Drude pole: drive of the window's cells, by lane
 
 // value of the next / previous lane (0 past the wavefront's ends, which only halo columns see)
 __device__ __forceinline__ float lane_next(float v)
@@ -63,7 +69,7 @@ __device__ __forceinline__ float4 coef_at(uint32_t byte_offset)
 // Sheet sources and flux lines (bits of d.source, d.monitor) that reach a window: a source with any of its cells (or any
 // window that wraps around a periodic axis), a flux line with owned ones.
 struct WindowRecords {
-    uint32_t sources, monitors;
+    uint32_t sources, monitors, regions;   // regions: DFT regions with owned cells (EXTRA)
 };
 
 struct Window {
@@ -74,7 +80,7 @@ struct Window {
 
 __device__ __forceinline__ WindowRecords window_records(const yee2d_desc& d, const Window& w, int columns)
 {
-    WindowRecords out{0, 0};
+    WindowRecords out{0, 0, 0};
     const bool wrap_x = d.periodic_x != 0 && (w.w0 < 0 || w.w0 + w.rows > d.nx);
     const bool wrap_y = d.periodic_y != 0 && (w.k0 < 0 || w.k0 + columns > d.ny);
     for (int s = 0; s < d.n_sources; ++s) {
@@ -93,6 +99,29 @@ __device__ __forceinline__ WindowRecords window_records(const yee2d_desc& d, con
         if (r0 < w.i1 && r1 > w.i0 && k0 < w.c1 && k1 > w.c0) out.monitors |= 1u << m;
     }
     return out;
+}
+
+// DFT regions with sampled cells among the owned ones (by their bounding boxes).
+__device__ __forceinline__ uint32_t window_regions(const yee2d_desc& d, const Window& w)
+{
+    uint32_t out = 0;
+    for (int k = 0; k < d.n_dft; ++k) {
+        const yee_dft_region& g = d.dft[k];
+        if (g.start[0] < w.i1 && g.start[0] + g.stride[0] * (g.count[0] - 1) >= w.i0 && g.start[1] < w.c1 &&
+            g.start[1] + g.stride[1] * (g.count[1] - 1) >= w.c0)
+            out |= 1u << k;
+    }
+    return out;
+}
+
+// Whether a window, halo included, may meet the box of a Drude pole (one that wraps around a periodic axis may).
+__device__ __forceinline__ bool window_pole(const yee2d_desc& d, const Window& w, int columns)
+{
+    if (d.n_poles == 0) return false;
+    const yee_pole& p = d.pole[0];
+    const bool wrap_x = d.periodic_x != 0 && (w.w0 < 0 || w.w0 + w.rows > d.nx);
+    const bool wrap_y = d.periodic_y != 0 && (w.k0 < 0 || w.k0 + columns > d.ny);
+    return (wrap_x || (p.i0 < w.w0 + w.rows && p.i1 > w.w0)) && (wrap_y || (p.j0 < w.k0 + columns && p.j1 > w.k0));
 }
 
 template <int VEC>
@@ -257,7 +286,7 @@ struct WindowEarly {
 // E_x) and fy the one on the hi-x faces (H_y or E_y). EDGE: the general form; XL: some of its rows lie in an x CPML
 // layer; FULL: materials that are not simple (stage_multi_tables). Simple forms keep 1 * x in the updates: exact, and the
 // rounding of each expression stays that of the general one.
-template <int POL, int VEC, int R, int NW, bool EDGE, bool XL, bool FULL>
+template <int POL, int VEC, int R, int NW, bool EDGE, bool XL, bool FULL, bool EXTRA, bool POLE>
 struct MultiWindow {
     static constexpr bool HZ = POL == YEE_HZ;
     using Early = WindowEarly<VEC, R, EDGE>;
@@ -276,6 +305,14 @@ struct MultiWindow {
     float cax[FULL && HZ ? R : 1][VEC], cay[FULL && HZ ? R : 1][VEC];
     float cbx[HZ || !FULL ? R : 1][VEC], cby[HZ ? R : 1][VEC];
     float yh[EDGE ? R : 1][VEC], ye[EDGE ? R : 1][VEC], xh[XL ? R : 1][VEC], xe[XL ? R : 1][VEC];
+    // Drude pole: current of the cells, the rows (bits) and elements (bits) inside its box
+    float jp[POLE ? R : 1][VEC];
+    uint32_t pole_rows, pole_cols;
+    float damping;
+    // Probes (EXTRA): lane p holds probe p as component << 16 | row of the wavefront << 8 | column of the window
+    // (bits of probes_mine: those on owned cells of this wavefront), or the value of one outside the grid (probes_stray)
+    uint64_t probes_mine, probes_stray;
+    uint32_t probe;
 
     __device__ __forceinline__ MultiWindow(const yee2d_desc& desc, const Window& window) : d(desc), w(window) {}
 
@@ -440,6 +477,57 @@ struct MultiWindow {
         return k == 0 ? prev : v[k > 0 ? k - 1 : 0];
     }
 
+    // The drive of a cell (read and written by its own lane only).
+    static __device__ __forceinline__ float& drive(int r, int k)
+    {
+        return lds_drive[(r * VEC + k) * 64 * NW + threadIdx.x];
+    }
+
+    // Current and drive of the cells inside the pole's box; launch `launch` of a call reads state[launch & 1].
+    __device__ __forceinline__ void load_pole(int launch)
+    {
+        pole_rows = pole_cols = 0;
+        const yee_pole& p = d.pole[0];
+        damping = uniform(p.damping);
+        const float* __restrict__ state = p.state[launch & 1];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            const int at = col.column(k);
+            pole_cols |= (uint32_t)(at >= p.j0 && at < p.j1) << k;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int f = fold_row(q0 + r);
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) jp[r][k] = 0.f;
+            if (f < p.i0 || f >= p.i1) continue;
+            pole_rows |= 1u << r;
+            const int64_t base = (int64_t)(f - p.i0) * (p.j1 - p.j0) - p.j0;
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                if (!((pole_cols >> k) & 1)) continue;
+                jp[r][k] = state[base + col.column(k)];
+                drive(r, k) = p.drive[base + col.column(k)];
+            }
+        }
+    }
+
+    __device__ __forceinline__ void store_pole(int launch) const
+    {
+        if (!col.owner) return;
+        const yee_pole& p = d.pole[0];
+        float* __restrict__ state = p.state[(launch & 1) ^ 1];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int q = q0 + r;
+            if (!((pole_rows >> r) & 1) || q < w.i0 || q >= w.i1) continue;
+            const int64_t base = (int64_t)(q - p.i0) * (p.j1 - p.j0) - p.j0;
+#pragma unroll
+            for (int k = 0; k < VEC; ++k)
+                if ((pole_cols >> k) & 1) state[base + col.column(k)] = jp[r][k];
+        }
+    }
+
     // (ca, cb, da, db) of an E_z cell
     __device__ __forceinline__ float4 ez_coef(int r, int k) const
     {
@@ -491,6 +579,15 @@ struct MultiWindow {
             if constexpr (EDGE) {
                 ye[r][k] = col.b_e[k] * ye[r][k] + col.g_e[k] * dhx;
                 v -= m.y * ye[r][k];
+            }
+            if constexpr (POLE) {
+                const bool inside = (pole_rows >> r) & 1 && (pole_cols >> k) & 1;   // selects: what lies outside keeps
+                float jc = jp[r][k];                                                // its infinities and NaN
+                jc += damping * jc + drive(r, k) * c[r][k];
+                float u = v;
+                u -= m.y * jc;
+                jp[r][k] = inside ? jc : jp[r][k];
+                v = inside ? u : v;
             }
             c[r][k] = v;
         }
@@ -678,6 +775,121 @@ struct MultiWindow {
         }
     }
 
+    // Row q0 + r (r uniform) of field `component`: selects, because an indexed access, or a choice between the arrays,
+    // would move the fields to scratch memory.
+    __device__ __forceinline__ void pick(int component, int r, float out[VEC]) const
+    {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            float a = c[0][k], b = fx[0][k], e = fy[0][k];
+#pragma unroll
+            for (int q = 1; q < R; ++q) {
+                a = q == r ? c[q][k] : a;
+                b = q == r ? fx[q][k] : b;
+                e = q == r ? fy[q][k] : e;
+            }
+            out[k] = component == 0 ? a : component == 1 ? b : e;
+        }
+    }
+
+    // DFT regions' samples of the owned cells after `done` steps. A mean with the lower neighbour along x needs the row
+    // that the wavefront below holds: every wavefront of the block takes part in that exchange.
+    __device__ __forceinline__ void sample_regions(uint32_t regions, int64_t done, float* down, const float* from_below)
+    {
+        const int64_t index = done / d.sample_interval - 1;
+        float row[VEC];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) down[k] = fy[R - 1][k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) row[k] = from_below[k];
+        __syncthreads();
+        for (uint32_t rest = regions; rest; rest &= rest - 1) {
+            const yee_dft_region& g = d.dft[__builtin_ctz(rest)];
+            if (index >= g.n_samples) continue;
+            const int64_t cells = (int64_t)g.count[0] * g.count[1];
+            const int step = g.stride[0];
+            const int first = max(max(w.i0, q0), g.start[0]);
+            const int end = min(min(w.i1, q0 + R), g.start[0] + step * (g.count[0] - 1) + 1);
+            int64_t along[VEC];   // sampled column of element k, -1 for none
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                const int at = col.column(k), from = at - g.start[1];
+                const bool hit = col.owner && at < d.ny && from >= 0 && from % g.stride[1] == 0 &&
+                                 from / g.stride[1] < g.count[1];
+                along[k] = hit ? from / g.stride[1] : -1;
+            }
+            int t0 = (first - g.start[0] + step - 1) / step;
+            for (int q = g.start[0] + t0 * step; q < end; q += step, ++t0) {
+                const int r = q - q0;
+                for (int s = 0; s < g.n_comp; ++s) {
+                    float v[VEC], low[VEC];
+                    pick(g.comp[s], r, v);
+                    const bool self = !g.pair_wrap[s];   // the lower neighbour of index 0 is the cell itself
+                    const float prev = lane_prev(v[VEC - 1]);
+                    if (g.pair_axis[s] == 0) {
+                        pick(2, r - 1, low);
+#pragma unroll
+                        for (int k = 0; k < VEC; ++k) {
+                            low[k] = r == 0 ? row[k] : low[k];
+                            low[k] = q == 0 && self ? v[k] : low[k];
+                        }
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < VEC; ++k) low[k] = col.column(k) == 0 && self ? v[k] : left(v, k, prev);
+                    }
+#pragma unroll
+                    for (int k = 0; k < VEC; ++k) {
+                        if (along[k] < 0) continue;
+                        const float x = g.pair_axis[s] >= 0 ? 0.5f * (v[k] + low[k]) : v[k];
+                        dft_region_add(g, s, cells, (int64_t)t0 * g.count[1] + along[k], index, x);
+                    }
+                }
+            }
+        }
+    }
+
+    // The probes of this wavefront, at most 64 (the host's rule); the window of cell (0, 0) takes those outside the grid.
+    __device__ __forceinline__ void find_probes()
+    {
+        probes_mine = probes_stray = 0;
+        probe = 0;
+        if (d.probes.n_probes == 0) return;
+        const int p = threadIdx.x & (YEE_WAVE - 1);
+        bool mine = false, stray = false;
+        if (p < d.probes.n_probes) {
+            const int64_t cell = d.probes.cell[p];
+            const int32_t component = d.probes.component[p];
+            const bool known = component >= 0 && component < 3 && cell >= 0 && cell < (int64_t)d.nx * d.pitch;
+            const int32_t i = known ? (int32_t)(cell / d.pitch) : 0;
+            const int32_t j = known ? (int32_t)(cell - (int64_t)i * d.pitch) : 0;
+            stray = !known || j >= d.ny;   // past the grid: NaN; a padding column: what it holds (0)
+            mine = !stray && i >= max(q0, w.i0) && i < min(q0 + R, w.i1) && j >= w.c0 && j < w.c1;
+            stray = stray && wave == 0 && w.i0 == 0 && w.c0 == 0;
+            if (mine) probe = (uint32_t)component << 16 | (uint32_t)(i - q0) << 8 | (uint32_t)(j - w.k0);
+            if (stray) probe = __float_as_uint(known ? d.field[par][component][cell] : __builtin_nanf(""));
+        }
+        probes_mine = __ballot(mine);
+        probes_stray = __ballot(stray);
+    }
+
+    // Probe samples of step `step` (row `step` of the table).
+    __device__ __forceinline__ void sample_probes(int64_t step) const
+    {
+        if (step >= d.probes.capacity) return;
+        float* const row = d.probes.samples + step * d.probes.n_probes;
+        const int lane = threadIdx.x & (YEE_WAVE - 1);
+        if ((probes_stray >> lane) & 1) row[lane] = __uint_as_float(probe);
+        for (uint64_t left = probes_mine; left; left &= left - 1) {
+            const int p = __builtin_ctzll(left);
+            const uint32_t word = __builtin_amdgcn_readlane(probe, p);
+            const int component = word >> 16, r = (word >> 8) & 0xff, column = word & 0xff;
+            float v[VEC];
+            pick(component, r, v);
+            if (lane == column / VEC) row[p] = VEC > 1 && column % VEC ? v[VEC - 1] : v[0];
+        }
+    }
+
     __device__ __forceinline__ void store()
     {
         if (!col.owner) return;
@@ -761,7 +973,7 @@ struct MultiWindow {
     }
 
     // The second round of loads, behind the first one's results (Early): constants by psi row, fields and psi.
-    __device__ __forceinline__ void begin(const Early& early, int64_t n_start, int set)
+    __device__ __forceinline__ void begin(const Early& early, int64_t n_start, int set, int launch)
     {
         n = n_start;
         par = set;
@@ -797,9 +1009,11 @@ struct MultiWindow {
         } else {
             load();
         }
+        if constexpr (EXTRA) find_probes();
+        if constexpr (POLE) load_pole(launch);
     }
 
-    __device__ __forceinline__ void run(int steps, const Early& early, const WindowRecords& records)
+    __device__ __forceinline__ void run(int steps, const Early& early, const WindowRecords& records, int launch)
     {
         if (records.sources) stage_sources(records.sources, steps);
         finish(early);
@@ -812,48 +1026,69 @@ struct MultiWindow {
         float* const down = lds_down + wave * 128 + VEC * lane;
         const float* const from_above = lds_up + (wave + 1 < NW ? wave + 1 : wave) * 128 + VEC * lane;
         const float* const from_below = lds_down + (wave > 0 ? wave - 1 : 0) * 128 + VEC * lane;
-        int left = records.monitors ? d.sample_interval - (int)(n % d.sample_interval) : 0;   // steps to the next sample
+        int left = records.monitors | records.regions ? d.sample_interval - (int)(n % d.sample_interval) : 0;   // steps to the next sample
         for (int s = 0; s < steps; ++s) {
             if constexpr (HZ) hz_step(up, down, from_above, from_below, mine, s);
             else ez_step(up, down, from_above, from_below);
             if (mine) add_sources(mine, YEE_SOURCE_E, s);
-            if (records.monitors && --left == 0) {
+            if ((records.monitors | records.regions) && --left == 0) {
                 sample(records.monitors, n + s + 1);
+                if constexpr (EXTRA)
+                    if (records.regions) sample_regions(records.regions, n + s + 1, down, from_below);
                 left = d.sample_interval;
             }
+            if constexpr (EXTRA)
+                if (probes_mine | probes_stray) sample_probes(n + s);
         }
         store();
+        if constexpr (POLE) store_pole(launch);
     }
 };
 
 // One window of `steps` steps: a first round of loads with the tables among them, the choice of the form, a second round
 // behind the first one's results, the steps and the stores. The two rounds are what a launch waits for before it steps.
-template <int POL, int VEC, int R, int NW, bool EDGE, bool XL>
+template <int POL, int VEC, int R, int NW, bool EDGE, bool XL, bool EXTRA>
 __device__ __forceinline__ void run_window(const yee2d_desc& d, const Window& w, int64_t clock, int32_t offset,
                                            int32_t launch, int steps)
 {
-    const WindowRecords records = window_records(d, w, 64 * VEC);
+    WindowRecords records = window_records(d, w, 64 * VEC);
+    if constexpr (EXTRA) records.regions = window_regions(d, w);
     WindowEarly<VEC, R, EDGE> early;
-    MultiWindow<POL, VEC, R, NW, EDGE, XL, false>::early(d, w, early);
+    MultiWindow<POL, VEC, R, NW, EDGE, XL, false, EXTRA, false>::early(d, w, early);
     const bool odd = stage_multi_tables<POL, NW>(d);
     clock = (int64_t)__builtin_amdgcn_readfirstlane((int)(clock >> 32)) << 32 |
             (uint32_t)__builtin_amdgcn_readfirstlane((int)clock);
     const int64_t n = clock + offset;
     const int set = (int)((clock + launch) & 1);
-    if (__syncthreads_or(odd)) {
-        MultiWindow<POL, VEC, R, NW, EDGE, XL, true> window(d, w);
-        window.begin(early, n, set);
-        window.run(steps, early, records);
+    const bool full = __syncthreads_or(odd);
+    const auto run = [&](auto& window) {
+        window.begin(early, n, set, launch);
+        window.run(steps, early, records, launch);
+    };
+    if constexpr (EXTRA && POL == YEE_EZ) {
+        if (window_pole(d, w, 64 * VEC)) {
+            if (full) {
+                MultiWindow<POL, VEC, R, NW, EDGE, XL, true, true, true> window(d, w);
+                run(window);
+            } else {
+                MultiWindow<POL, VEC, R, NW, EDGE, XL, false, true, true> window(d, w);
+                run(window);
+            }
+            return;
+        }
+    }
+    if (full) {
+        MultiWindow<POL, VEC, R, NW, EDGE, XL, true, EXTRA, false> window(d, w);
+        run(window);
     } else {
-        MultiWindow<POL, VEC, R, NW, EDGE, XL, false> window(d, w);
-        window.begin(early, n, set);
-        window.run(steps, early, records);
+        MultiWindow<POL, VEC, R, NW, EDGE, XL, false, EXTRA, false> window(d, w);
+        run(window);
     }
 }
 
 // Window `block` of one instance, in the form its place asks for: `steps` steps (at most plan.steps, which the windows'
 // halo is laid out for).
-template <int POL, int VEC, int R, int TV, int TR, int NW>
+template <int POL, int VEC, int R, int TV, int TR, int NW, bool EXTRA>
 __device__ __forceinline__ void multi_block(const yee2d_desc& d, const yee2d_multi_plan& plan, int block, int64_t clock,
                                             int32_t offset, int32_t launch, int steps)
 {
@@ -876,18 +1111,18 @@ __device__ __forceinline__ void multi_block(const yee2d_desc& d, const yee2d_mul
     w.k0 = w.c0 - yee2d_multi_halo(t, tall ? TV : VEC);
     if constexpr (TR > 0) {
         if (tall) {
-            run_window<POL, TV, TR, NW, false, false>(d, w, clock, offset, launch, steps);
+            run_window<POL, TV, TR, NW, false, false, EXTRA>(d, w, clock, offset, launch, steps);
             return;
         }
     }
     const bool lean = w.w0 >= 0 && w.w0 >= d.layer_x_lo && w.w0 + w.rows < d.nx && w.w0 + w.rows <= d.layer_x_hi &&
                       w.k0 >= 0 && w.k0 >= d.layer_y_lo && w.k0 + columns < d.ny && w.k0 + columns <= d.layer_y_hi;
     if (lean)
-        run_window<POL, VEC, R, NW, false, false>(d, w, clock, offset, launch, steps);
+        run_window<POL, VEC, R, NW, false, false, EXTRA>(d, w, clock, offset, launch, steps);
     else if (d.cpml[0].n_rows == 0 || (w.w0 >= d.layer_x_lo && w.w0 + w.rows <= d.layer_x_hi))
-        run_window<POL, VEC, R, NW, true, false>(d, w, clock, offset, launch, steps);
+        run_window<POL, VEC, R, NW, true, false, EXTRA>(d, w, clock, offset, launch, steps);
     else
-        run_window<POL, VEC, R, NW, true, true>(d, w, clock, offset, launch, steps);
+        run_window<POL, VEC, R, NW, true, true, EXTRA>(d, w, clock, offset, launch, steps);
 }
 
 }  // namespace yee

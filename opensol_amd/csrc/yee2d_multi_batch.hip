@@ -37,9 +37,9 @@ __global__ void __launch_bounds__(64 * NW, 4)
     }
     const int index = block - __builtin_amdgcn_readfirstlane(prefix[lo]);
     if (d.polarization == YEE_EZ)
-        yee::multi_block<YEE_EZ, VEC, R, TV, TR, NW>(d, plan, index, clock, offset, launch, take);
+        yee::multi_block<YEE_EZ, VEC, R, TV, TR, NW, false>(d, plan, index, clock, offset, launch, take);
     else
-        yee::multi_block<YEE_HZ, VEC, R, TV, 0, NW>(d, plan, index, clock, offset, launch, take);
+        yee::multi_block<YEE_HZ, VEC, R, TV, 0, NW, false>(d, plan, index, clock, offset, launch, take);
 }
 
 #define YEE_MULTI_BATCH_KERNEL(VEC, R, TV, TR, NW)                                                                    \

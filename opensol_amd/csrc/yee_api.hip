@@ -20,8 +20,9 @@ __global__ void yee2d_step_kernel(yee2d_desc d, yee2d_tile_sets sets, int32_t of
 template <int VEC, bool EDGE, bool LEFT>
 __global__ void yee2d_batch_kernel(const yee2d_desc* __restrict__ descs, const yee2d_tile_sets* __restrict__ sets,
                                    const int32_t* __restrict__ prefix, int32_t n_inst, int32_t offset);
-template <int POL, int VEC, int R, int TV, int TR, int NW>
+template <int POL, int VEC, int R, int TV, int TR, int NW, bool EXTRA>
 __global__ void yee2d_multi_kernel(yee2d_desc d, yee2d_multi_plan plan, int32_t offset, int32_t launch);
+__global__ void yee2d_pole_copy_kernel(const float* __restrict__ from, float* __restrict__ to, int64_t count);
 template <int VEC, int R, int TV, int TR, int NW>
 __global__ void yee2d_multi_batch_kernel(const yee2d_desc* __restrict__ descs, const yee2d_multi_plan* __restrict__ plans,
                                          const int32_t* __restrict__ prefix, int32_t n_inst, int32_t offset,
@@ -458,12 +459,35 @@ bool has_walls(const yee2d_desc& d)
 }
 
 // Whether several steps of an instance can share a launch: no feature that reads or writes the state between steps
-// outside the multi-step kernel, and a coefficient table that fits its LDS. (A step limit is for batches only.)
-bool multi_ok(const yee2d_desc& d)
+// outside the multi-step kernels, and a coefficient table that fits their LDS. `extra`: the features of the EXTRA kernels
+// are allowed, namely a single Drude pole of an E_z instance with its work array (yee2d_set_pole_work), at most a probe a
+// lane, and DFT regions of values at the cells or of face means as the windows form them. (A step limit is for batches.)
+bool multi_ok(const yee2d_desc& d, bool extra)
 {
     const int ids = d.polarization == YEE_EZ ? kMultiIds : kMultiIds / 2;   // H_z keeps two entries an id
-    return d.n_poles == 0 && d.n_tfsf == 0 && !has_walls(d) && d.n_dft == 0 && d.probes.n_probes == 0 &&
-           d.n_materials < ids;
+    if (d.n_tfsf != 0 || has_walls(d) || d.n_materials >= ids) return false;
+    if (!extra) return d.n_poles == 0 && d.n_dft == 0 && d.probes.n_probes == 0;
+    if (d.n_poles > 1 || d.probes.n_probes > kMultiProbes) return false;
+    if (d.n_poles == 1 && (d.polarization != YEE_EZ || d.pole[0].kind != YEE_DRUDE || !d.pole[0].state[1])) return false;
+    for (int k = 0; k < d.n_dft; ++k)
+        for (int c = 0; c < d.dft[k].n_comp; ++c) {
+            const int a = d.dft[k].pair_axis[c];
+            const int face = a == 0 ? 2 : 1;   // the mean along x is one of hi-x faces, along y of hi-y faces
+            if (a >= 0 && d.dft[k].comp[c] != face) return false;
+            if (a >= 0 && d.dft[k].pair_wrap[c] && !(a == 0 ? d.periodic_x : d.periodic_y)) return false;
+        }
+    return true;
+}
+
+bool multi_extra(const yee2d_desc& d) { return d.n_poles > 0 || d.n_dft > 0 || d.probes.n_probes > 0; }
+
+// Rows and columns of halo past a launch's steps: one for face means, which read one face below the owned cells.
+int32_t multi_pad(const yee2d_desc& d)
+{
+    for (int k = 0; k < d.n_dft; ++k)
+        for (int c = 0; c < d.dft[k].n_comp; ++c)
+            if (d.dft[k].pair_axis[c] >= 0) return 1;
+    return 0;
 }
 
 typedef void (*MultiKernel)(yee2d_desc, yee2d_multi_plan, int32_t, int32_t);
@@ -477,7 +501,7 @@ struct MultiShape {
     // time of a launch of t steps (multi_time): fixed + step * t us while its windows fit the chip side by side, and
     // window_fixed + window_step * t ns more for every further window (the first mostly its loads and stores)
     float fixed, step, window_fixed, window_step;
-    MultiKernel kernel[2];  // by polarisation
+    MultiKernel kernel[2][2];  // by polarisation; [1]: with DFT regions, probes and a pole (multi_extra)
     MultiBatchKernel batch; // for batches (null: a shape for few windows only)
 };
 template <int VEC, int R, int TV, int TR, int NW>
@@ -485,7 +509,10 @@ MultiShape multi_shape(int most, float fixed, float step, float window_fixed, fl
                        MultiBatchKernel batch)
 {
     return MultiShape{VEC, R, TV, TR, NW, most, fixed, step, window_fixed, window_step,
-                      {yee2d_multi_kernel<YEE_EZ, VEC, R, TV, TR, NW>, yee2d_multi_kernel<YEE_HZ, VEC, R, TV, TR, NW>},
+                      {{yee2d_multi_kernel<YEE_EZ, VEC, R, TV, TR, NW, false>,
+                        yee2d_multi_kernel<YEE_EZ, VEC, R, TV, TR, NW, true>},
+                       {yee2d_multi_kernel<YEE_HZ, VEC, R, TV, TR, NW, false>,
+                        yee2d_multi_kernel<YEE_HZ, VEC, R, TV, TR, NW, true>}},
                       batch};
 }
 // Small windows step fastest while there are few of them, tall ones waste least on their halo. Measured (us a step, E_z,
@@ -508,12 +535,14 @@ void add_region(yee2d_multi_plan& p, int32_t i0, int32_t i1, int32_t j0, int32_t
     p.blocks += (i1 - i0 + rows - 1) / rows * g.tiles_j;
 }
 
-// The windows of a launch of `steps` steps: with `tall` the lean windows that fit, halo included, between the CPML
+// The windows of a launch of `take` steps: with `tall` the lean windows that fit, halo included, between the CPML
 // layers, and general windows on the frame around them; else general windows everywhere.
-yee2d_multi_plan multi_plan(const yee2d_desc& d, int32_t steps, const MultiShape& shape, bool tall)
+yee2d_multi_plan multi_plan(const yee2d_desc& d, int32_t take, const MultiShape& shape, bool tall)
 {
+    const int32_t steps = take + multi_pad(d);
     yee2d_multi_plan p{};
     p.steps = steps;
+    p.take = take;
     const int32_t rows = yee2d_multi_rows(steps, shape.waves, shape.r), columns = yee2d_multi_columns(steps, shape.vec);
     if (tall && shape.tall_r) {
         const int32_t high = yee2d_multi_rows(steps, shape.waves, shape.tall_r);
@@ -570,7 +599,7 @@ void choose_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, i
     float best = 0.f;
     *shape = nullptr;
     for (const MultiShape& s : kMultiShape)
-        for (int32_t most = 1; most <= std::min(s.most, count); ++most) {
+        for (int32_t most = 1; most <= std::min(s.most - multi_pad(ctx->d2), count); ++most) {
             const int32_t n = multi_launches(count, most);
             const int32_t steps = multi_steps(count, n, 0);
             const float time = n * multi_time(multi_plan(ctx->d2, steps, s, tall_windows(ctx)).blocks, steps, s);
@@ -582,9 +611,16 @@ void choose_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, i
         }
 }
 
+// A descriptor's Drude poles say nothing in state[1]; a context keeps the work array there (yee2d_set_pole_work).
+void clear_pole_work(yee2d_desc& d)
+{
+    for (int p = 0; p < d.n_poles; ++p)
+        if (d.pole[p].kind == YEE_DRUDE) d.pole[p].state[1] = nullptr;
+}
+
 void set_geometry(yee_ctx* ctx)
 {
-    ctx->multi = multi_ok(ctx->d2) && ctx->d2.step_limit == INT64_MAX;
+    ctx->multi = multi_ok(ctx->d2, true) && ctx->d2.step_limit == INT64_MAX;
     const yee2d_desc& d = ctx->d2;
     ctx->sets = tile_sets(d);
     const yee2d_tile_sets& s = ctx->sets;
@@ -889,9 +925,15 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
         for (int32_t k = 0, offset = 0; k < launches; ++k) {
             const yee2d_multi_plan plan = multi_plan(ctx->d2, multi_steps(count, launches, k), *shape, tall_windows(ctx));
             const int blocks = (plan.blocks + 7) / 8 * 8;   // a multiple of the XCDs
-            hipLaunchKernelGGL(shape->kernel[ctx->d2.polarization], dim3(blocks), dim3(64 * shape->waves), 0, stream,
-                               ctx->d2, plan, offset, k);
-            offset += plan.steps;
+            hipLaunchKernelGGL(shape->kernel[ctx->d2.polarization][multi_extra(ctx->d2)], dim3(blocks),
+                               dim3(64 * shape->waves), 0, stream, ctx->d2, plan, offset, k);
+            offset += plan.take;
+        }
+        if (ctx->d2.n_poles > 0 && launches % 2 == 1) {
+            const yee_pole& p = ctx->d2.pole[0];
+            const int64_t cells = (int64_t)(p.i1 - p.i0) * (p.j1 - p.j0);
+            hipLaunchKernelGGL(yee2d_pole_copy_kernel, dim3((unsigned)std::min<int64_t>(2048, (cells + 255) / 256)),
+                               dim3(256), 0, stream, p.state[1], p.state[0], cells);
         }
         YEE_HIP(hipGetLastError());
         hipLaunchKernelGGL(yee_clock_advance, dim3(1), dim3(64), 0, stream, ctx->d2.clock, (int64_t)count,
@@ -1047,7 +1089,7 @@ void choose_multi_batch(const yee2d_desc* descs, int32_t n, int32_t count, Batch
 {
     int64_t cells = 0;
     for (int32_t k = 0; k < n; ++k) {
-        if (!multi_ok(descs[k])) return;
+        if (!multi_ok(descs[k], false)) return;
         cells += (int64_t)descs[k].nx * descs[k].ny;
     }
     work->least = cells < kMultiBatchCells ? kMultiBatchShort : kMultiBatchLeast;
@@ -1175,6 +1217,7 @@ int32_t yee2d_create(const yee2d_desc* desc, yee_ctx** out)
     yee_ctx* ctx = new yee_ctx();
     ctx->kind = kSingle2D;
     ctx->d2 = d;
+    clear_pole_work(ctx->d2);
     set_geometry(ctx);
     *out = ctx;
     return YEE_OK;
@@ -1189,6 +1232,18 @@ int32_t yee2d_update(yee_ctx* ctx, const yee2d_desc* desc)
     if (status != YEE_OK) return status;
     drop_graph(ctx);
     ctx->d2 = d;
+    clear_pole_work(ctx->d2);
+    set_geometry(ctx);
+    return YEE_OK;
+}
+
+int32_t yee2d_set_pole_work(yee_ctx* ctx, float* work)
+{
+    if (!ctx || ctx->kind != kSingle2D) return fail(YEE_ESTATE, "not a single 2D context");
+    if (ctx->d2.n_poles != 1 || ctx->d2.pole[0].kind != YEE_DRUDE)
+        return fail(YEE_EINVAL, "a pole work array needs a single Drude pole");
+    if (ctx->d2.pole[0].state[1] != work) drop_graph(ctx);
+    ctx->d2.pole[0].state[1] = work;
     set_geometry(ctx);
     return YEE_OK;
 }

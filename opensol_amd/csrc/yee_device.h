@@ -42,6 +42,22 @@ __device__ __forceinline__ void dft_accumulate(const yee_flux_line& mon, int64_t
     }
 }
 
+// Accumulate sample `sample` of cell t (of `cells`) of a DFT region's spectrum c: v * phase to the FP64 Kahan records
+// (sum re, sum im, comp re, comp im) of every frequency.
+__device__ __forceinline__ void dft_region_add(const yee_dft_region& r, int c, int64_t cells, int64_t t, int64_t sample,
+                                               float v)
+{
+    const double* phase = r.phase + sample * r.n_freq * 2;
+    double4* acc = reinterpret_cast<double4*>(r.acc) + (int64_t)c * r.n_freq * cells + t;
+    const double x = (double)v;
+    for (int q = 0; q < r.n_freq; ++q) {
+        double4 a = acc[(int64_t)q * cells];
+        kahan_add(&a.x, &a.z, x * phase[2 * q]);
+        kahan_add(&a.y, &a.w, x * phase[2 * q + 1]);
+        acc[(int64_t)q * cells] = a;
+    }
+}
+
 // Source value injected after the E update of step n (0 past the table).
 __device__ __forceinline__ float wave_value(const yee_line_source& s, int64_t n)
 {

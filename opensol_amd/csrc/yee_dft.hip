@@ -17,20 +17,9 @@
 //   2D box monitor     physics/em/monitors.py:248-322 (DFTMonitor), :152-169 (dft_sample_slice, _centre_pairs)
 //   3D plane monitor   physics/em3d/monitors3d.py:165-238 (DFTPlane3D)
 //   phase              physics/em/monitors.py:22-34 (exp(-j omega t) m dt)
-#include "yee.h"
-#include <hip/hip_runtime.h>
+#include "yee_device.h"
 
 namespace {
-
-// FP64 Kahan-compensated accumulation of x into (sum, comp) held in registers: the true running sum is sum - comp
-// (Kahan 1965; hipcc compiles without fast-math, so the compensation survives).
-__device__ __forceinline__ void kahan(double& sum, double& comp, double x)
-{
-    const double y = x - comp;
-    const double t = sum + y;
-    comp = (t - sum) - y;
-    sum = t;
-}
 
 // Accumulate one sampled cell `t` of region `r`. field: the new state set's component pointers; n_axis: grid extent
 // per axis; axis_stride: element stride per axis.
@@ -46,7 +35,6 @@ __device__ __forceinline__ void dft_cell(const yee_dft_region& r, float* const* 
     const int64_t index[3] = {r.start[0] + t0 * r.stride[0], r.start[1] + t1 * r.stride[1],
                               r.start[2] + t2 * r.stride[2]};
     const int64_t cell = index[0] * axis_stride[0] + index[1] * axis_stride[1] + index[2] * axis_stride[2];
-    const double* phase = r.phase + sample * r.n_freq * 2;
     for (int c = 0; c < r.n_comp; ++c) {
         const float* f = field[r.comp[c]];
         float v = f[cell];
@@ -57,14 +45,7 @@ __device__ __forceinline__ void dft_cell(const yee_dft_region& r, float* const* 
                                                                  : cell);
             v = 0.5f * (v + f[lower]);
         }
-        double4* acc = reinterpret_cast<double4*>(r.acc) + (int64_t)c * r.n_freq * cells + t;
-        const double x = (double)v;
-        for (int q = 0; q < r.n_freq; ++q) {
-            double4 a = acc[(int64_t)q * cells];   // (sum re, sum im, comp re, comp im)
-            kahan(a.x, a.z, x * phase[2 * q]);
-            kahan(a.y, a.w, x * phase[2 * q + 1]);
-            acc[(int64_t)q * cells] = a;
-        }
+        yee::dft_region_add(r, c, cells, t, sample, v);
     }
 }
 

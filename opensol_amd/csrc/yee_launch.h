@@ -56,6 +56,8 @@ constexpr int kMultiWavesMax = 8;
 constexpr int kMultiIds = 1024;        // entries of the coefficient table in LDS, the zero entry included
 constexpr int kMultiRowsMax = 64;      // rows of a window
 constexpr int kMultiMax = 16;          // steps of a launch
+constexpr int kMultiCells = 8192;      // cells of the largest window
+constexpr int kMultiProbes = 64;       // probes of an instance: one a lane
 
 // Columns left of the owned ones: `steps`, rounded up so that a lane's columns start at a multiple of vec.
 constexpr int yee2d_multi_halo(int steps, int vec) { return (steps + vec - 1) / vec * vec; }
@@ -76,5 +78,7 @@ typedef struct yee2d_multi_plan {
     yee2d_multi_region region[5];
     int32_t n_regions, interior;
     int32_t blocks;
-    int32_t steps;
+    int32_t steps;   // rows and columns of halo: the steps of a launch, or one more (multi_pad)
+    int32_t take;    // steps of a launch (a batch passes each launch's own)
+    int32_t pad_;
 } yee2d_multi_plan;

@@ -587,6 +587,10 @@ class Engine2D:
                       for _ in range(1 if isinstance(pole, DrudePole) else 2)]
             self.poles.append(dict(pole=pole, component=component, box=box, coefficients=coefficients, drive=drive,
                                    states=states))
+        # launches of several steps pass a single Drude pole's current through a second array
+        self.pole_work = None
+        if model.polarization == 'ez' and len(self.poles) == 1 and isinstance(self.poles[0]['pole'], DrudePole):
+            self.pole_work = torch.empty_like(self.poles[0]['states'][0])
         components = COMPONENTS[model.polarization]
         self.probes = ProbeTable(model.probes, [p.cell[0] * pitch + p.cell[1] for p in model.probes],
                                  [components.index(p.field_component) for p in model.probes], dev)
@@ -735,6 +739,8 @@ class Engine2D:
         else:
             _lib.check(self.lib.yee2d_update(self._ctx, ctypes_byref(d)), 'yee2d_update')
         _lib.check(self.lib.yee2d_set_lossless(self._ctx, int(self.model.materials.lossless())), 'yee2d_set_lossless')
+        if self.pole_work is not None:
+            _lib.check(self.lib.yee2d_set_pole_work(self._ctx, self.pole_work.data_ptr()), 'yee2d_set_pole_work')
 
     def launch_geometry(self):
         """(rows_per_tile, lane_columns) the library resolved for this instance."""

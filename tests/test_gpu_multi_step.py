@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 DX, NPML = 25e-9, 8
 
 
-def build(pol, nx, ny, boundaries, media, graph_steps=0):
+def build(pol, nx, ny, boundaries, media, graph_steps=0, extras=None):
     from opensol_amd import Simulation
     px, py = boundaries in ('periodic_x', 'periodic'), boundaries in ('periodic_y', 'periodic')
     wx, wy = nx - (0 if px else 2 * NPML), ny - (0 if py else 2 * NPML)
@@ -32,6 +32,8 @@ def build(pol, nx, ny, boundaries, media, graph_steps=0):
         sim.add_electric_dipole(0.7 * wx * DX, 0.3 * wy * DX, wavelength=600e-9, orientation=30.0, waveform='ricker')
     sim.add_flux_monitor(axis='y', position=0.7 * wx * DX, span=(0.0, wy * DX), wavelengths=[500e-9, 700e-9])
     sim.add_flux_monitor(axis='x', position=0.2 * wy * DX, span=(0.2 * wx * DX, wx * DX), wavelengths=[600e-9])
+    if extras:
+        extras(sim, wx, wy)
     sim.finalize()
     torch = sim.engine.torch
     generator = torch.Generator().manual_seed(nx * 1000 + ny)
@@ -121,3 +123,44 @@ def test_multi_step_batch_members(gpu, graph_steps, large):
             for name in got:
                 assert bool((got[name] == expected[name]).all()), (k, name, call)
     batch.close()
+
+
+def add_extras(sim, pol, wx, wy, downsample):
+    """A Drude rectangle (E_z), DFT boxes with and without a stride, and probes near the window edges."""
+    from opensol_amd import DrudePole
+    if pol == 'ez':
+        sim.add_drude_rectangle(0.3 * wx * DX, 0.1 * wy * DX, 0.8 * wx * DX, 0.9 * wy * DX,
+                                DrudePole(omega_p=1.5e15, gamma=1e14, eps_inf=4.0))
+    sim.add_dft_monitor(0.5 * DX, 0.5 * DX, (wx - 0.5) * DX, (wy - 0.5) * DX, wavelengths=[550e-9, 700e-9],
+                        downsample=downsample)
+    sim.add_dft_monitor(0.2 * wx * DX, 0.3 * wy * DX, 0.7 * wx * DX, 0.8 * wy * DX, wavelengths=[600e-9])
+    rng = np.random.default_rng([wx, wy])
+    components = ('ez', 'hx', 'hy') if pol == 'ez' else ('hz', 'ex', 'ey')
+    spots = [(0, 0), (wx - 1, wy - 1)] + [(rng.integers(wx), rng.integers(wy)) for _ in range(9)]
+    for k, (i, j) in enumerate(spots):
+        sim.add_field_probe((i + 0.5) * DX, (j + 0.5) * DX, field_component=components[k % 3])
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+@pytest.mark.parametrize('nx,ny', [(34, 64), (61, 37), (129, 130), (300, 257), (611, 523)])
+@pytest.mark.parametrize('boundaries,media', [('pml', 'plain'), ('periodic_y', 'lossy'), ('periodic_x', 'plain'),
+                                              ('periodic', 'pec')])
+@pytest.mark.parametrize('graph_steps', [0, 9])
+def test_multi_step_with_pole_regions_and_probes(gpu, pol, nx, ny, boundaries, media, graph_steps):
+    def make(graph):
+        return build(pol, nx, ny, boundaries, media, graph,
+                     extras=lambda sim, wx, wy: add_extras(sim, pol, wx, wy, 3 if nx % 2 else 1))
+    multi, single = make(graph_steps), make(0)
+    total = 0
+    for steps in (1, 2, 7, 20, 33):
+        multi.engine.step(steps)
+        single.engine.step_timed(steps)
+        total += steps
+        a, b = arrays(multi, total), arrays(single, total)
+        for sim, out in ((multi, a), (single, b)):
+            out.update({f'dft {k}': acc for k, acc in enumerate(sim.engine.dft_accumulators)})
+            out.update({f'current {k}': entry['states'][0] for k, entry in enumerate(sim.engine.poles)})
+            out['probes'] = sim.engine.probes.samples[:total]
+        for name in a:
+            assert bool((a[name] == b[name]).all()), (name, total, int((a[name] != b[name]).sum()))
+    assert all(bool((acc != 0).any()) for acc in multi.engine.dft_accumulators)
