@@ -10,6 +10,7 @@
 //
 // Fields and the H psi are double-buffered (step n reads set n & 1): the H launch writes H of the other set, the E launch
 // reads that and writes E of it; the E psi is read and written by the one thread that owns its cell.
+#include "yee3d_after.h"
 #include "yee3d_cells.h"
 
 namespace yee3 {
@@ -304,16 +305,25 @@ __device__ __forceinline__ void e_block(const yee3d_desc& d, int64_t n, int bloc
 
 }  // namespace yee3
 
-// One 3D instance; the descriptor is read in place at the kernel-argument pointer.
-__global__ void __launch_bounds__(256) yee3d_h_kernel(yee3d_desc desc, int32_t offset)
+// One 3D instance; the descriptor is read in place at the kernel-argument pointer. AFTER: the blocks past a.first take the
+// samples of the step before, from the set that this launch only reads. As launches of their own after every step they cost
+// what a small grid's update does: 97 x 88 x 75 with a flux plane, a DFT plane and probes took 28.5 us a step, five launches.
+template <bool AFTER>
+__global__ void __launch_bounds__(256) yee3d_h_kernel(yee3d_desc desc, yee3d_after a, int32_t offset)
 {
     typedef const __attribute__((address_space(4))) yee3d_desc ConstDesc;
     const yee3d_desc& d = *(const yee3d_desc*)(ConstDesc*)__builtin_amdgcn_kernarg_segment_ptr();
     if (d.clock != desc.clock) return;
     const int64_t n = *d.clock + offset;
+    if (AFTER && (int)blockIdx.x >= a.first) {
+        yee3::after_block(d, a, n - 1, (int)blockIdx.x - a.first);
+        return;
+    }
     if (n >= d.step_limit) return;
     yee3::h_block(d, n, blockIdx.x);
 }
+template __global__ void yee3d_h_kernel<false>(yee3d_desc, yee3d_after, int32_t);
+template __global__ void yee3d_h_kernel<true>(yee3d_desc, yee3d_after, int32_t);
 
 template <bool POLES>
 __global__ void __launch_bounds__(256) yee3d_e_kernel(yee3d_desc desc, int32_t offset)

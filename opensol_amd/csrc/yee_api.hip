@@ -27,7 +27,8 @@ template <int VEC, int R, int TV, int TR, int NW>
 __global__ void yee2d_multi_batch_kernel(const yee2d_desc* __restrict__ descs, const yee2d_multi_plan* __restrict__ plans,
                                          const int32_t* __restrict__ prefix, int32_t n_inst, int32_t offset,
                                          int32_t launch, int32_t steps, int32_t previous);
-__global__ void yee3d_h_kernel(yee3d_desc desc, int32_t offset);
+template <bool AFTER>
+__global__ void yee3d_h_kernel(yee3d_desc desc, yee3d_after a, int32_t offset);
 template <bool POLES>
 __global__ void yee3d_e_kernel(yee3d_desc desc, int32_t offset);
 template <bool E>
@@ -37,17 +38,15 @@ template <bool POLES>
 __global__ void yee3d_step_kernel(yee3d_desc desc, int32_t blocks, int32_t offset);
 __global__ void yee3d_batch_kernel(const yee3d_desc* __restrict__ descs, const int32_t* __restrict__ prefix,
                                    int32_t n_inst, int32_t offset);
-__global__ void yee3d_sample_kernel(yee3d_desc d, int64_t cells_total, int32_t offset);
+__global__ void yee3d_after_kernel(yee3d_desc d, yee3d_after a, int32_t offset);
 __global__ void yee3d_batch_sample_kernel(const yee3d_desc* __restrict__ descs, const int64_t* __restrict__ prefix,
                                           int32_t n_inst, int32_t offset);
 __global__ void yee_clock_advance_batch3d(const yee3d_desc* __restrict__ descs, int32_t n_inst, int64_t k);
 __global__ void yee_clock_advance(int64_t* clock, int64_t k, int64_t limit);
 __global__ void yee2d_probe_kernel(yee2d_desc d, int32_t offset);
 __global__ void yee2d_wall_kernel(yee2d_desc d, int32_t offset);
-__global__ void yee3d_probe_kernel(yee3d_desc d, int32_t offset);
 __global__ void yee3d_mirror_kernel(yee3d_desc d, int32_t face, int32_t offset);
 __global__ void yee2d_dft_kernel(yee2d_desc d, int32_t offset);
-__global__ void yee3d_dft_kernel(yee3d_desc d, int32_t offset);
 __global__ void yee_clock_advance_batch(const yee2d_desc* __restrict__ descs, int32_t n_inst, int64_t k);
 __global__ void yee2d_batch_probe_kernel(const yee2d_desc* __restrict__ descs, int32_t offset);
 __global__ void yee2d_batch_wall_kernel(const yee2d_desc* __restrict__ descs, int32_t offset);
@@ -693,8 +692,26 @@ void set_geometry_3d(yee_ctx* ctx)
     ctx->sample_cells = sample_cells_3d(d);
 }
 
-// The launches of step *clock + offset of a single 3D instance up to its mirror planes.
-void launch_step_3d(const yee_ctx* ctx, int32_t offset, hipStream_t stream)
+// The blocks that take an instance's samples after a step.
+yee3d_after after_blocks_3d(const yee_ctx* ctx)
+{
+    const yee3d_desc& d = ctx->d3;
+    yee3d_after a{};
+    a.sample_cells = ctx->sample_cells;
+    a.sample_blocks = (int32_t)((ctx->sample_cells + 255) / 256);
+    a.dft_blocks = d.n_dft > 0 ? dft_blocks(d.dft, d.n_dft) : 0;
+    a.probe_blocks = d.probes.n_probes > 0 ? 1 : 0;
+    a.first = ctx->blocks;
+    return a;
+}
+int32_t count_after(const yee_ctx* ctx, const yee3d_after& a)
+{
+    return a.sample_blocks + a.dft_blocks * ctx->d3.n_dft + a.probe_blocks;
+}
+
+// The launches of step *clock + offset of a single 3D instance up to its mirror planes. `after`: the samples of the step
+// before join the H launch of the two-launch form (none: null).
+void launch_step_3d(const yee_ctx* ctx, const yee3d_after* after, int32_t offset, hipStream_t stream)
 {
     const yee3d_desc& d = ctx->d3;
     if (ctx->fused) {
@@ -702,7 +719,11 @@ void launch_step_3d(const yee_ctx* ctx, int32_t offset, hipStream_t stream)
                            dim3(kThreads3D), 0, stream, d, (int32_t)ctx->tiles, offset);
         return;
     }
-    hipLaunchKernelGGL(yee3d_h_kernel, dim3(ctx->blocks), dim3(256), 0, stream, d, offset);
+    if (after)
+        hipLaunchKernelGGL(yee3d_h_kernel<true>, dim3(ctx->blocks + count_after(ctx, *after)), dim3(256), 0, stream, d,
+                           *after, offset);
+    else
+        hipLaunchKernelGGL(yee3d_h_kernel<false>, dim3(ctx->blocks), dim3(256), 0, stream, d, yee3d_after{}, offset);
     hipLaunchKernelGGL(d.n_poles > 0 ? yee3d_e_kernel<true> : yee3d_e_kernel<false>, dim3(ctx->blocks), dim3(256), 0, stream,
                        d, offset);
 }
@@ -980,18 +1001,13 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
         return YEE_OK;
     }
     if (ctx->kind == kSingle3D) {
-        const int sample_blocks = (int)((ctx->sample_cells + 255) / 256);
+        const yee3d_after after = after_blocks_3d(ctx);
+        const int32_t after_blocks = count_after(ctx, after);
         for (int32_t k = 0; k < count; ++k) {
-            launch_step_3d(ctx, k, stream);
+            launch_step_3d(ctx, k > 0 && after_blocks > 0 ? &after : nullptr, k, stream);
             launch_mirrors_3d(ctx->d3, k, stream);
-            if (sample_blocks > 0)
-                hipLaunchKernelGGL(yee3d_sample_kernel, dim3(sample_blocks), dim3(256), 0, stream, ctx->d3,
-                                   ctx->sample_cells, k);
-            if (ctx->d3.n_dft > 0)
-                hipLaunchKernelGGL(yee3d_dft_kernel, dim3(dft_blocks(ctx->d3.dft, ctx->d3.n_dft), ctx->d3.n_dft),
-                                   dim3(256), 0, stream, ctx->d3, k);
-            if (ctx->d3.probes.n_probes > 0)
-                hipLaunchKernelGGL(yee3d_probe_kernel, dim3(1), dim3(256), 0, stream, ctx->d3, k);
+            if (after_blocks > 0 && (ctx->fused || k == count - 1))
+                hipLaunchKernelGGL(yee3d_after_kernel, dim3(after_blocks), dim3(256), 0, stream, ctx->d3, after, k);
         }
         YEE_HIP(hipGetLastError());
         hipLaunchKernelGGL(yee_clock_advance, dim3(1), dim3(64), 0, stream, ctx->d3.clock, (int64_t)count,
@@ -1382,21 +1398,22 @@ int32_t step_timed_3d(yee_ctx* ctx, int64_t n_steps, hipStream_t s, double* kern
     cells[0] = (int64_t)d.nx * d.ny * d.nz;
     cells[1] = ctx->sample_cells;
     kernel_ms[0] = kernel_ms[1] = 0.0;
-    const int sample_blocks = (int)((ctx->sample_cells + 255) / 256);
+    yee3d_after samples = after_blocks_3d(ctx), rest = samples;
+    samples.dft_blocks = samples.probe_blocks = 0;
+    rest.sample_blocks = 0;
+    const int32_t rest_blocks = count_after(ctx, rest);
     hipEvent_t ev[3];
     for (auto& e : ev) YEE_HIP(hipEventCreate(&e));
     int32_t status = YEE_OK;
     for (int64_t k = 0; k < n_steps && status == YEE_OK; ++k) {
         (void)hipEventRecord(ev[0], s);
-        launch_step_3d(ctx, 0, s);
+        launch_step_3d(ctx, nullptr, 0, s);
         (void)hipEventRecord(ev[1], s);
         launch_mirrors_3d(d, 0, s);
-        if (sample_blocks > 0)
-            hipLaunchKernelGGL(yee3d_sample_kernel, dim3(sample_blocks), dim3(256), 0, s, d, ctx->sample_cells, 0);
+        if (samples.sample_blocks > 0)
+            hipLaunchKernelGGL(yee3d_after_kernel, dim3(samples.sample_blocks), dim3(256), 0, s, d, samples, 0);
         (void)hipEventRecord(ev[2], s);
-        if (d.n_dft > 0)
-            hipLaunchKernelGGL(yee3d_dft_kernel, dim3(dft_blocks(d.dft, d.n_dft), d.n_dft), dim3(256), 0, s, d, 0);
-        if (d.probes.n_probes > 0) hipLaunchKernelGGL(yee3d_probe_kernel, dim3(1), dim3(256), 0, s, d, 0);
+        if (rest_blocks > 0) hipLaunchKernelGGL(yee3d_after_kernel, dim3(rest_blocks), dim3(256), 0, s, d, rest, 0);
         hipLaunchKernelGGL(yee_clock_advance, dim3(1), dim3(64), 0, s, d.clock, (int64_t)1, d.step_limit);
         hipError_t e = hipEventSynchronize(ev[2]);
         float a = 0.f, b = 0.f;

@@ -82,3 +82,10 @@ typedef struct yee2d_multi_plan {
     int32_t take;    // steps of a launch (a batch passes each launch's own)
     int32_t pad_;
 } yee2d_multi_plan;
+
+// Blocks of 256 threads that take the samples of a 3D instance after a step (yee3d_after.h): one a run of plane cells, `dft_blocks` a DFT region, one for the probes.
+typedef struct yee3d_after {
+    int64_t sample_cells;
+    int32_t sample_blocks, dft_blocks, probe_blocks;
+    int32_t first;   // first of these blocks in an H launch, behind those of the update
+} yee3d_after;
