@@ -480,7 +480,7 @@ struct MultiWindow {
     // The drive of a cell (read and written by its own lane only).
     static __device__ __forceinline__ float& drive(int r, int k)
     {
-        return lds_drive[(r * VEC + k) * 64 * NW + threadIdx.x];
+        return lds_drive[(r * 64 * NW + threadIdx.x) * VEC + k];
     }
 
     // Current and drive of the cells inside the pole's box; launch `launch` of a call reads state[launch & 1].
@@ -499,7 +499,7 @@ struct MultiWindow {
         for (int r = 0; r < R; ++r) {
             const int f = fold_row(q0 + r);
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) jp[r][k] = 0.f;
+            for (int k = 0; k < VEC; ++k) jp[r][k] = drive(r, k) = 0.f;
             if (f < p.i0 || f >= p.i1) continue;
             pole_rows |= 1u << r;
             const int64_t base = (int64_t)(f - p.i0) * (p.j1 - p.j0) - p.j0;
@@ -581,13 +581,12 @@ struct MultiWindow {
                 v -= m.y * ye[r][k];
             }
             if constexpr (POLE) {
-                const bool inside = (pole_rows >> r) & 1 && (pole_cols >> k) & 1;   // selects: what lies outside keeps
-                float jc = jp[r][k];                                                // its infinities and NaN
-                jc += damping * jc + drive(r, k) * c[r][k];
-                float u = v;
-                u -= m.y * jc;
-                jp[r][k] = inside ? jc : jp[r][k];
-                v = inside ? u : v;
+                // cells outside the box have no current and no drive: their E passes unread (it may be infinite)
+                const float e_n = (pole_rows >> r) & 1 && (pole_cols >> k) & 1 ? c[r][k] : 0.f;
+                float jc = jp[r][k];
+                jc += damping * jc + drive(r, k) * e_n;
+                jp[r][k] = jc;
+                v -= m.y * jc;
             }
             c[r][k] = v;
         }
