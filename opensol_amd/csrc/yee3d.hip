@@ -561,22 +561,12 @@ __global__ void __launch_bounds__(256) yee3d_after_kernel(yee3d_desc desc, yee3d
     yee3::after_block(d, a, *d.clock + offset, blockIdx.x);
 }
 
-// Samples of many instances in one launch: thread t belongs to the instance whose plane-cell range
-// [prefix[k], prefix[k+1]) holds it.
+// Samples of many instances after their step *clock + offset, in one launch (sample_members).
 __global__ void __launch_bounds__(256) yee3d_batch_sample_kernel(const yee3d_desc* __restrict__ descs,
                                                                 const int64_t* __restrict__ prefix, int32_t n_inst,
                                                                 int32_t offset)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= prefix[n_inst]) return;
-    int lo = 0, hi = n_inst;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (prefix[mid] <= t) lo = mid; else hi = mid;
-    }
-    typedef const __attribute__((address_space(4))) yee3d_desc ConstDesc;
-    const yee3d_desc& d = *(const yee3d_desc*)((ConstDesc*)descs + lo);
-    yee3::sample_cell(d, *d.clock + offset, t - prefix[lo]);
+    yee3::sample_members(descs, prefix, n_inst, offset, blockIdx.x);
 }
 
 namespace yee3 {

@@ -69,6 +69,23 @@ __device__ __forceinline__ void probes_3d(const yee3d_desc& d, int64_t n)
     }
 }
 
+// Flux-plane samples of many instances after their step *clock + offset: thread t of the blocks belongs to the instance
+// whose plane-cell range [prefix[k], prefix[k+1]) holds it.
+__device__ __forceinline__ void sample_members(const yee3d_desc* __restrict__ descs, const int64_t* __restrict__ prefix,
+                                               int32_t n_inst, int32_t offset, int block)
+{
+    const int64_t t = (int64_t)block * 256 + threadIdx.x;
+    if (t >= prefix[n_inst]) return;
+    int lo = 0, hi = n_inst;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (prefix[mid] <= t) lo = mid; else hi = mid;
+    }
+    typedef const __attribute__((address_space(4))) yee3d_desc ConstDesc;
+    const yee3d_desc& d = *(const yee3d_desc*)((ConstDesc*)descs + lo);
+    sample_cell(d, *d.clock + offset, t - prefix[lo]);
+}
+
 // Block `block` of those of `a`, after step n.
 __device__ __forceinline__ void after_block(const yee3d_desc& d, const yee3d_after& a, int64_t n, int block)
 {

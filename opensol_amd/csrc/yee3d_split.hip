@@ -307,7 +307,8 @@ __device__ __forceinline__ void e_block(const yee3d_desc& d, int64_t n, int bloc
 
 // One 3D instance; the descriptor is read in place at the kernel-argument pointer. AFTER: the blocks past a.first take the
 // samples of the step before, from the set that this launch only reads. As launches of their own after every step they cost
-// what a small grid's update does: 97 x 88 x 75 with a flux plane, a DFT plane and probes took 28.5 us a step, five launches.
+// what a small grid's update does: 97 x 88 x 75 with a flux plane, a DFT plane and probes took 28.5 us a step with
+// five launches, 21 with these two.
 template <bool AFTER>
 __global__ void __launch_bounds__(256) yee3d_h_kernel(yee3d_desc desc, yee3d_after a, int32_t offset)
 {
@@ -339,12 +340,20 @@ template __global__ void yee3d_e_kernel<false>(yee3d_desc, int32_t);
 template __global__ void yee3d_e_kernel<true>(yee3d_desc, int32_t);
 
 // The H or the E update of many instances: block b belongs to the member whose range [prefix[k], prefix[k + 1]) holds it.
+// Blocks of an H launch past prefix[n_inst], rounded up to `first`, take the members' plane samples of the step before, as
+// those of a single instance do (six members of 64 to 140 cells a side: 95 us a step, 101 with a
+// launch of their own).
 template <bool E>
 __global__ void __launch_bounds__(256) yee3d_batch_half_kernel(const yee3d_desc* __restrict__ descs,
-                                                              const int32_t* __restrict__ prefix, int32_t n_inst,
-                                                              int32_t offset)
+                                                              const int32_t* __restrict__ prefix,
+                                                              const int64_t* __restrict__ sample_prefix, int32_t n_inst,
+                                                              int32_t first, int32_t offset)
 {
     const int block = blockIdx.x;
+    if (!E && block >= first) {
+        yee3::sample_members(descs, sample_prefix, n_inst, offset - 1, block - first);
+        return;
+    }
     int lo = 0, hi = n_inst;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -359,7 +368,7 @@ __global__ void __launch_bounds__(256) yee3d_batch_half_kernel(const yee3d_desc*
     else if (d.n_poles > 0) yee3::e_block<true>(d, n, own);
     else yee3::e_block<false>(d, n, own);
 }
-template __global__ void yee3d_batch_half_kernel<false>(const yee3d_desc* __restrict__, const int32_t* __restrict__, int32_t,
-                                                        int32_t);
-template __global__ void yee3d_batch_half_kernel<true>(const yee3d_desc* __restrict__, const int32_t* __restrict__, int32_t,
-                                                       int32_t);
+template __global__ void yee3d_batch_half_kernel<false>(const yee3d_desc* __restrict__, const int32_t* __restrict__,
+                                                        const int64_t* __restrict__, int32_t, int32_t, int32_t);
+template __global__ void yee3d_batch_half_kernel<true>(const yee3d_desc* __restrict__, const int32_t* __restrict__,
+                                                       const int64_t* __restrict__, int32_t, int32_t, int32_t);

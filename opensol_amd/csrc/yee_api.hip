@@ -33,7 +33,8 @@ template <bool POLES>
 __global__ void yee3d_e_kernel(yee3d_desc desc, int32_t offset);
 template <bool E>
 __global__ void yee3d_batch_half_kernel(const yee3d_desc* __restrict__ descs, const int32_t* __restrict__ prefix,
-                                        int32_t n_inst, int32_t offset);
+                                        const int64_t* __restrict__ sample_prefix, int32_t n_inst, int32_t first,
+                                        int32_t offset);
 template <bool POLES>
 __global__ void yee3d_step_kernel(yee3d_desc desc, int32_t blocks, int32_t offset);
 __global__ void yee3d_batch_kernel(const yee3d_desc* __restrict__ descs, const int32_t* __restrict__ prefix,
@@ -1023,10 +1024,13 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
                 hipLaunchKernelGGL(yee3d_batch_kernel, dim3(ctx->blocks), dim3(kThreads3D), 0, stream, ctx->descs3_dev,
                                    ctx->block_prefix_dev, ctx->n_inst, k);
             } else {
-                hipLaunchKernelGGL(yee3d_batch_half_kernel<false>, dim3(ctx->blocks), dim3(256), 0, stream,
-                                   ctx->descs3_dev, ctx->block_prefix_dev, ctx->n_inst, k);
+                // from the second step on the H launch takes the samples of the step before
+                hipLaunchKernelGGL(yee3d_batch_half_kernel<false>, dim3(ctx->blocks + (k > 0 ? sample_blocks : 0)),
+                                   dim3(256), 0, stream, ctx->descs3_dev, ctx->block_prefix_dev, ctx->sample_prefix_dev,
+                                   ctx->n_inst, ctx->blocks, k);
                 hipLaunchKernelGGL(yee3d_batch_half_kernel<true>, dim3(ctx->blocks), dim3(256), 0, stream,
-                                   ctx->descs3_dev, ctx->block_prefix_dev, ctx->n_inst, k);
+                                   ctx->descs3_dev, ctx->block_prefix_dev, ctx->sample_prefix_dev, ctx->n_inst,
+                                   ctx->blocks, k);
             }
             // mirror faces as a single instance orders them: every symmetric face, then the antisymmetric ones
             for (int kind = 0; kind < 2; ++kind)
@@ -1035,7 +1039,7 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
                         hipLaunchKernelGGL(yee3d_batch_mirror_kernel, dim3(a.mirror_blocks[kind][face], ctx->n_inst),
                                            dim3(256), 0, stream, ctx->descs3_dev, face,
                                            kind == 0 ? YEE_MIRROR_SYMMETRIC : YEE_MIRROR_ANTISYMMETRIC, k);
-            if (sample_blocks > 0)
+            if (sample_blocks > 0 && (ctx->fused || k == count - 1))
                 hipLaunchKernelGGL(yee3d_batch_sample_kernel, dim3(sample_blocks), dim3(256), 0, stream,
                                    ctx->descs3_dev, ctx->sample_prefix_dev, ctx->n_inst, k);
             if (a.dft_blocks > 0)
