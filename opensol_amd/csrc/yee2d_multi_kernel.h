@@ -18,7 +18,8 @@ __global__ void __launch_bounds__(64 * NW, 4) yee2d_multi_kernel(yee2d_desc desc
     const int block = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (block >= plan.blocks) return;
     const int64_t clock = *d.clock;
-    yee::multi_block<POL, VEC, R, TV, TR, NW, EXTRA>(d, plan, block, clock, offset, launch, plan.take);
+    yee::multi_block<POL, VEC, R, TV, TR, NW, EXTRA>(d, plan, block, clock, offset, launch,
+                                                       EXTRA ? plan.take : plan.steps);   // equal without EXTRA
 }
 
 #define YEE_MULTI_KERNEL(POL, VEC, R, TV, TR, NW, EXTRA)                                                                 \
