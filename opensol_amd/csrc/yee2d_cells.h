@@ -1,4 +1,4 @@
-// Vector access and the single-cell updates shared by the 2D kernels (yee2d.hip one step per launch, yee2d_march.hip
+// Vector access and the single-cell updates shared by the 2D kernels (yee2d.hip one step per launch, yee2d_multi.h
 // several). Every copy of a cell, in either file, goes through these helpers and the library is built with
 // -ffp-contract=on, so a recomputed value equals its owner's bit for bit.
 #pragma once

@@ -618,6 +618,17 @@ void clear_pole_work(yee2d_desc& d)
         if (d.pole[p].kind == YEE_DRUDE) d.pole[p].state[1] = nullptr;
 }
 
+// Calls of one or two steps (two: a launch each, for the parity of the state) step large grids with the one-step kernels:
+// a window of one step loads its halo and its tables for little. Measured, us for one step, one-step kernels / windows:
+// E_z 2400^2 61 / 45, 4000^2 113 / 102, 5500^2 177 / 225, 8000^2 384 / 442 (H_z 425 / 471); with a pole and a DFT region
+// E_z 2400^2 71 / 72, 4000^2 143 / 151, 8000^2 446 / 599, H_z 78 / 90, 153 / 210, 517 / 798. Three steps: windows everywhere
+// (8000^2 439, with the extra features 742 and 1066).
+bool one_step_launches(const yee2d_desc& d, int32_t count, int32_t launches)
+{
+    const int64_t least = multi_extra(d) ? (int64_t)1 << 22 : (int64_t)1 << 24;
+    return launches == count && (int64_t)d.nx * d.ny >= least;
+}
+
 void set_geometry(yee_ctx* ctx)
 {
     ctx->multi = multi_ok(ctx->d2, true) && ctx->d2.step_limit == INT64_MAX;
@@ -940,10 +951,10 @@ int32_t ensure_side(yee_ctx* ctx)
 int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
 {
     if (count <= 0) return YEE_OK;
-    if (ctx->kind == kSingle2D && ctx->multi) {
-        const MultiShape* shape = nullptr;
-        int32_t launches = 0;
-        choose_multi(ctx, count, &shape, &launches);
+    const MultiShape* shape = nullptr;
+    int32_t launches = 0;
+    if (ctx->kind == kSingle2D && ctx->multi) choose_multi(ctx, count, &shape, &launches);
+    if (shape && !one_step_launches(ctx->d2, count, launches)) {
         for (int32_t k = 0, offset = 0; k < launches; ++k) {
             const yee2d_multi_plan plan = multi_plan(ctx->d2, multi_steps(count, launches, k), *shape, tall_windows(ctx));
             const int blocks = (plan.blocks + 7) / 8 * 8;   // a multiple of the XCDs

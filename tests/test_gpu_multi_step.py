@@ -164,3 +164,21 @@ def test_multi_step_with_pole_regions_and_probes(gpu, pol, nx, ny, boundaries, m
         for name in a:
             assert bool((a[name] == b[name]).all()), (name, total, int((a[name] != b[name]).sum()))
     assert all(bool((acc != 0).any()) for acc in multi.engine.dft_accumulators)
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+def test_calls_of_one_and_two_steps_of_a_large_grid(gpu, pol):
+    """One- and two-step calls of a large grid take other kernels than longer ones: the state passes between them."""
+    multi, single = (build(pol, 2051, 2046, 'pml', 'plain',
+                           extras=lambda sim, wx, wy: add_extras(sim, pol, wx, wy, 4)) for _ in range(2))
+    total = 0
+    for steps in (1, 3, 2, 7, 1):
+        multi.engine.step(steps)
+        single.engine.step_timed(steps)
+        total += steps
+        a, b = arrays(multi, total), arrays(single, total)
+        for sim, out in ((multi, a), (single, b)):
+            out.update({f'current {k}': entry['states'][0] for k, entry in enumerate(sim.engine.poles)})
+            out['probes'] = sim.engine.probes.samples[:total]
+        for name in a:
+            assert bool((a[name] == b[name]).all()), (name, total)
