@@ -36,7 +36,7 @@
 namespace yee {
 
 __shared__ float4 lds_coef[kMultiIds];
-__shared__ float4 lds_row[2 * kMultiRowsMax];             // x constants of a window row: (inv_h, inv_e, b_h, g_h), (b_e, g_e)
+__shared__ float4 lds_row[2 * kMultiRowsMax];             // x constants of a window row: (inv, b, g, psi bits) of h and of e
 __shared__ float lds_wave[YEE_MAX_SOURCES * kMultiMax];   // source values of the launch's steps
 __shared__ float lds_profile[YEE_MAX_SOURCES * 128];      // source profiles along the window (0 past their span)
 __shared__ float lds_up[kMultiWavesMax * 128];            // the row each wavefront hands down (its lowest)
@@ -138,6 +138,14 @@ __device__ __forceinline__ void store_n(float* __restrict__ p, const float v[VEC
     else stv<VEC>(p, v);
 }
 
+// `v` where `bits` are set, 0 where none are: what a recursion takes where there is no psi. Its factors are 0 there as well,
+// but 0 times an infinite difference is NaN, and an overflowed field stays what the one-step kernels make of it. An AND with
+// bits in a vector register: 300 steps of 1031 x 773 E_z take 0.85 ms so, 0.81 without it, 0.98 with selects on lane masks or
+// scalar branches around the recursions, which the general windows have no scalar registers left for (8192^2 E_z, 40 steps:
+// 2.48, 2.37 and 2.65 ms).
+__device__ __forceinline__ float keep_bits(uint32_t bits, float v) { return __uint_as_float(bits & __float_as_uint(v)); }
+__device__ __forceinline__ float keep_bits(float bits, float v) { return keep_bits(__float_as_uint(bits), v); }
+
 // Columns of a lane and their y constants; the lean form knows that all of them are inside the grid's bulk.
 template <int VEC, bool EDGE>
 struct LaneColumns {
@@ -149,6 +157,7 @@ struct LaneColumns {
     bool split;              // the columns of a lane are not adjacent after folding
     int ry_h[VEC], ry_e[VEC];
     float inv_e[VEC], inv_h[VEC], b_h[VEC], g_h[VEC], b_e[VEC], g_e[VEC];
+    uint32_t psi_h[VEC], psi_e[VEC], moves[VEC];   // all bits set, or none: has a psi row; not `stays` (keep_bits)
 
     // positions, and the loads that need nothing loaded before
     __device__ __forceinline__ void begin(const yee2d_desc& d, const Window& w)
@@ -190,7 +199,8 @@ struct LaneColumns {
             const yee_cpml_axis& cy = d.cpml[1];
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
-                if (!in[k]) ry_h[k] = ry_e[k] = -1;
+                if (!in[k]) ry_e[k] = -1;
+                if (stays[k]) ry_h[k] = -1;
                 b_h[k] = g_h[k] = b_e[k] = g_e[k] = 0.f;
                 if (cy.n_rows > 0) {
                     const int h = max(ry_h[k], 0), e = max(ry_e[k], 0);
@@ -213,6 +223,11 @@ struct LaneColumns {
                 g_h[k] = ry_h[k] >= 0 ? g_h[k] : 0.f;
                 b_e[k] = ry_e[k] >= 0 ? b_e[k] : 0.f;
                 g_e[k] = ry_e[k] >= 0 ? g_e[k] : 0.f;
+                psi_h[k] = ry_h[k] >= 0 ? ~0u : 0u;
+                psi_e[k] = ry_e[k] >= 0 ? ~0u : 0u;
+                moves[k] = stays[k] ? 0u : ~0u;
+                // not lane masks in scalar registers, which are full
+                asm volatile("" : "+v"(psi_h[k]), "+v"(psi_e[k]), "+v"(moves[k]));
             }
         }
     }
@@ -547,11 +562,15 @@ struct MultiWindow {
             const float de_y = right(c[r], k, next) - c[r][k];
             float unused;
             if constexpr (EDGE) {
-                float v;
-                if constexpr (XL) v = ez_hy(m, fy[r][k], de_x, x.x, true, x.z, x.w, xh[r][k], &xh[r][k]);
-                else v = ez_hy(m, fy[r][k], de_x, idx, false, 0.f, 0.f, 0.f, &unused);
+                float v = ez_hy(m, fy[r][k], de_x, XL ? x.x : idx, false, 0.f, 0.f, 0.f, &unused);
+                if constexpr (XL) {
+                    xh[r][k] = x.y * xh[r][k] + x.z * keep_bits(x.w, de_x);
+                    v += m.w * xh[r][k];
+                }
                 fy[r][k] = (stays >> r) & 1 ? fy[r][k] : v;
-                const float u = ez_hx(m, fx[r][k], de_y, col.inv_h[k], true, col.b_h[k], col.g_h[k], yh[r][k], &yh[r][k]);
+                float u = ez_hx(m, fx[r][k], de_y, col.inv_h[k], false, 0.f, 0.f, 0.f, &unused);
+                yh[r][k] = col.b_h[k] * yh[r][k] + col.g_h[k] * keep_bits(col.psi_h[k], de_y);
+                u -= m.w * yh[r][k];
                 fx[r][k] = col.stays[k] ? fx[r][k] : u;
             } else {
                 fy[r][k] = ez_hy(m, fy[r][k], de_x, idx, false, 0.f, 0.f, 0.f, &unused);
@@ -563,8 +582,8 @@ struct MultiWindow {
     // E_z: E of row r from H_y of the row below it
     __device__ __forceinline__ void ez_e_row(int r, const float below[VEC])
     {
-        const float ie = XL ? lds_row[2 * (wave * R + r)].y : idx;
         const float4 x = XL ? lds_row[2 * (wave * R + r) + 1] : float4{};
+        const float ie = XL ? x.x : idx;
         const float prev = lane_prev(fx[r][VEC - 1]);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
@@ -573,11 +592,11 @@ struct MultiWindow {
             const float dhx = fx[r][k] - left(fx[r], k, prev);
             float v = ez_centre(m, c[r][k], dhy, dhx, ie, EDGE ? col.inv_e[k] : idy);
             if constexpr (XL) {
-                xe[r][k] = x.x * xe[r][k] + x.y * dhy;
+                xe[r][k] = x.y * xe[r][k] + x.z * keep_bits(x.w, dhy);
                 v += m.y * xe[r][k];
             }
             if constexpr (EDGE) {
-                ye[r][k] = col.b_e[k] * ye[r][k] + col.g_e[k] * dhx;
+                ye[r][k] = col.b_e[k] * ye[r][k] + col.g_e[k] * keep_bits(col.psi_e[k], dhx);
                 v -= m.y * ye[r][k];
             }
             if constexpr (POLE) {
@@ -595,8 +614,8 @@ struct MultiWindow {
     // H_z: H of row r from E_y of the row below it
     __device__ __forceinline__ void hz_h_row(int r, const float below[VEC])
     {
-        const float ie = XL ? lds_row[2 * (wave * R + r)].y : idx;
         const float4 x = XL ? lds_row[2 * (wave * R + r) + 1] : float4{};
+        const float ie = XL ? x.x : idx;
         const float prev = lane_prev(fx[r][VEC - 1]);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
@@ -605,15 +624,16 @@ struct MultiWindow {
             const float dex = fx[r][k] - left(fx[r], k, prev);
             const float dey = fy[r][k] - below[k];
             float no_x, no_y;
-            if constexpr (XL)
-                c[r][k] = hz_centre(m, c[r][k], dex, dey, col.inv_e[k], ie, true, x.x, x.y, xe[r][k],
-                                    &xe[r][k], true, col.b_e[k], col.g_e[k], ye[r][k], &ye[r][k]);
-            else if constexpr (EDGE)
-                c[r][k] = hz_centre(m, c[r][k], dex, dey, col.inv_e[k], ie, false, 0.f, 0.f, 0.f, &no_x, true,
-                                    col.b_e[k], col.g_e[k], ye[r][k], &ye[r][k]);
-            else
-                c[r][k] = hz_centre(m, c[r][k], dex, dey, idy, ie, false, 0.f, 0.f, 0.f, &no_x, false, 0.f, 0.f, 0.f,
-                                    &no_y);
+            c[r][k] = hz_centre(m, c[r][k], dex, dey, EDGE ? col.inv_e[k] : idy, ie, false, 0.f, 0.f, 0.f, &no_x, false,
+                                0.f, 0.f, 0.f, &no_y);
+            if constexpr (XL) {
+                xe[r][k] = x.y * xe[r][k] + x.z * keep_bits(x.w, dey);
+                c[r][k] -= m.y * xe[r][k];
+            }
+            if constexpr (EDGE) {
+                ye[r][k] = col.b_e[k] * ye[r][k] + col.g_e[k] * keep_bits(col.psi_e[k], dex);
+                c[r][k] += m.y * ye[r][k];
+            }
         }
     }
 
@@ -623,10 +643,12 @@ struct MultiWindow {
         const float next = lane_next(c[r][0]);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
-            const float dh = right(c[r], k, next) - c[r][k];
+            // faces that keep their value have cb = 0, which an infinite difference would not survive
+            float dh = right(c[r], k, next) - c[r][k];
+            if constexpr (EDGE) dh = keep_bits(col.moves[k], dh);
             fx[r][k] = hz_ex(FULL ? cax[FULL ? r : 0][k] : 1.f, cbx[r][k], fx[r][k], dh, EDGE ? col.inv_h[k] : idy);
             if constexpr (EDGE) {
-                yh[r][k] = col.b_h[k] * yh[r][k] + col.g_h[k] * dh;
+                yh[r][k] = col.b_h[k] * yh[r][k] + col.g_h[k] * keep_bits(col.psi_h[k], dh);
                 fx[r][k] += cbx[r][k] * yh[r][k];
             }
         }
@@ -638,10 +660,11 @@ struct MultiWindow {
         const float4 x = XL ? lds_row[2 * (wave * R + r)] : float4{};
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
-            const float dh = above[k] - c[r][k];
+            float dh = above[k] - c[r][k];
+            if constexpr (EDGE) dh = keep_bits(((stays >> r) & 1) - 1u, dh);
             fy[r][k] = hz_ey(FULL ? cay[FULL ? r : 0][k] : 1.f, cby[r][k], fy[r][k], dh, XL ? x.x : idx);
             if constexpr (XL) {
-                xh[r][k] = x.z * xh[r][k] + x.w * dh;
+                xh[r][k] = x.y * xh[r][k] + x.z * keep_bits(x.w, dh);
                 fy[r][k] -= cby[r][k] * xh[r][k];
             }
         }
@@ -992,8 +1015,8 @@ struct MultiWindow {
             const yee_cpml_axis& cx = d.cpml[0];
             const int lane = threadIdx.x & (YEE_WAVE - 1);
             const int h = max(early.row_h, 0), e = max(early.row_e, 0);
-            const float4 a = make_float4(early.inv_h, early.inv_e, cx.b_h[h], cx.g_h[h]);
-            const float4 b = make_float4(cx.b_e[e], cx.g_e[e], 0.f, 0.f);
+            const float4 a = make_float4(early.inv_h, cx.b_h[h], cx.g_h[h], 0.f);
+            const float4 b = make_float4(early.inv_e, cx.b_e[e], cx.g_e[e], 0.f);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 ph[r] = __builtin_amdgcn_readlane(early.row_h, r);
@@ -1002,8 +1025,10 @@ struct MultiWindow {
             load();
             if (lane < R) {
                 const bool layer_h = early.row_h >= 0, layer_e = early.row_e >= 0;
-                lds_row[2 * (wave * R + lane)] = make_float4(a.x, a.y, layer_h ? a.z : 0.f, layer_h ? a.w : 0.f);
-                lds_row[2 * (wave * R + lane) + 1] = make_float4(layer_e ? b.x : 0.f, layer_e ? b.y : 0.f, 0.f, 0.f);
+                lds_row[2 * (wave * R + lane)] = make_float4(a.x, layer_h ? a.y : 0.f, layer_h ? a.z : 0.f,
+                                                             __uint_as_float(layer_h ? ~0u : 0u));
+                lds_row[2 * (wave * R + lane) + 1] = make_float4(b.x, layer_e ? b.y : 0.f, layer_e ? b.z : 0.f,
+                                                                 __uint_as_float(layer_e ? ~0u : 0u));
             }
         } else {
             load();

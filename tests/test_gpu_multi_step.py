@@ -182,3 +182,43 @@ def test_calls_of_one_and_two_steps_of_a_large_grid(gpu, pol):
             out['probes'] = sim.engine.probes.samples[:total]
         for name in a:
             assert bool((a[name] == b[name]).all()), (name, total)
+
+
+def overflowed(sim, nx, ny):
+    """Infinities and values near the largest float in and beside the layers, the grid's last rows and the bulk."""
+    torch = sim.engine.torch
+    fields = sim.engine.fields[0]
+    huge = 3.0e38
+    for c in range(3):
+        for i, j, v in ((0, 3, float('inf')), (nx - 1, ny // 3, -float('inf')), (nx // 3, ny - 1, float('inf')),
+                        (nx // 2, 0, -huge), (nx // 2 + 3, ny // 2, huge), (nx // 2 + 3, ny // 2 + 1, -huge),
+                        (NPML + 2, NPML + 2, float('inf')), (nx - NPML - 3, ny - NPML - 4, huge),
+                        (nx - NPML - 3, ny - NPML - 3, -huge)):
+            fields[c, min(max(i + c, 0), nx - 1), min(max(j + c, 0), ny - 1)] = v
+    assert torch.isinf(fields).any()
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+@pytest.mark.parametrize('nx,ny', [(34, 64), (129, 130), (300, 257)])
+@pytest.mark.parametrize('boundaries,media', [('pml', 'plain'), ('periodic_y', 'lossy'), ('periodic_x', 'plain'),
+                                              ('pml', 'pec')])
+@pytest.mark.parametrize('extras', [False, True])
+def test_overflowed_fields_stay_what_single_steps_make_of_them(gpu, pol, nx, ny, boundaries, media, extras):
+    """An infinity spreads and cancels to NaN in the same cells, however many steps a launch takes."""
+    def make():
+        return build(pol, nx, ny, boundaries, media,
+                     extras=(lambda sim, wx, wy: add_extras(sim, pol, wx, wy, 2)) if extras else None)
+    multi, single = make(), make()
+    for sim in (multi, single):
+        overflowed(sim, nx, ny)
+    total = 0
+    for steps in (1, 2, 5, 9):
+        multi.engine.step(steps)
+        single.engine.step_timed(steps)
+        total += steps
+        a, b = arrays(multi, total), arrays(single, total)
+        for name in a:
+            same = (a[name] == b[name]) | (a[name].isnan() & b[name].isnan()) if a[name].is_floating_point() else \
+                a[name] == b[name]
+            assert bool(same.all()), (name, total, int((~same).sum()))
+    assert bool(arrays(multi, total)['fields'].isnan().any())
