@@ -713,15 +713,20 @@ struct MultiWindow {
     __device__ __forceinline__ void add_line(float (&field)[R][VEC], int s, uint32_t rows, int step) const
     {
         const int lane = threadIdx.x & (YEE_WAVE - 1);
+        const int lo = d.source[s].lo, hi = d.source[s].hi;
         const float v = lds_wave[s * kMultiMax + step];
         float add[VEC];
+        bool in[VEC];   // within the span: past it an infinite value times the profile's 0 would be NaN
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) add[k] = __fmul_rn(v, lds_profile[s * 128 + VEC * lane + k]);
+        for (int k = 0; k < VEC; ++k) {
+            add[k] = __fmul_rn(v, lds_profile[s * 128 + VEC * lane + k]);
+            in[k] = col.column(k) >= lo && col.column(k) < hi;
+        }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (!((rows >> r) & 1)) continue;
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) field[r][k] += add[k];
+            for (int k = 0; k < VEC; ++k) field[r][k] = in[k] ? field[r][k] + add[k] : field[r][k];
         }
     }
     __device__ __forceinline__ void add_column(float (&field)[R][VEC], int s, uint32_t rows, int step) const

@@ -222,3 +222,16 @@ def test_overflowed_fields_stay_what_single_steps_make_of_them(gpu, pol, nx, ny,
                 a[name] == b[name]
             assert bool(same.all()), (name, total, int((~same).sum()))
     assert bool(arrays(multi, total)['fields'].isnan().any())
+
+
+def test_infinite_source_value_stays_within_its_span(gpu):
+    """A source table that holds an infinity adds it to the cells of its span and leaves the others of its line alone."""
+    def line(sim, wx, wy):
+        sim.add_line_source(axis='y', position=0.5 * wx * DX, wavelength=600e-9, span=(0.3 * wy * DX, 0.6 * wy * DX))
+    sims = [build('ez', 129, 130, 'pml', 'plain', extras=line) for _ in range(2)]
+    for sim in sims:
+        sim.engine.waves[-1][2] = float('inf')
+    sims[0].engine.step(3)
+    sims[1].engine.step_timed(3)
+    a, b = (arrays(sim, 3)['fields'] for sim in sims)
+    assert bool(((a == b) | (a.isnan() & b.isnan())).all()) and bool(a.isinf().any())
