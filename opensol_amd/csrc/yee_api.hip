@@ -589,9 +589,42 @@ int32_t multi_launches(int32_t count, int32_t most)
 
 int32_t multi_steps(int32_t count, int32_t launches, int32_t k) { return count / launches + (k < count % launches); }
 
-// Tall windows: not for H_z with lossy or PEC materials, whose four coefficients a cell do not fit the registers of a
+// Bytes of spectrum records that the DFT regions of an instance read and write, a step and grid cell. `adjacent`: of the
+// regions that sample every column alone.
+double dft_bytes_per_cell(const yee2d_desc& d, bool adjacent)
+{
+    double bytes = 0.0;
+    for (int k = 0; k < d.n_dft; ++k) {
+        const yee_dft_region& r = d.dft[k];
+        if (!adjacent || r.stride[1] == 1)
+            bytes += 64.0 * r.count[0] * r.count[1] * r.n_comp * r.n_freq / d.sample_interval;
+    }
+    return bytes / ((double)d.nx * d.ny);
+}
+
+// DFT regions that are all of a step: a launch of their own streams the records better than the windows, which come to them in
+// turns. Measured (us a step, general windows / one-step kernels), 40 wavelengths every 3 steps, 2560 B a cell: H_z 300^2 101 /
+// 86, 1000^2 601 / 549, 2048^2 2535 / 2266; every 8 steps, 960 B: 39 / 55, 224 / 229, 938 / 880; E_z, 853 B: 20 / 43, 201 /
+// 204, 779 / 790.
+bool dft_dominates(const yee2d_desc& d)
+{
+    const double per_cell = dft_bytes_per_cell(d, false);
+    return per_cell >= 600.0 && per_cell * d.nx * d.ny >= 1.5e8;
+}
+
+// Tall windows: not with DFT regions that are most of a step. A lane of two columns goes over the records of its columns one
+// after the other, each time half of their cache lines. Measured (us a step; tall / general windows / one-step kernels and a
+// DFT launch), every cell sampled at 1, 3, 8, 16 wavelengths every 8 steps, 8, 24, 64, 128 B a cell in E_z, three times that
+// in H_z: E_z 4000^2 49 / 64 / 139, 136 / 116 / 191, 399 / 249 / 324, 798 / 471 / 532; H_z 137 / 121 / 211, 401 / 280 / 369,
+// 1232 / 694 / 763, 2499 / 1362 / 1393. Every second cell, where the lanes have one record each: E_z 16 wavelengths (32 B) 127
+// / 152 / 218, H_z 3 (18 B) 100 / 117 / 189, 16 (96 B) 391 / 407 / 448.
+// Nor for H_z with lossy or PEC materials, whose four coefficients a cell do not fit the registers of a
 // 128 x 64 window (1200^2: 14.5 us a step with them, 4.8 without; lossless 3.6 with them, 4.6 without).
-bool tall_windows(const yee_ctx* ctx) { return ctx->d2.polarization == YEE_EZ || ctx->lossless; }
+bool tall_windows(const yee_ctx* ctx)
+{
+    if (dft_bytes_per_cell(ctx->d2, true) >= 20.0 || dft_bytes_per_cell(ctx->d2, false) >= 96.0) return false;
+    return ctx->d2.polarization == YEE_EZ || ctx->lossless;
+}
 
 // Shape and number of launches with the least estimated time for `count` steps.
 void choose_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, int32_t* launches)
@@ -631,7 +664,7 @@ bool one_step_launches(const yee2d_desc& d, int32_t count, int32_t launches)
 
 void set_geometry(yee_ctx* ctx)
 {
-    ctx->multi = multi_ok(ctx->d2, true) && ctx->d2.step_limit == INT64_MAX;
+    ctx->multi = multi_ok(ctx->d2, true) && !dft_dominates(ctx->d2) && ctx->d2.step_limit == INT64_MAX;
     const yee2d_desc& d = ctx->d2;
     ctx->sets = tile_sets(d);
     const yee2d_tile_sets& s = ctx->sets;

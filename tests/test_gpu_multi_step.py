@@ -235,3 +235,24 @@ def test_infinite_source_value_stays_within_its_span(gpu):
     sims[1].engine.step_timed(3)
     a, b = (arrays(sim, 3)['fields'] for sim in sims)
     assert bool(((a == b) | (a.isnan() & b.isnan())).all()) and bool(a.isinf().any())
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+@pytest.mark.parametrize('downsample,wavelengths', [(1, 1), (1, 2), (1, 8), (2, 24), (1, 100)])
+def test_multi_step_with_dense_regions(gpu, pol, downsample, wavelengths):
+    """DFT regions over the whole grid, from a small share of a step to all of it: the windows and kernels chosen for them
+    take the same samples."""
+    def region(sim, wx, wy):
+        sim.add_dft_monitor(0.5 * DX, 0.5 * DX, (wx - 0.5) * DX, (wy - 0.5) * DX, downsample=downsample,
+                            wavelengths=list(np.linspace(500e-9, 800e-9, wavelengths)))
+    multi, single = (build(pol, 611, 523, 'pml', 'plain', extras=region) for _ in range(2))
+    total = 0
+    for steps in (2, 7, 20):
+        multi.engine.step(steps)
+        single.engine.step_timed(steps)
+        total += steps
+    a, b = arrays(multi, total), arrays(single, total)
+    a['dft'], b['dft'] = (sim.engine.dft_accumulators[0] for sim in (multi, single))
+    for name in a:
+        assert bool((a[name] == b[name]).all()), (name, total)
+    assert bool((a['dft'] != 0).any())
