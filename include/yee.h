@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define YEE_ABI_VERSION 20
+#define YEE_ABI_VERSION 21
 #define YEE_MAX_SOURCES 8
 #define YEE_MAX_MONITORS 4
 #define YEE_MAX_DFT 4
@@ -453,6 +453,17 @@ int32_t yee2d_set_lossless(yee_ctx* ctx, int32_t lossless);
  * (physics/em/solvers/fdtd_ez_2d.py:262-358).
  */
 int32_t yee2d_set_pole_work(yee_ctx* ctx, float* work);
+
+/*
+ * Whether calls of a 2D context (single or batch) may take several steps a launch. Default 1; yee2d_update keeps it. Same
+ * bits either way. For callers that time or pace the one-step launches. Drops cached graphs. The reference steps one at a
+ * time (physics/em/solvers/fdtd_ez_2d.py:71-119).
+ */
+int32_t yee_set_multi_step(yee_ctx* ctx, int32_t allowed);
+
+/* Steps of the first launch of yee_step(ctx, n_steps, ...) as the context now stands: 1 where a step is a launch or more, 0
+ * for no context or no steps. */
+int32_t yee_steps_per_launch(const yee_ctx* ctx, int64_t n_steps);
 
 /* The descriptor a single 2D context steps, with the defaults it resolved (rows_per_tile, lane_columns). */
 int32_t yee2d_get_desc(const yee_ctx* ctx, yee2d_desc* out);

@@ -19,6 +19,7 @@ class _Batch:
     each simulation keeps its own fields, monitors and readout."""
 
     three_d = False
+    multi_step = True   # 2D: launches of several steps allowed (yee_set_multi_step)
 
     def __init__(self, simulations, graph_steps=0, autotune=False):
         if not simulations:
@@ -74,6 +75,8 @@ class _Batch:
         stream = torch.cuda.current_stream(device).cuda_stream
         _lib.check(self._create(descs, len(self.simulations), self._descs_dev.data_ptr(), stream,
                                 ctypes.byref(self._ctx)), self._create_name)
+        if not self.multi_step:
+            _lib.check(self.lib.yee_set_multi_step(self._ctx, 0), 'yee_set_multi_step')
         if self.graph_steps:
             _lib.check(self.lib.yee_set_graph_steps(self._ctx, self.graph_steps), 'yee_set_graph_steps')
             _lib.check(self.lib.yee_build_graph(self._ctx), 'yee_build_graph')   # capture here, not in launch()

@@ -93,7 +93,6 @@ struct Batch2DWork {
     int64_t bulk_tiles = 0, edge_tiles = 0, windows = 0;
     const MultiShape* shape = nullptr;
     int32_t steps = 0;
-    int32_t least = 0;   // steps of a call below which it steps one at a time
 };
 
 }  // namespace
@@ -112,6 +111,7 @@ struct yee_ctx {
     int edge_blocks = 0;   // blocks of the edge kernel (sets.edge_parts wavefronts per tile, 4 per block)
     yee2d_tile_sets sets{};
     bool multi = false;    // several steps per launch (yee2d_multi.hip)
+    bool multi_allowed = true;   // yee_set_multi_step
     bool fused = false;    // 3D: one launch a step (yee3d.hip), else two (yee3d_split.hip)
     bool lossless = false; // yee2d_set_lossless
     // 3D
@@ -664,7 +664,7 @@ bool one_step_launches(const yee2d_desc& d, int32_t count, int32_t launches)
 
 void set_geometry(yee_ctx* ctx)
 {
-    ctx->multi = multi_ok(ctx->d2, true) && !dft_dominates(ctx->d2) && ctx->d2.step_limit == INT64_MAX;
+    ctx->multi = ctx->multi_allowed && multi_ok(ctx->d2, true) && !dft_dominates(ctx->d2) && ctx->d2.step_limit == INT64_MAX;
     const yee2d_desc& d = ctx->d2;
     ctx->sets = tile_sets(d);
     const yee2d_tile_sets& s = ctx->sets;
@@ -904,12 +904,8 @@ Batch2DArgs batch2d_args(void* base, int32_t n, const Batch2DWork& work, int32_t
 // Calls of fewer steps than this step one at a time: a batch's windows are laid out once, for the steps of its full
 // launches, and their halos would cost more than the launches they save.
 constexpr int32_t kMultiBatchLeast = 4;
-// Batches of fewer cells than this in calls of fewer steps also step one at a time. Not for speed: members of 84 x 69 and
-// 61 x 73 cells take 44 us a step so in calls of 25, and 9 with several steps a launch. A server that preempts a long job of
-// a few thousand cells between such calls (tests/test_gpu_serve.py, 3000 steps and a rival after 50 ms) counts on its
-// still running then.
-constexpr int64_t kMultiBatchCells = 1 << 14;
-constexpr int32_t kMultiBatchShort = 32;
+
+bool takes_multi_batch(const Batch2DWork& work, int32_t count) { return work.shape && count >= kMultiBatchLeast; }
 
 // `count` steps of a batch whose members all share launches of up to work.steps steps, and one launch more for members
 // that end with the wrong parity (yee2d_multi_batch_kernel).
@@ -942,7 +938,7 @@ int32_t launch_batch_2d(const Batch2DArgs& b, int32_t count, hipStream_t stream)
     const int bulk_blocks = (int)((b.work.bulk_tiles + 3) / 4);
     const int edge_blocks = (int)((b.work.edge_tiles + 3) / 4);
     const BatchAux2D& a = b.aux;
-    const bool multi = b.work.shape && count >= b.work.least;
+    const bool multi = takes_multi_batch(b.work, count);
     if (multi) {
         const int32_t status = launch_multi_batch_2d(b, count, stream);
         if (status != YEE_OK) return status;
@@ -980,14 +976,29 @@ int32_t ensure_side(yee_ctx* ctx)
     return YEE_OK;
 }
 
+// Whether `count` steps of a single 2D instance take several a launch, and in which shape and number of launches.
+bool takes_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, int32_t* launches)
+{
+    if (ctx->kind != kSingle2D || !ctx->multi) return false;
+    choose_multi(ctx, count, shape, launches);
+    return *shape && !one_step_launches(ctx->d2, count, *launches);
+}
+
+// What a batch launches, several steps a launch only if allowed.
+Batch2DWork batch_work(const yee_ctx* ctx)
+{
+    Batch2DWork work = ctx->batch;
+    if (!ctx->multi_allowed) work.shape = nullptr;
+    return work;
+}
+
 // Launch `count` steps (offsets 0..count-1 from the device clock) followed by the clock advance.
 int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
 {
     if (count <= 0) return YEE_OK;
     const MultiShape* shape = nullptr;
     int32_t launches = 0;
-    if (ctx->kind == kSingle2D && ctx->multi) choose_multi(ctx, count, &shape, &launches);
-    if (shape && !one_step_launches(ctx->d2, count, launches)) {
+    if (takes_multi(ctx, count, &shape, &launches)) {
         for (int32_t k = 0, offset = 0; k < launches; ++k) {
             const yee2d_multi_plan plan = multi_plan(ctx->d2, multi_steps(count, launches, k), *shape, tall_windows(ctx));
             const int blocks = (plan.blocks + 7) / 8 * 8;   // a multiple of the XCDs
@@ -1101,7 +1112,7 @@ int32_t launch_steps(yee_ctx* ctx, int32_t count, hipStream_t stream)
         return YEE_OK;
     }
     if (ctx->kind == kBatch2D)
-        return launch_batch_2d(batch2d_args(ctx->descs_dev, ctx->n_inst, ctx->batch, ctx->descs[0].lane_columns,
+        return launch_batch_2d(batch2d_args(ctx->descs_dev, ctx->n_inst, batch_work(ctx), ctx->descs[0].lane_columns,
                                             batch_aux_2d(ctx->descs.data(), ctx->n_inst)),
                                count, stream);
     return fail(YEE_ESTATE, "context has no instances");
@@ -1151,13 +1162,9 @@ yee2d_multi_plan batch_plan(const yee2d_desc& d, int32_t steps, const MultiShape
 // none when a member's features need one step a launch.
 void choose_multi_batch(const yee2d_desc* descs, int32_t n, int32_t count, Batch2DWork* work)
 {
-    int64_t cells = 0;
-    for (int32_t k = 0; k < n; ++k) {
+    for (int32_t k = 0; k < n; ++k)
         if (!multi_ok(descs[k], false)) return;
-        cells += (int64_t)descs[k].nx * descs[k].ny;
-    }
-    work->least = cells < kMultiBatchCells ? kMultiBatchShort : kMultiBatchLeast;
-    if (count < work->least) return;
+    if (count < kMultiBatchLeast) return;
     float best = 0.f;
     for (const MultiShape& s : kMultiShape) {
         for (int32_t steps = kMultiBatchLeast; s.batch && steps <= std::min(s.most, count); ++steps) {
@@ -1318,6 +1325,28 @@ int32_t yee2d_set_lossless(yee_ctx* ctx, int32_t lossless)
     if (ctx->lossless != (lossless != 0)) drop_graph(ctx);
     ctx->lossless = lossless != 0;
     return YEE_OK;
+}
+
+int32_t yee_set_multi_step(yee_ctx* ctx, int32_t allowed)
+{
+    if (!ctx || (ctx->kind != kSingle2D && ctx->kind != kBatch2D)) return fail(YEE_ESTATE, "not a 2D context");
+    if (ctx->multi_allowed != (allowed != 0)) drop_graph(ctx);
+    ctx->multi_allowed = allowed != 0;
+    if (ctx->kind == kSingle2D) set_geometry(ctx);
+    return YEE_OK;
+}
+
+int32_t yee_steps_per_launch(const yee_ctx* ctx, int64_t n_steps)
+{
+    if (!ctx || n_steps < 1) return 0;
+    const bool graph = ctx->graph_steps > 0 && n_steps >= ctx->graph_steps;
+    const int32_t count = graph ? ctx->graph_steps : (int32_t)std::min<int64_t>(n_steps, kStepChunk);
+    const MultiShape* shape = nullptr;
+    int32_t launches = 0;
+    if (takes_multi(ctx, count, &shape, &launches)) return multi_steps(count, launches, 0);
+    if (ctx->kind == kBatch2D && takes_multi_batch(batch_work(ctx), count))
+        return multi_steps(count, multi_launches(count, ctx->batch.steps), 0);
+    return 1;
 }
 
 int32_t yee2d_batch_create(const yee2d_desc* descs, int32_t n, void* descs_dev, void* stream, yee_ctx** out)

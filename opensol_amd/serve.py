@@ -122,6 +122,9 @@ def choose_victims(head_bytes, free_bytes, running):
     return chosen if free >= head_bytes else []
 
 
+PACED_CELLS, PACED_STEPS = 1 << 14, 32   # FDTDServer._paced
+
+
 class FDTDServer:
     """Continuous-batching server over one GPU. hbm_budget [B] bounds the resident device state; chunk_steps is the
     granularity at which jobs join and leave; preempt_after [s], if set, lets a queued job that has waited that long
@@ -220,6 +223,13 @@ class FDTDServer:
             return []   # refused at admission, or it fits anyway
         running = [j for j in active if j.done_steps < j.steps and j.status == 'running']
         return choose_victims(need, self.hbm_budget - self._used, running)
+
+    def _paced(self, members):
+        """Whether a chunk's members step one launch at a time: with preemption, short chunks and few cells. Preemption
+        is by the clock, and such jobs would be over before a rival has waited (84 x 69 and 61 x 73 cells in chunks of
+        25 take 44 us a step so, 9 with several steps a launch)."""
+        return (self.preempt_after is not None and self.chunk_steps < PACED_STEPS and not members[0].three_d
+                and sum(j.cells for j in members) < PACED_CELLS)
 
     def _preempt(self, job, pending, active):
         """Move a running job's state to the host, free its device state and queue it behind the head job."""
@@ -340,6 +350,7 @@ class FDTDServer:
                     stream = streams[parity][kind_index]
                     with torch.cuda.stream(stream):
                         batch = kind([j.sim for j in members], graph_steps=self.graph_steps)
+                        batch.multi_step = not self._paced(members)
                         counts = [min(self.chunk_steps, j.steps - j.done_steps) for j in members]
                         batch.prepare(counts)   # synchronizes this stream, which holds only finished chunks
                         stream.wait_stream(main)   # new engines were zeroed on the main stream

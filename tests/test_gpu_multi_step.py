@@ -256,3 +256,22 @@ def test_multi_step_with_dense_regions(gpu, pol, downsample, wavelengths):
     for name in a:
         assert bool((a[name] == b[name]).all()), (name, total)
     assert bool((a['dft'] != 0).any())
+
+
+def test_small_batches_take_several_steps_a_launch(gpu):
+    """Two small members in calls of 25 steps: several steps a launch, unless the batch is told to take one."""
+    from opensol_amd.batch import Batch2D
+    members, singles = ([build('ez', 84, 69, 'pml', 'plain'), build('hz', 61, 73, 'pml', 'plain')] for _ in range(2))
+    paced, free = Batch2D(singles), Batch2D(members)
+    paced.multi_step = False
+    for batch, several in ((paced, False), (free, True)):
+        for _ in range(3):
+            batch.prepare(25)
+            assert (batch.lib.yee_steps_per_launch(batch._ctx, 25) > 1) == several
+            batch.launch()
+    for a, b in zip(members, singles):
+        got, expected = arrays(a, 75), arrays(b, 75)
+        for name in got:
+            assert bool((got[name] == expected[name]).all()), name
+    paced.close()
+    free.close()
