@@ -275,3 +275,21 @@ def test_small_batches_take_several_steps_a_launch(gpu):
             assert bool((got[name] == expected[name]).all()), name
     paced.close()
     free.close()
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+@pytest.mark.parametrize('axis', ['x', 'y'])
+def test_periodic_axis_with_layers(gpu, pol, axis):
+    """A descriptor may wrap an axis that has CPML rows, which no model does: both launch forms step it alike."""
+    import ctypes
+    from opensol_amd import _lib
+    sims = [build(pol, 129, 130, 'pml', 'lossy') for _ in range(2)]
+    for sim in sims:
+        d = sim.engine.descriptor()
+        setattr(d, f'periodic_{axis}', 1)
+        _lib.check(sim.engine.lib.yee2d_update(sim.engine._ctx, ctypes.byref(d)), 'yee2d_update')
+    sims[0].engine.step(20)
+    sims[1].engine.step_timed(20)
+    a, b = (arrays(sim, 20) for sim in sims)
+    for name in a:
+        assert bool((a[name] == b[name]).all()), name

@@ -57,6 +57,18 @@ def test_calls_take_several_steps_a_launch_unless_told_otherwise(lib):
     assert lib.yee_steps_per_launch(None, 5) == 0
 
 
+def test_layers_of_a_periodic_x_axis_are_stepped_one_launch_at_a_time(lib):
+    """The windows hold the x layers' rows by the grid's own index, so they do not follow a wrap around such an axis."""
+    d = descriptor(300, 257)
+    layers(d, 0, 16)
+    assert steps_per_launch(lib, d, 100) > 3
+    d.periodic_x = 1
+    assert steps_per_launch(lib, d, 100) == 1
+    d.periodic_x, d.periodic_y = 0, 1
+    layers(d, 1, 16)
+    assert steps_per_launch(lib, d, 100) > 3
+
+
 def test_a_server_paces_small_members_only_when_it_preempts():
     from opensol_amd.serve import FDTDServer, Job
     small = [Job(build=None, steps=10, arrival=0.0, cells=5000) for _ in range(2)]
