@@ -526,6 +526,7 @@ const MultiShape kMultiShape[] = {multi_shape<1, 8, 2, 8, 8>(14, 11.0f, 1.25f, 3
                                   multi_shape<1, 4, 1, 0, 8>(12, 6.7f, 0.8f, 11.0f, 0.25f,
                                                              yee2d_multi_batch_kernel<1, 4, 1, 0, 8>),
                                   multi_shape<1, 2, 1, 0, 8>(7, 4.5f, 0.7f, 7.5f, 0.2f, nullptr)};
+constexpr int32_t kMultiWindows = (1 << 23) - 8;   // of a launch: it holds less than 2^32 threads, 512 a window
 constexpr int32_t kMultiSideBySide = 400;   // windows that run at once (two blocks of 8 wavefronts a CU, unevenly)
 
 void add_region(yee2d_multi_plan& p, int32_t i0, int32_t i1, int32_t j0, int32_t j1, int32_t rows, int32_t columns)
@@ -627,17 +628,20 @@ bool tall_windows(const yee_ctx* ctx)
     return ctx->d2.polarization == YEE_EZ || ctx->lossless;
 }
 
-// Shape and number of launches with the least estimated time for `count` steps.
+// Shape and number of launches with the least estimated time for `count` steps (none: grids of a few rows and hundreds of
+// millions of columns, whose windows no launch holds).
 void choose_multi(const yee_ctx* ctx, int32_t count, const MultiShape** shape, int32_t* launches)
 {
     float best = 0.f;
     *shape = nullptr;
+    const bool tall = tall_windows(ctx);
     for (const MultiShape& s : kMultiShape)
         for (int32_t most = 1; most <= std::min(s.most - multi_pad(ctx->d2), count); ++most) {
             const int32_t n = multi_launches(count, most);
             const int32_t steps = multi_steps(count, n, 0);
-            const float time = n * multi_time(multi_plan(ctx->d2, steps, s, tall_windows(ctx)).blocks, steps, s);
-            if (!*shape || time < best) {
+            const int32_t windows = multi_plan(ctx->d2, steps, s, tall).blocks;
+            const float time = n * multi_time(windows, steps, s);
+            if (windows <= kMultiWindows && (!*shape || time < best)) {
                 best = time;
                 *shape = &s;
                 *launches = n;
@@ -703,6 +707,7 @@ int64_t blocks_3d(const yee3d_desc& d, bool fused)
     return chunks * ((((int64_t)d.ny * d.nz + 255) / 256 + 7) / 8 * 8);
 }
 constexpr int kThreads3D = 64 * (yee3idx::kRows + 2);
+constexpr int64_t kBlocks3D = (int64_t)1 << 22;   // a fused launch of this many blocks has the 2^32 threads that none holds
 int grid_3d(int64_t blocks) { return (int)((blocks + 7) / 8 * 8); }   // a multiple of the XCDs
 
 // Defaults of a 3D descriptor.
@@ -714,8 +719,7 @@ void apply_defaults_3d(yee3d_desc& d, bool fused)
         const int64_t chunks = (d.nx + planes - 1) / planes;
         d.planes_per_tile = (int32_t)((d.nx + chunks - 1) / chunks);
     }
-    // a launch holds at most 2^32 threads
-    while (fused && d.planes_per_tile > 0 && d.planes_per_tile < d.nx && blocks_3d(d, fused) >= (int64_t)1 << 22)
+    while (fused && d.planes_per_tile > 0 && d.planes_per_tile < d.nx && blocks_3d(d, fused) >= kBlocks3D)
         d.planes_per_tile *= 2;
 }
 
@@ -1172,7 +1176,7 @@ void choose_multi_batch(const yee2d_desc* descs, int32_t n, int32_t count, Batch
             int64_t windows = 0;
             for (int32_t k = 0; k < n; ++k) windows += batch_plan(descs[k], steps, s).blocks;
             const float time = multi_time(windows, steps, s) / (float)steps;
-            if (windows > INT32_MAX / 16 || (work->shape && time >= best)) continue;
+            if (windows > kMultiWindows || (work->shape && time >= best)) continue;
             best = time;
             work->shape = &s;
             work->steps = steps;

@@ -69,6 +69,13 @@ def test_layers_of_a_periodic_x_axis_are_stepped_one_launch_at_a_time(lib):
     assert steps_per_launch(lib, d, 100) > 3
 
 
+@pytest.mark.parametrize('nx,ny,several', [(2, 2_000_000_000, False), (2, 300_000_000, True), (100_000, 100_000, True)])
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+def test_grids_with_more_windows_than_a_launch_holds_step_one_launch_at_a_time(lib, pol, nx, ny, several):
+    """A launch has fewer than 2^32 threads, 512 a window of at most 64 columns."""
+    assert (steps_per_launch(lib, descriptor(nx, ny, pol), 100) > 1) == several
+
+
 def test_a_server_paces_small_members_only_when_it_preempts():
     from opensol_amd.serve import FDTDServer, Job
     small = [Job(build=None, steps=10, arrival=0.0, cells=5000) for _ in range(2)]
