@@ -1642,7 +1642,15 @@ int32_t yee3d_batch_create(const yee3d_desc* descs, int32_t n, void* descs_dev, 
     std::vector<int32_t> block_prefix(n + 1, 0);
     int64_t cells = 0;
     for (const yee3d_desc& d : host) cells += cells_3d(d);
-    const bool fused = cells >= kFused3D;
+    bool fused = cells >= kFused3D;
+    if (fused) {   // members of many short tiles together may have more blocks than a fused launch holds
+        int64_t blocks = 0;
+        for (yee3d_desc d : host) {
+            apply_defaults_3d(d, fused);
+            if (check_3d(&d) == YEE_OK) blocks += blocks_3d(d, fused);
+        }
+        fused = blocks < kBlocks3D;
+    }
     for (int32_t k = 0; k < n; ++k) {
         apply_defaults_3d(host[k], fused);
         const int32_t status = check_3d(&host[k]);
