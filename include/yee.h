@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define YEE_ABI_VERSION 21
+#define YEE_ABI_VERSION 22
 #define YEE_MAX_SOURCES 8
 #define YEE_MAX_MONITORS 4
 #define YEE_MAX_DFT 4
@@ -502,6 +502,9 @@ int32_t yee2d_batch_create(const yee2d_desc* descs, int32_t n, void* descs_dev, 
  * counterpart in the reference, which steps one model at a time (model/study.py:437-447).
  */
 size_t yee3d_batch_bytes(int32_t n);
+/* Whether a 3D instance, or a batch, of `cells` cells in sum steps in one fused launch (1) or in an H and an E launch (0): what
+ * a planes_per_tile other than 0 is chosen for. */
+int32_t yee3d_fused(int64_t cells);
 int32_t yee3d_batch_create(const yee3d_desc* descs, int32_t n, void* descs_dev, void* stream, yee_ctx** out);
 
 /*

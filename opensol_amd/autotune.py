@@ -9,11 +9,17 @@ batched launch, whose kernels differ:
   * single 2D instance: columns per lane x rows per tile, timed on a throwaway engine over the same model;
   * single 3D instance: x planes per tile, likewise;
   * batch member, 2D: rows per tile (columns per lane are shared by the whole batch), timed as a one-member batch
-    (Batch2D over a throwaway engine, the same kernels a real batch launches);
+    (Batch2D over a throwaway engine);
   * batch member, 3D: x planes per tile, timed as a one-member Batch3D.
 
+The 2D options are those of the one-step kernels, which step instances with walls, TFSF or other poles, batches with any of
+those, DFT regions or probes, and the shortest calls; launches of several steps read none of them. So they are timed with
+one step a launch, whatever the model would take. In 3D there are two step forms, one fused launch and an H and an E launch
+(yee3d_fused): the form is part of the class, and a member tuned in one form goes into a batch of the other one with that
+form's default.
+
 The cache file is JSON, {device: {class key: {"options": ..., "ms": {candidate: ms per step}}}}, with the device named
-by its architecture and compute-unit count (e.g. "gfx950:256"). Its path is OPENSOL_AMD_TUNE_CACHE, else
+by its architecture, compute-unit count and the generation of the kernels (e.g. "gfx950:256:k2"). Its path is OPENSOL_AMD_TUNE_CACHE, else
 ~/.cache/opensol_amd/autotune.json; it is written atomically after every new class. Batch2D / Batch3D take
 autotune=True, FDTDServer(autotune=True) tunes every admitted job's class before its engine exists, and bench.py
 tunes the batched workload's members before its timed region.
@@ -28,7 +34,9 @@ import threading
 CANDIDATES_2D = [(2, 0), (2, 16), (2, 32), (2, 64), (4, 0), (4, 32)]
 CANDIDATES_3D = [0, 4, 8, 16, 32, 64]
 BATCH_ROWS_2D = [8, 16, 32, 64]
-BATCH_PLANES_3D = [2, 4, 8]
+BATCH_PLANES_3D = [1, 2, 4, 8]
+BATCH_PLANES_3D_FUSED = [8, 16, 32]
+KERNELS = 2   # goes up when other kernels or launch rules make the cached choices stale
 
 
 def size_class(shape):
@@ -103,7 +111,26 @@ def default_cache():
 
 def device_key(torch, device=None):
     props = torch.cuda.get_device_properties(torch.cuda.current_device() if device is None else device)
-    return f'{getattr(props, "gcnArchName", props.name).split(":")[0]}:{props.multi_processor_count}'
+    return f'{getattr(props, "gcnArchName", props.name).split(":")[0]}:{props.multi_processor_count}:k{KERNELS}'
+
+
+def fused_3d(model):
+    """Whether a 3D model alone steps in one fused launch."""
+    from . import _lib
+    return bool(_lib.load().yee3d_fused(math.prod(int(n) for n in model.shape)))
+
+
+def tuned_key(kind, model, lane_columns=2):
+    """Cache key of a model's choice: its size class, with the step form (3D) or a batch's columns per lane (2D)."""
+    if len(model.shape) == 3:
+        return class_key(kind, model) + (':fused' if fused_3d(model) else ':split')
+    return class_key(kind, model) + (f':lanes{int(lane_columns)}' if kind == 'batch' else '')
+
+
+def _apply(sim, options):
+    sim._engine_options.update(options)
+    if len(sim.model.shape) == 3:
+        sim._planes_fused = fused_3d(sim.model)   # Batch3D: the form the planes were chosen for
 
 
 def _elapsed_ms(run, steps, torch):
@@ -146,10 +173,10 @@ def tune(sim, steps=10, candidates=None, use_cache=True, cache=None):
     if sim.engine is not None:
         raise ValueError('tune() chooses launch options before the first run()')
     model = sim.model
-    key = class_key('single', model)
+    key = tuned_key('single', model)
     cache, device, options = _lookup(key, cache, use_cache, torch)
     if options is not None:
-        sim._engine_options.update(options)
+        _apply(sim, options)
         return options, {}
     model.finalize()
     timings = {}
@@ -163,9 +190,11 @@ def tune(sim, steps=10, candidates=None, use_cache=True, cache=None):
                 engine.close()
         options = {'planes_per_tile': min(timings, key=timings.get)}
     else:
+        from . import _lib
         from .fdtd2d import Engine2D
         for lanes, rows in candidates or CANDIDATES_2D:
             engine = Engine2D(model, lane_columns=lanes, rows_per_tile=rows, capacity=steps + 4)
+            _lib.check(engine.lib.yee_set_multi_step(engine._ctx, 0), 'yee_set_multi_step')
             try:
                 timings[(lanes, rows)] = _elapsed_ms(engine.step, steps, torch)
             finally:
@@ -173,7 +202,7 @@ def tune(sim, steps=10, candidates=None, use_cache=True, cache=None):
         lanes, rows = min(timings, key=timings.get)
         options = {'lane_columns': lanes, 'rows_per_tile': rows}
     torch.cuda.empty_cache()
-    sim._engine_options.update(options)
+    _apply(sim, options)
     cache.put(device, key, options, timings)
     return options, timings
 
@@ -200,16 +229,16 @@ def tune_batch_member(sim, steps=10, lane_columns=2, candidates=None, use_cache=
         raise ValueError('tune_batch_member() chooses launch options before the engine exists')
     model = sim.model
     three = len(model.shape) == 3
-    key = class_key('batch', model) + ('' if three else f':lanes{int(lane_columns)}')
+    key = tuned_key('batch', model, lane_columns)
     cache, device, options = _lookup(key, cache, use_cache, torch)
     if options is not None:
-        sim._engine_options.update(options)
+        _apply(sim, options)
         return options, {}
     model.finalize()
     timings = {}
     if three:
         from .fdtd3d import Engine3D
-        for planes in candidates or BATCH_PLANES_3D:
+        for planes in candidates or (BATCH_PLANES_3D_FUSED if fused_3d(model) else BATCH_PLANES_3D):
             engine = Engine3D(model, planes_per_tile=planes, capacity=steps + 8)
             batch = Batch3D([_Member(model, engine)])
             try:
@@ -223,6 +252,7 @@ def tune_batch_member(sim, steps=10, lane_columns=2, candidates=None, use_cache=
         for rows in candidates or BATCH_ROWS_2D:
             engine = Engine2D(model, lane_columns=lane_columns, rows_per_tile=rows, capacity=steps + 8)
             batch = Batch2D([_Member(model, engine)], lane_columns=lane_columns)
+            batch.multi_step = False
             try:
                 timings[rows] = _batch_ms(batch, steps, torch)
             finally:
@@ -230,7 +260,7 @@ def tune_batch_member(sim, steps=10, lane_columns=2, candidates=None, use_cache=
                 engine.close()
         options = {'rows_per_tile': min(timings, key=timings.get)}
     torch.cuda.empty_cache()
-    sim._engine_options.update(options)
+    _apply(sim, options)
     cache.put(device, key, options, timings)
     return options, timings
 
@@ -240,5 +270,5 @@ def clear_cache():
     default_cache().clear()
 
 
-__all__ = ['tune', 'tune_batch_member', 'size_class', 'class_key', 'TuneCache', 'default_cache', 'clear_cache',
-           'CANDIDATES_2D', 'CANDIDATES_3D', 'BATCH_ROWS_2D', 'BATCH_PLANES_3D']
+__all__ = ['tune', 'tune_batch_member', 'size_class', 'class_key', 'tuned_key', 'TuneCache', 'default_cache', 'clear_cache',
+           'CANDIDATES_2D', 'CANDIDATES_3D', 'BATCH_ROWS_2D', 'BATCH_PLANES_3D', 'BATCH_PLANES_3D_FUSED']

@@ -68,6 +68,7 @@ class _Batch:
             engine._ensure_capacity(engine.n_step + count)
             descs[k] = self._cached_descriptor(engine)
             descs[k].step_limit = engine.n_step + count
+            self._adjust(descs[k], sim)
         size = self._bytes(len(self.simulations))
         torch = self.torch
         device = self.simulations[0].engine.device
@@ -81,6 +82,9 @@ class _Batch:
             _lib.check(self.lib.yee_set_graph_steps(self._ctx, self.graph_steps), 'yee_set_graph_steps')
             _lib.check(self.lib.yee_build_graph(self._ctx), 'yee_build_graph')   # capture here, not in launch()
         return longest
+
+    def _adjust(self, desc, sim):
+        """What a member's descriptor owes to the batch it is in."""
 
     def _cached_descriptor(self, engine):
         """The engine's batch descriptor, rebuilt only when its tables or options change (a chunked caller prepares
@@ -188,6 +192,12 @@ class Batch3D(_Batch):
         if self.planes_per_tile:
             d.planes_per_tile = self.planes_per_tile
         return d
+
+    def _adjust(self, desc, sim):
+        # planes tuned for the member alone are no choice for the other step form, which the whole batch's size may ask for
+        form = bool(self.lib.yee3d_fused(sum(self.cell_counts)))
+        if not self.planes_per_tile and getattr(sim, '_planes_fused', form) != form:
+            desc.planes_per_tile = 0
 
     def _options_key(self):
         return self.planes_per_tile

@@ -1632,6 +1632,8 @@ int32_t yee3d_update(yee_ctx* ctx, const yee3d_desc* desc)
     return YEE_OK;
 }
 
+int32_t yee3d_fused(int64_t cells) { return cells >= kFused3D; }
+
 int32_t yee3d_batch_create(const yee3d_desc* descs, int32_t n, void* descs_dev, void* stream, yee_ctx** out)
 {
     if (!out) return fail(YEE_EINVAL, "null output pointer");

@@ -189,11 +189,11 @@ class FDTDServer:
     def tune_classes(self, jobs):
         """Tune the batch-member launch shape of every size class among `jobs` ahead of serving them (each job is
         built once for it and dropped; a class already in the cache costs nothing). Returns the classes seen."""
-        from .autotune import class_key, tune_batch_member
+        from .autotune import tune_batch_member, tuned_key
         seen = set()
         for job in jobs:
             sim = job.build()
-            key = class_key('batch', sim.model)
+            key = tuned_key('batch', sim.model)
             if key not in seen:
                 seen.add(key)
                 tune_batch_member(sim)

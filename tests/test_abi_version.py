@@ -4,7 +4,7 @@ from opensol_amd import _lib
 from tests.test_abi import declared_functions
 
 # entry points declared at each version whose declarations changed
-DECLARED = {19: 20, 20: 22, 21: 24}
+DECLARED = {19: 20, 20: 22, 21: 24, 22: 25}
 
 
 def test_version_goes_up_with_the_declared_entry_points():
