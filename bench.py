@@ -13,7 +13,7 @@ seeded dielectric boxes (edges uniform 0.2-3 um, eps_r uniform in [1, 12]), a Ga
 
 --workload batch256: 256 seeded 2D instances (half E_z, half H_z), sides log-uniform in [128, 1024] cells, dx = 25 nm,
 12-cell CPML, 20-100 rectangles each (eps_r in [1, 12]), 1000-4000 steps each, one Gaussian line source (lambda0 in
-[0.6, 1.6] um) and one flux line at 3 wavelengths each. Reports the cell-updates/s of one batched launch per step
+[0.6, 1.6] um) and one flux line at 3 wavelengths each. Reports the cell-updates/s of the instances stepped together
 (Batch2D) and of the plain form (each instance run alone, one after another, with the same kernels and graphs).
 
 --workload serve: a seeded stream of jobs with Poisson arrivals at 50, 100, 200 and 400 jobs/s (--jobs per rate): 80 %
@@ -332,15 +332,20 @@ def run_2d(args, torch):
         # The timed region takes several steps a launch, so the state passes HBM once in several steps: the fraction is
         # of the bytes a step moves (counters), not of the 26 B a cell that step_achieved counts for every step.
         # yee_step_timed's eager one-step time (bulk and edge tiles side by side) is reported beside it.
+        # The counters were taken at one number of steps a launch and say nothing of another. A launch's cells are cell
+        # updates; what it cannot do without is the state once, however many steps it takes.
         tiles_ms, tiles_cells = kernels['tiles']
-        moved = measured_traffic(workload, 'multi_bytes_per_step')
+        per_launch = engine.steps_per_launch(args.steps)
+        moved = None
+        if measured_traffic(workload, 'multi_steps_per_launch') == per_launch:
+            moved = measured_traffic(workload, 'multi_bytes_per_step')
         achieved = None if moved is None else moved / per_step / 1e9
         roofline.update(achieved=achieved, frac=None if moved is None else achieved / HBM_PEAK_GBS,
-                        launch_ms=per_step * 1e3, cells_per_launch=cells,
-                        algorithmic_bytes_per_launch=BYTES_PER_CELL_2D * cells,
-                        kernel='yee2d_multi_kernel<EZ>, several steps a launch (period of a step)', traffic=moved,
+                        launch_ms=per_step * per_launch * 1e3, cells_per_launch=cells * per_launch,
+                        algorithmic_bytes_per_launch=BYTES_PER_CELL_2D * cells, steps_per_launch=per_launch,
+                        kernel='yee2d_multi_kernel<EZ>, several steps a launch', traffic=moved,
                         eager_tiles_ms=tiles_ms)
-        print(f'# kernels: several steps a launch, {per_step * 1e6:.1f} us per step in the timed region '
+        print(f'# kernels: {per_launch} steps a launch, {per_step * 1e6:.1f} us per step in the timed region '
               f'({"no counters" if moved is None else f"{achieved:.1f} GB/s moved"}); one step a launch '
               f'{tiles_ms * 1e3:.1f} us', file=sys.stderr, flush=True)
     elif kernels is not None:
@@ -472,23 +477,25 @@ def run_batch(args, torch):
     torch.cuda.synchronize()
     plain_s = start.elapsed_time(stop) / 1e3
     print(f'# plain: {plain_s:.3f} s, {cell_updates / plain_s:.4e} cell-updates/s', file=sys.stderr, flush=True)
-    tune_start = time.perf_counter()   # each member's rows per tile from its size class (tuned once per device)
+    # each member's rows per tile in the one-step kernels, from its size class (tuned once per device)
+    tune_start = time.perf_counter()
     batch = Batch2D(batch_sims, graph_steps=args.graph_steps, autotune=True)
     tune_s = time.perf_counter() - tune_start
     chosen = {}
     for sim in batch_sims:
         rows = int(sim._engine_options.get('rows_per_tile') or 0)
         chosen[str(rows)] = chosen.get(str(rows), 0) + 1
-    print(f'# autotuned members in {tune_s:.2f} s: rows per tile {chosen}', file=sys.stderr, flush=True)
+    print(f'# autotuned members in {tune_s:.2f} s: rows per tile of one-step launches {chosen}', file=sys.stderr, flush=True)
     batch.prepare(steps)   # descriptors and the step graph, outside the timed region
     torch.cuda.synchronize()
     start.record()
-    launches = batch.launch()
+    longest = batch.launch()
     stop.record()
     torch.cuda.synchronize()
     batch_s = start.elapsed_time(stop) / 1e3
+    per_launch = batch.steps_per_launch(longest)
     value = cell_updates / batch_s
-    print(f'# batched: {batch_s:.3f} s, {value:.4e} cell-updates/s, {launches} launches, '
+    print(f'# batched: {batch_s:.3f} s, {value:.4e} cell-updates/s, {longest} steps, {per_launch} a launch, '
           f'{(cell_updates / plain_s and value / (cell_updates / plain_s)):.2f}x plain', file=sys.stderr, flush=True)
     # every instance matches the same instance stepped alone (bit for bit; checked on a sample here and fully in
     # tests/test_gpu_batch.py)
@@ -497,13 +504,13 @@ def run_batch(args, torch):
             assert np.array_equal(plain_sims[k].engine.field(name), batch_sims[k].engine.field(name)), (k, name)
     return {'metric': 'Yee cell-updates/s, batched vs plain one-launch-per-instance', 'value': value,
             'unit': 'cell-updates/s', 'n_gpus': 1, 'steps': max(steps), 'warmup': 0,
-            'ms_per_step': batch_s / launches * 1e3, 'higher_is_better': True, 'scaling': 'weak', 'vs_baseline': None,
+            'ms_per_step': batch_s / longest * 1e3, 'higher_is_better': True, 'scaling': 'weak', 'vs_baseline': None,
             'dtype': 'f32', 'data': 'synthetic (seeded instances: rectangles, Gaussian line source, flux line)',
             'config': {'workload': 'batch256_2d_ez_hz_128to1024', 'instances': len(steps), 'seed': SEED,
                        'cell_updates': cell_updates, 'graph_steps': args.graph_steps,
                        'autotune': {'seconds': tune_s, 'rows_per_tile': chosen}},
             'plain': {'value': cell_updates / plain_s, 'seconds': plain_s},
-            'batched': {'value': value, 'seconds': batch_s, 'launches': launches},
+            'batched': {'value': value, 'seconds': batch_s, 'steps': longest, 'steps_per_launch': per_launch},
             'speedup_vs_plain': value / (cell_updates / plain_s),
             'roofline': None, 'cpu_baseline': None}
 
@@ -517,9 +524,9 @@ def main():
     parser.add_argument('--steps', type=int, default=None, help='timed steps (default 2000 2D, 500 3D)')
     parser.add_argument('--warmup', type=int, default=None, help='untimed steps (default 50 2D, 20 3D)')
     parser.add_argument('--graph-steps', type=int, default=None, help='steps per HIP graph (default 50 2D, 10 3D)')
-    parser.add_argument('--rows-per-tile', type=int, default=0, help='2D: rows per tile (0: the library default, 8)')
-    parser.add_argument('--lane-columns', type=int, default=0, choices=(0, 2, 4), help='2D: 0 = library default')
-    parser.add_argument('--planes-per-tile', type=int, default=0, help='3D: x planes per tile (0: the library default, 4)')
+    parser.add_argument('--rows-per-tile', type=int, default=0, help='2D one-step kernels: rows per tile (0: 8)')
+    parser.add_argument('--lane-columns', type=int, default=0, choices=(0, 2, 4), help='2D one-step kernels: columns per lane (0: 2)')
+    parser.add_argument('--planes-per-tile', type=int, default=0, help='3D: x planes per tile (0: the library default, by the size)')
     parser.add_argument('--cpu-steps', type=int, default=None,
                         help='steps of the CPU baseline sample (default 8 2D, 1 3D; 0 skips it)')
     parser.add_argument('--kernel-steps', type=int, default=None,

@@ -1,11 +1,12 @@
-"""Batched instances: many Simulations (2D: E_z and H_z mixed) or Simulation3Ds of uneven sizes stepped by one launch
-per step.
+"""Batched instances: many Simulations (2D: E_z and H_z mixed) or Simulation3Ds of uneven sizes stepped by the same
+launches.
 
 The reference steps one model at a time (a parameter sweep builds and runs one model per value,
-model/study.py:437-447). Here every instance keeps its own device state, clock and step limit, and one kernel launch
-per step walks the tiles of all instances (yee2d_batch_create, yee3d_batch_create): instances with fewer steps stop
-when their clock reaches their limit while the others go on, and the step loop replays from HIP graphs. An instance's
-results are the same alone and in a batch, bit for bit.
+model/study.py:437-447). Here every instance keeps its own device state, clock and step limit, and each launch walks the
+windows or tiles of all instances (yee2d_batch_create, yee3d_batch_create): in 2D several steps a launch where every member
+allows it, in 3D one step in one or two launches. Instances with fewer steps stop when their clock reaches their limit while
+the others go on, and the step loop replays from HIP graphs. An instance's results are the same alone and in a batch, bit
+for bit.
 """
 import ctypes
 
@@ -46,13 +47,13 @@ class _Batch:
 
     def run(self, n_steps):
         """Advance instance k by n_steps[k] steps (an int applies to all), asynchronously on the current stream.
-        Returns the number of launches (the largest step count)."""
+        Returns the largest step count."""
         self.prepare(n_steps)
         return self.launch()
 
     def prepare(self, n_steps):
         """Copy the descriptors for a run of n_steps[k] steps per instance to the device (synchronizes the current
-        stream once); launch() then enqueues the steps. Returns the number of launches the run will take."""
+        stream once); launch() then enqueues the steps. Returns the largest step count."""
         counts = [int(n_steps)] * len(self.simulations) if np.isscalar(n_steps) else [int(n) for n in n_steps]
         if len(counts) != len(self.simulations) or min(counts) < 0:
             raise ValueError('n_steps must be one non-negative count per simulation')
@@ -97,7 +98,7 @@ class _Batch:
         return cached[1]
 
     def launch(self):
-        """Enqueue the steps prepared by prepare() on the current stream (asynchronous); returns the launches."""
+        """Enqueue the steps prepared by prepare() on the current stream (asynchronous); returns the largest step count."""
         if not self._ctx:
             return 0
         longest = max(self._counts)
@@ -107,6 +108,10 @@ class _Batch:
             sim.engine.n_step += count
         self._counts = [0] * len(self._counts)
         return longest
+
+    def steps_per_launch(self, n_steps):
+        """Steps of the first launch of a prepared run of n_steps steps: 1 where a step is a launch or more."""
+        return self.lib.yee_steps_per_launch(self._ctx, int(n_steps))
 
     def synchronize(self):
         self.torch.cuda.synchronize(self.simulations[0].engine.device)

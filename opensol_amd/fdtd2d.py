@@ -742,6 +742,10 @@ class Engine2D:
         if self.pole_work is not None:
             _lib.check(self.lib.yee2d_set_pole_work(self._ctx, self.pole_work.data_ptr()), 'yee2d_set_pole_work')
 
+    def steps_per_launch(self, n_steps):
+        """Steps of the first launch of step(n_steps): 1 where a step is a launch or more."""
+        return self.lib.yee_steps_per_launch(self._ctx, int(n_steps))
+
     def launch_geometry(self):
         """(rows_per_tile, lane_columns) the library resolved for this instance."""
         d = _lib.Desc2DC()
