@@ -355,8 +355,8 @@ typedef struct yee3d_pole {
 typedef struct yee3d_desc {
     int32_t nx, ny, nz;
     int32_t periodic[3];
-    int32_t rows_per_tile;   /* y rows per wavefront tile: 4 (0: 4) */
-    int32_t planes_per_tile; /* x planes marched by one wavefront (0: 4, balanced over nx) */
+    int32_t rows_per_tile;   /* 4 or 0; without effect (the step forms have tiles of their own) */
+    int32_t planes_per_tile; /* x planes marched by one block (0: 1 to 4 in two launches, 16 or 32 fused, balanced over nx) */
     float* field[2][6];      /* [set][ex, ey, ez, hx, hy, hz], (nx, ny, nz) z contiguous */
     const uint16_t* material;
     const float* table;      /* (n_materials, 8) */
@@ -479,9 +479,10 @@ int32_t yee3d_get_desc(const yee_ctx* ctx, yee3d_desc* out);
 int32_t yee_destroy(yee_ctx* ctx);
 
 /*
- * Batched 2D instances (mixed E_z / H_z, uneven sizes) stepped by one launch per step over their tiles.
+ * Batched 2D instances (mixed E_z / H_z, uneven sizes) stepped together. When no member has walls, TFSF boxes, poles, DFT
+ * regions or probes, calls of 4 steps and more take several steps a launch over all members' windows.
  * descs_dev: caller device buffer of yee2d_batch_bytes(n) bytes that receives the descriptors, each member's tile sets
- * and the bulk and edge tile prefixes (copied on `stream`, which is synchronized once before the call returns). A step
+ * and plan of windows and the prefixes of their tiles and windows (copied on `stream`, which is synchronized once before the call returns). Else a step
  * is two launches: the members' bulk tiles in the lean loops and their edge tiles (CPML, source, monitor and TFSF
  * lines, E_z and H_z pole rows, H_z wall rows) in the general loops; then, when any member has them, one launch each
  * over all members for E_z wall rows, DFT regions and field probes, in the single-instance order. Members share
@@ -493,12 +494,13 @@ size_t yee2d_batch_bytes(int32_t n);
 int32_t yee2d_batch_create(const yee2d_desc* descs, int32_t n, void* descs_dev, void* stream, yee_ctx** out);
 
 /*
- * Batched 3D instances of uneven sizes stepped by one launch per step over their tiles (members with dispersive poles
- * take the E update that carries them), then one launch per mirror kind and face present in any member (symmetric
- * faces first, as a single instance orders them), one sample launch over all their flux-plane cells, and one launch
- * each over all members for DFT planes and field probes. descs_dev: caller device buffer of yee3d_batch_bytes(n) bytes
+ * Batched 3D instances of uneven sizes stepped together over their tiles (members with dispersive poles take the E update
+ * that carries them): a step is one fused launch or an H and an E launch, by the members' cells in sum (yee3d_fused), then
+ * one launch per mirror kind and face present in any member (symmetric faces first, as a single instance orders them), one
+ * sample launch over all their flux-plane cells (in the two-launch form the next step's H launch takes these samples, but
+ * for a call's last step), and one launch each over all members for DFT planes and field probes. descs_dev: caller device buffer of yee3d_batch_bytes(n) bytes
  * that receives the descriptors and the block and plane-cell prefixes (copied on `stream`, which is synchronized once
- * before the call returns). Each instance keeps its own clock, step_limit and planes_per_tile (4 rows per tile). No
+ * before the call returns). Each instance keeps its own clock, step_limit and planes_per_tile. No
  * counterpart in the reference, which steps one model at a time (model/study.py:437-447).
  */
 size_t yee3d_batch_bytes(int32_t n);
@@ -511,7 +513,7 @@ int32_t yee3d_batch_create(const yee3d_desc* descs, int32_t n, void* descs_dev, 
  * yee2d_batch_step_static: the no-allocation form of yee2d_batch_create + yee_step. No counterpart in the reference;
  * it is for callers that cannot allocate device memory (tight serving loops, harnesses that forbid hipMalloc): it
  * calls no hipMalloc / hipFree and takes no workspace. Steps n batched 2D instances (n <= YEE_STATIC_BATCH_MAX) by
- * n_steps launches on `stream`, as a batch context would: each instance stops at its step_limit and keeps its own
+ * n_steps steps on `stream`, as a batch context would: each instance stops at its step_limit and keeps its own
  * clock. The descriptors (lane_columns and rows_per_tile set, as yee2d_get_desc resolves them; the batch's other
  * rules apply), their tile sets and the tile prefixes are copied on `stream` into a static device array of the
  * library, one per GPU (yee2d_batch_bytes(YEE_STATIC_BATCH_MAX) bytes, held until the process ends),

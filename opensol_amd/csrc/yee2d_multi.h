@@ -10,12 +10,12 @@
 // that passes between wavefronts per half step goes through LDS; the rows that do not need it are computed on the near
 // side of the barrier.
 //
-// What bounds it. A step costs 174 instructions for the 8 cells of a lean E_z lane, 28 to 39 a cell in general windows;
-// a large grid is bound by the windows' loads and stores (46 ns per 128 x 64 window of 10 steps, 172 KB: 4 TB/s, with 35
-// ns at 0 steps extrapolated), a small one by the two rounds of loads before the first step (about 4 us of the 9 a
-// 7-step launch takes). Two blocks of 8 wavefronts a CU, so that one loads while the other steps: one block of 16
-// wavefronts and 128 x 128 cells took 88 us a step at 8192^2 where this takes 65 (10 steps a launch). One step a launch
-// moves the whole state and took 343. Material tables: read once, into one coefficient a cell or face, when all
+// What bounds it. A step costs 174 instructions for the 8 cells of a lean E_z lane of one column (a tall one holds 16), 30 to
+// 43 a cell in general windows; a large grid is bound by the windows' loads and stores (43 ns per 128 x 64 window of 10
+// steps, 172 KB: 4 TB/s, with 35 ns at 0 steps extrapolated), a small one by the two rounds of loads before the first step
+// (about 4 us of the 9 a 7-step launch takes). Two blocks of 8 wavefronts a CU, so that one loads while the other steps: one
+// block of 16 wavefronts and 128 x 128 cells took 88 us a step at 8192^2 where this took 65 (10 steps a launch; 61 now).
+// One step a launch moves the whole state and took 343. Material tables: read once, into one coefficient a cell or face, when all
 // materials are lossless with one mu_r (the usual case); the general form keeps or looks up all four.
 //
 // The state arrays stay double-buffered: launch k of a call reads set (clock + k) & 1 and writes the other one, and the
@@ -149,12 +149,12 @@ __device__ __forceinline__ float keep_bits(float bits, float v) { return keep_bi
 // Columns of a lane and their y constants; the lean form knows that all of them are inside the grid's bulk.
 template <int VEC, bool EDGE>
 struct LaneColumns {
+    static_assert(!EDGE || VEC == 1, "general windows hold one column a lane: two beside each other may fold apart");
     int j;                   // first column before folding
     bool owner;
     uint32_t at[VEC];        // column of the grid (a stand-in of 0 outside it)
     bool in[VEC], last[VEC]; // inside the grid; the last column of a bounded axis
     bool stays[VEC];         // fx keeps its value: the last column of a bounded axis, or outside the grid
-    bool split;              // the columns of a lane are not adjacent after folding
     int ry_h[VEC], ry_e[VEC];
     float inv_e[VEC], inv_h[VEC], b_h[VEC], g_h[VEC], b_e[VEC], g_e[VEC];
     uint32_t psi_h[VEC], psi_e[VEC], moves[VEC];   // all bits set, or none: has a psi row; not `stays` (keep_bits)
@@ -169,7 +169,6 @@ struct LaneColumns {
         if constexpr (EDGE) {
             const int ny = d.ny;
             const bool py = d.periodic_y != 0;
-            split = VEC > 1 && py && (ny % VEC) != 0;
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
                 int c = j + k;
@@ -241,13 +240,6 @@ struct LaneColumns {
 
     __device__ __forceinline__ void read(const float* __restrict__ row, float out[VEC]) const
     {
-        if constexpr (EDGE) {
-            if (split) {
-#pragma unroll
-                for (int k = 0; k < VEC; ++k) out[k] = row[at[k]];
-                return;
-            }
-        }
         load_n<VEC>(row + at[0], out);
     }
 };
@@ -284,7 +276,7 @@ __device__ __forceinline__ bool stage_multi_tables(const yee2d_desc& d)
 // What a window loads first, before its form (FULL or not) and state set are known.
 template <int VEC, int R, bool EDGE>
 struct WindowEarly {
-    static constexpr int IDS = EDGE || VEC == 1 ? VEC : VEC / 2;   // one to a register, or two
+    static constexpr int IDS = VEC == 1 ? VEC : VEC / 2;   // one to a register, or two
     LaneColumns<VEC, EDGE> col;
     uint32_t ids[R + 1][IDS];    // ids of the rows (H_z: and of the one after them)
     float inv_h, inv_e;          // lane r: x constants of row r (windows with x layers)
@@ -350,7 +342,7 @@ struct MultiWindow {
         for (int r = 0; r < R + 1; ++r) {
             if (r == R && !HZ) break;
             const uint16_t* row = d.material + (int64_t)max(0, fold_row(d, q0 + r)) * d.pitch;
-            if constexpr (EDGE || VEC == 1) {
+            if constexpr (VEC == 1) {
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) out.ids[r][k] = row[out.col.at[k]];
             } else {
@@ -928,10 +920,6 @@ struct MultiWindow {
             const int q = q0 + r;
             if (q < w.i0 || q >= w.i1) continue;
             const int64_t base = (int64_t)q * d.pitch + col.j;
-            if constexpr (EDGE && HZ) {   // padding columns stay 0 (those of E_z and of the faces never left it)
-#pragma unroll
-                for (int k = 0; k < VEC; ++k) c[r][k] = col.in[k] ? c[r][k] : 0.f;
-            }
             store_n<VEC>(d.field[out][0] + base, c[r]);
             store_n<VEC>(d.field[out][1] + base, fx[r]);
             store_n<VEC>(d.field[out][2] + base, fy[r]);

@@ -1,6 +1,6 @@
 // Fused 3D Yee step for gfx950: one launch advances a 3D instance by one full step (H update with its CPML on every
-// axis, E update with its CPML, point dipole injection); a second, small launch takes the FP64 Kahan DFT samples of
-// the flux planes on sample steps.
+// axis, E update with its CPML, point dipole injection); a second, small launch takes what is sampled after a step
+// (yee3d_after.h).
 //
 // It takes instances and batches from kFused3D cells (yee_api.hip) on; smaller ones step in two launches (yee3d_split.hip).
 //
@@ -545,12 +545,6 @@ __global__ void __launch_bounds__(64 * yee3::WAVES) yee3d_batch_kernel(const yee
 
 template __global__ void yee3d_step_kernel<false>(yee3d_desc, int32_t, int32_t);
 template __global__ void yee3d_step_kernel<true>(yee3d_desc, int32_t, int32_t);
-
-// FP64 Kahan DFT samples of the flux planes after step n (when (n + 1) % m == 0): one thread per plane cell and pair;
-// E = mean of the layers edge - 1 and edge along the normal, H on layer edge - 1 (monitors3d.py:90-101).
-namespace yee3 {
-
-}  // namespace yee3
 
 // Samples after step n = *clock + offset (after_block). The descriptor is read in place.
 __global__ void __launch_bounds__(256) yee3d_after_kernel(yee3d_desc desc, yee3d_after a, int32_t offset)

@@ -5,7 +5,8 @@
 
 namespace yee3 {
 
-// Sample of plane cell t (cells of plane 0 pair 0, then pair 1, then plane 1 ...) after step n.
+// FP64 Kahan DFT sample of plane cell t (cells of plane 0 pair 0, then pair 1, then plane 1 ...) after step n, when (n + 1) % m
+// == 0: E = mean of the layers edge - 1 and edge along the normal, H on layer edge - 1 (monitors3d.py:90-101).
 __device__ __forceinline__ void sample_cell(const yee3d_desc& d, int64_t n, int64_t t)
 {
     if (n >= d.step_limit || d.n_planes == 0) return;

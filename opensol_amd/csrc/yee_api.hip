@@ -683,7 +683,9 @@ void set_geometry(yee_ctx* ctx)
 
 // Instances and batches of at least this many cells step in one fused launch (yee3d.hip), smaller ones in an H and an E
 // launch (yee3d_split.hip). Measured, us a step, fused / split at the planes per tile below: 140 x 130 x 120 (2.2M cells)
-// 53 / 37, 256^3 (16.8M) 265 / 293, 512^3 1640 / 2120.
+// 53 / 37, 256^3 (16.8M) 265 / 293, 512^3 1640 / 2120. Batches, whose members the fused tiles of 64 x 14 cells fill worse, go
+// either way past it, by less than a tenth: members of 64 to 192 cells a side 10.8M cells in sum 275 / 252, 12.0M 298 / 274,
+// 40.6M 889 / 908; of 48 to 72 9.1M 251 / 285; of 64 to 70 20.0M 603 / 617; of 150 to 192 14.5M 310 / 308, 43.3M 838 / 899.
 constexpr int64_t kFused3D = (int64_t)1 << 23;
 
 int64_t cells_3d(const yee3d_desc& d) { return (int64_t)d.nx * d.ny * d.nz; }
@@ -931,9 +933,9 @@ int32_t launch_multi_batch_2d(const Batch2DArgs& b, int32_t count, hipStream_t s
     return YEE_OK;
 }
 
-// count steps: several a launch when the members allow it; else count launches of the batched bulk-tile kernel (the lean loops) and of the batched edge-tile kernel (the general
-// loops, one wavefront per tile: the many members keep the device busy), each step followed by the members' E_z
-// walls, DFT regions and probes in the single-instance order, then the clocks.
+// count steps: several a launch when the members allow it; else count launches of the batched bulk-tile kernel (the lean
+// loops) and of the batched edge-tile kernel (the general loops, one wavefront per tile: the many members keep the device
+// busy), each step followed by the members' E_z walls, DFT regions and probes in the single-instance order, then the clocks.
 int32_t launch_batch_2d(const Batch2DArgs& b, int32_t count, hipStream_t stream)
 {
     auto bulk = b.lane_columns == 2 ? yee2d_batch_kernel<2, false, false> : yee2d_batch_kernel<4, false, false>;
