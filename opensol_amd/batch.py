@@ -69,7 +69,7 @@ class _Batch:
             engine._ensure_capacity(engine.n_step + count)
             descs[k] = self._cached_descriptor(engine)
             descs[k].step_limit = engine.n_step + count
-            self._adjust(descs[k], sim)
+        self._adjust(descs)
         size = self._bytes(len(self.simulations))
         torch = self.torch
         device = self.simulations[0].engine.device
@@ -84,8 +84,8 @@ class _Batch:
             _lib.check(self.lib.yee_build_graph(self._ctx), 'yee_build_graph')   # capture here, not in launch()
         return longest
 
-    def _adjust(self, desc, sim):
-        """What a member's descriptor owes to the batch it is in."""
+    def _adjust(self, descs):
+        """What the members' descriptors owe to the batch they are in."""
 
     def _cached_descriptor(self, engine):
         """The engine's batch descriptor, rebuilt only when its tables or options change (a chunked caller prepares
@@ -198,11 +198,15 @@ class Batch3D(_Batch):
             d.planes_per_tile = self.planes_per_tile
         return d
 
-    def _adjust(self, desc, sim):
-        # planes tuned for the member alone are no choice for the other step form, which the whole batch's size may ask for
-        form = bool(self.lib.yee3d_fused(sum(self.cell_counts)))
-        if not self.planes_per_tile and getattr(sim, '_planes_fused', form) != form:
-            desc.planes_per_tile = 0
+    def _adjust(self, descs):
+        # planes tuned for a member alone are no choice for the other step form, which the whole batch's size may ask for
+        tuned = [k for k, sim in enumerate(self.simulations) if hasattr(sim, '_planes_fused')]
+        if not tuned or self.planes_per_tile:
+            return
+        fused = bool(self.lib.yee3d_fused(sum(self.cell_counts)))
+        for k in tuned:
+            if self.simulations[k]._planes_fused != fused:
+                descs[k].planes_per_tile = 0
 
     def _options_key(self):
         return self.planes_per_tile
