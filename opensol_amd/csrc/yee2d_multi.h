@@ -140,14 +140,21 @@ __device__ __forceinline__ void store_n(float* __restrict__ p, const float v[VEC
 
 // `v` where `bits` are set, 0 where none are: what a recursion takes where there is no psi. Its factors are 0 there as well,
 // but 0 times an infinite difference is NaN, and an overflowed field stays what the one-step kernels make of it. An AND with
-// bits in a vector register: 300 steps of 1031 x 773 E_z take 0.85 ms so, 0.81 without it, 0.98 with selects on lane masks or
+// bits in a vector register: 300 steps of 1031 x 773 E_z take 0.83 ms so, 0.79 without it, 0.98 with selects on lane masks or
 // scalar branches around the recursions, which the general windows have no scalar registers left for (8192^2 E_z, 40 steps:
-// 2.48, 2.37 and 2.65 ms).
+// 2.39, 2.38 and 2.65 ms). Windows that reach no y layer have forms without its recursions (0.84 and 2.48 ms if they had not;
+// 1370 steps of 270 x 120 cells, periodic along y, 2.16 and 2.26).
 __device__ __forceinline__ float keep_bits(uint32_t bits, float v) { return __uint_as_float(bits & __float_as_uint(v)); }
 __device__ __forceinline__ float keep_bits(float bits, float v) { return keep_bits(__float_as_uint(bits), v); }
+// `v` where `bits` are set, `old` where none are.
+__device__ __forceinline__ float pick_bits(uint32_t bits, float v, float old)
+{
+    return __uint_as_float((bits & __float_as_uint(v)) | (~bits & __float_as_uint(old)));
+}
 
-// Columns of a lane and their y constants; the lean form knows that all of them are inside the grid's bulk.
-template <int VEC, bool EDGE>
+// Columns of a lane and their y constants; the lean form knows that all of them are inside the grid's bulk, and without YL
+// none lies in a y layer.
+template <int VEC, bool EDGE, bool YL>
 struct LaneColumns {
     static_assert(!EDGE || VEC == 1, "general windows hold one column a lane: two beside each other may fold apart");
     int j;                   // first column before folding
@@ -183,7 +190,7 @@ struct LaneColumns {
                 inv_e[k] = d.inv_dy_e[at[k]];
                 inv_h[k] = d.inv_dy_h[at[k]];
                 ry_h[k] = ry_e[k] = -1;
-                if (d.cpml[1].n_rows > 0) {
+                if constexpr (YL) {
                     ry_h[k] = d.cpml[1].row_h[at[k]];
                     ry_e[k] = d.cpml[1].row_e[at[k]];
                 }
@@ -194,20 +201,17 @@ struct LaneColumns {
     // the loads that follow the psi rows of the columns
     __device__ __forceinline__ void constants(const yee2d_desc& d)
     {
-        if constexpr (EDGE) {
+        if constexpr (YL) {
             const yee_cpml_axis& cy = d.cpml[1];
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
                 if (!in[k]) ry_e[k] = -1;
                 if (stays[k]) ry_h[k] = -1;
-                b_h[k] = g_h[k] = b_e[k] = g_e[k] = 0.f;
-                if (cy.n_rows > 0) {
-                    const int h = max(ry_h[k], 0), e = max(ry_e[k], 0);
-                    b_h[k] = cy.b_h[h];
-                    g_h[k] = cy.g_h[h];
-                    b_e[k] = cy.b_e[e];
-                    g_e[k] = cy.g_e[e];
-                }
+                const int h = max(ry_h[k], 0), e = max(ry_e[k], 0);
+                b_h[k] = cy.b_h[h];
+                g_h[k] = cy.g_h[h];
+                b_e[k] = cy.b_e[e];
+                g_e[k] = cy.g_e[e];
             }
         }
     }
@@ -215,7 +219,7 @@ struct LaneColumns {
     // after constants(): 0 for the columns without a psi row
     __device__ __forceinline__ void finish()
     {
-        if constexpr (EDGE) {
+        if constexpr (YL) {
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
                 b_h[k] = ry_h[k] >= 0 ? b_h[k] : 0.f;
@@ -224,9 +228,15 @@ struct LaneColumns {
                 g_e[k] = ry_e[k] >= 0 ? g_e[k] : 0.f;
                 psi_h[k] = ry_h[k] >= 0 ? ~0u : 0u;
                 psi_e[k] = ry_e[k] >= 0 ? ~0u : 0u;
-                moves[k] = stays[k] ? 0u : ~0u;
                 // not lane masks in scalar registers, which are full
-                asm volatile("" : "+v"(psi_h[k]), "+v"(psi_e[k]), "+v"(moves[k]));
+                asm volatile("" : "+v"(psi_h[k]), "+v"(psi_e[k]));
+            }
+        }
+        if constexpr (EDGE) {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                moves[k] = stays[k] ? 0u : ~0u;
+                asm volatile("" : "+v"(moves[k]));
             }
         }
     }
@@ -274,10 +284,10 @@ __device__ __forceinline__ bool stage_multi_tables(const yee2d_desc& d)
 }
 
 // What a window loads first, before its form (FULL or not) and state set are known.
-template <int VEC, int R, bool EDGE>
+template <int VEC, int R, bool EDGE, bool YL>
 struct WindowEarly {
     static constexpr int IDS = VEC == 1 ? VEC : VEC / 2;   // one to a register, or two
-    LaneColumns<VEC, EDGE> col;
+    LaneColumns<VEC, EDGE, YL> col;
     uint32_t ids[R + 1][IDS];    // ids of the rows (H_z: and of the one after them)
     float inv_h, inv_e;          // lane r: x constants of row r (windows with x layers)
     int row_h, row_e;
@@ -290,16 +300,16 @@ struct WindowEarly {
 };
 
 // A window of either polarisation: c is the field at the cell centres (E_z or H_z), fx the one on the hi-y faces (H_x or
-// E_x) and fy the one on the hi-x faces (H_y or E_y). EDGE: the general form; XL: some of its rows lie in an x CPML
+// E_x) and fy the one on the hi-x faces (H_y or E_y). EDGE: the general form; XL, YL: rows, columns of it lie in an x, a y CPML
 // layer; FULL: materials that are not simple (stage_multi_tables). Simple forms keep 1 * x in the updates: exact, and the
 // rounding of each expression stays that of the general one.
-template <int POL, int VEC, int R, int NW, bool EDGE, bool XL, bool FULL, bool EXTRA, bool POLE>
+template <int POL, int VEC, int R, int NW, bool EDGE, bool XL, bool YL, bool FULL, bool EXTRA, bool POLE>
 struct MultiWindow {
     static constexpr bool HZ = POL == YEE_HZ;
-    using Early = WindowEarly<VEC, R, EDGE>;
+    using Early = WindowEarly<VEC, R, EDGE, YL>;
     const yee2d_desc& d;
     const Window& w;
-    LaneColumns<VEC, EDGE> col;
+    LaneColumns<VEC, EDGE, YL> col;
     int wave, q0;            // this wavefront and its first row
     int par;
     int64_t n;               // step count before the launch
@@ -311,7 +321,7 @@ struct MultiWindow {
     // coefficients of the E updates: cb of the cells in cbx (simple E_z); of the E_x and E_y faces (H_z)
     float cax[FULL && HZ ? R : 1][VEC], cay[FULL && HZ ? R : 1][VEC];
     float cbx[HZ || !FULL ? R : 1][VEC], cby[HZ ? R : 1][VEC];
-    float yh[EDGE ? R : 1][VEC], ye[EDGE ? R : 1][VEC], xh[XL ? R : 1][VEC], xe[XL ? R : 1][VEC];
+    float yh[YL ? R : 1][VEC], ye[YL ? R : 1][VEC], xh[XL ? R : 1][VEC], xe[XL ? R : 1][VEC];
     // Drude pole: current of the cells, the rows (bits) and elements (bits) inside its box
     float jp[POLE ? R : 1][VEC];
     uint32_t pole_rows, pole_cols;
@@ -378,14 +388,12 @@ struct MultiWindow {
             col.read(d.field[par][0] + base, c[r]);
             col.read(d.field[par][1] + base, fx[r]);
             col.read(d.field[par][2] + base, fy[r]);
-            if constexpr (EDGE) {
-                if (cy.n_rows > 0) {
-                    const int64_t yrow = (int64_t)f * cy.n_rows;
+            if constexpr (YL) {
+                const int64_t yrow = (int64_t)f * cy.n_rows;
 #pragma unroll
-                    for (int k = 0; k < VEC; ++k) {
-                        yh[r][k] = cy.psi_h[par][yrow + max(col.ry_h[k], 0)];
-                        ye[r][k] = cy.psi_e[par][yrow + max(col.ry_e[k], 0)];
-                    }
+                for (int k = 0; k < VEC; ++k) {
+                    yh[r][k] = cy.psi_h[par][yrow + max(col.ry_h[k], 0)];
+                    ye[r][k] = cy.psi_e[par][yrow + max(col.ry_e[k], 0)];
                 }
             }
             if constexpr (XL) {
@@ -419,8 +427,10 @@ struct MultiWindow {
                     fx[r][k] = cell ? fx[r][k] : 0.f;
                     fy[r][k] = cell ? fy[r][k] : 0.f;
                     if constexpr (!HZ) ids[r][k] = cell ? ids[r][k] : (uint32_t)d.n_materials;   // the zero entry
-                    yh[r][k] = cell && col.ry_h[k] >= 0 ? yh[r][k] : 0.f;
-                    ye[r][k] = cell && col.ry_e[k] >= 0 ? ye[r][k] : 0.f;
+                    if constexpr (YL) {
+                        yh[r][k] = cell && col.ry_h[k] >= 0 ? yh[r][k] : 0.f;
+                        ye[r][k] = cell && col.ry_e[k] >= 0 ? ye[r][k] : 0.f;
+                    }
                     if constexpr (XL) {
                         xh[r][k] = cell && ph[r] >= 0 ? xh[r][k] : 0.f;
                         xe[r][k] = cell && pe[r] >= 0 ? xe[r][k] : 0.f;
@@ -561,9 +571,11 @@ struct MultiWindow {
                 }
                 fy[r][k] = (stays >> r) & 1 ? fy[r][k] : v;
                 float u = ez_hx(m, fx[r][k], de_y, col.inv_h[k], false, 0.f, 0.f, 0.f, &unused);
-                yh[r][k] = col.b_h[k] * yh[r][k] + col.g_h[k] * keep_bits(col.psi_h[k], de_y);
-                u -= m.w * yh[r][k];
-                fx[r][k] = col.stays[k] ? fx[r][k] : u;
+                if constexpr (YL) {
+                    yh[r][k] = col.b_h[k] * yh[r][k] + col.g_h[k] * keep_bits(col.psi_h[k], de_y);
+                    u -= m.w * yh[r][k];
+                }
+                fx[r][k] = pick_bits(col.moves[k], u, fx[r][k]);
             } else {
                 fy[r][k] = ez_hy(m, fy[r][k], de_x, idx, false, 0.f, 0.f, 0.f, &unused);
                 fx[r][k] = ez_hx(m, fx[r][k], de_y, idy, false, 0.f, 0.f, 0.f, &unused);
@@ -587,7 +599,7 @@ struct MultiWindow {
                 xe[r][k] = x.y * xe[r][k] + x.z * keep_bits(x.w, dhy);
                 v += m.y * xe[r][k];
             }
-            if constexpr (EDGE) {
+            if constexpr (YL) {
                 ye[r][k] = col.b_e[k] * ye[r][k] + col.g_e[k] * keep_bits(col.psi_e[k], dhx);
                 v -= m.y * ye[r][k];
             }
@@ -622,7 +634,7 @@ struct MultiWindow {
                 xe[r][k] = x.y * xe[r][k] + x.z * keep_bits(x.w, dey);
                 c[r][k] -= m.y * xe[r][k];
             }
-            if constexpr (EDGE) {
+            if constexpr (YL) {
                 ye[r][k] = col.b_e[k] * ye[r][k] + col.g_e[k] * keep_bits(col.psi_e[k], dex);
                 c[r][k] += m.y * ye[r][k];
             }
@@ -639,7 +651,7 @@ struct MultiWindow {
             float dh = right(c[r], k, next) - c[r][k];
             if constexpr (EDGE) dh = keep_bits(col.moves[k], dh);
             fx[r][k] = hz_ex(FULL ? cax[FULL ? r : 0][k] : 1.f, cbx[r][k], fx[r][k], dh, EDGE ? col.inv_h[k] : idy);
-            if constexpr (EDGE) {
+            if constexpr (YL) {
                 yh[r][k] = col.b_h[k] * yh[r][k] + col.g_h[k] * keep_bits(col.psi_h[k], dh);
                 fx[r][k] += cbx[r][k] * yh[r][k];
             }
@@ -923,17 +935,17 @@ struct MultiWindow {
             store_n<VEC>(d.field[out][0] + base, c[r]);
             store_n<VEC>(d.field[out][1] + base, fx[r]);
             store_n<VEC>(d.field[out][2] + base, fy[r]);
-            if constexpr (EDGE) {
+            if constexpr (YL) {
                 const int64_t yrow = (int64_t)q * cy.n_rows;
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) {
                     if (col.ry_h[k] >= 0 && !col.last[k]) cy.psi_h[out][yrow + col.ry_h[k]] = yh[r][k];
                     if (col.ry_e[k] >= 0) cy.psi_e[out][yrow + col.ry_e[k]] = ye[r][k];
                 }
-                if constexpr (XL) {
-                    if (ph[r] >= 0 && q < d.nx - 1) store_n<VEC>(cx.psi_h[out] + (int64_t)ph[r] * d.pitch + col.j, xh[r]);
-                    if (pe[r] >= 0) store_n<VEC>(cx.psi_e[out] + (int64_t)pe[r] * d.pitch + col.j, xe[r]);
-                }
+            }
+            if constexpr (XL) {
+                if (ph[r] >= 0 && q < d.nx - 1) store_n<VEC>(cx.psi_h[out] + (int64_t)ph[r] * d.pitch + col.j, xh[r]);
+                if (pe[r] >= 0) store_n<VEC>(cx.psi_e[out] + (int64_t)pe[r] * d.pitch + col.j, xe[r]);
             }
         }
     }
@@ -1064,14 +1076,14 @@ struct MultiWindow {
 
 // One window of `steps` steps: a first round of loads with the tables among them, the choice of the form, a second round
 // behind the first one's results, the steps and the stores. The two rounds are what a launch waits for before it steps.
-template <int POL, int VEC, int R, int NW, bool EDGE, bool XL, bool EXTRA>
+template <int POL, int VEC, int R, int NW, bool EDGE, bool XL, bool YL, bool EXTRA>
 __device__ __forceinline__ void run_window(const yee2d_desc& d, const Window& w, int64_t clock, int32_t offset,
                                            int32_t launch, int steps)
 {
     WindowRecords records = window_records(d, w, 64 * VEC);
     if constexpr (EXTRA) records.regions = window_regions(d, w);
-    WindowEarly<VEC, R, EDGE> early;
-    MultiWindow<POL, VEC, R, NW, EDGE, XL, false, EXTRA, false>::early(d, w, early);
+    WindowEarly<VEC, R, EDGE, YL> early;
+    MultiWindow<POL, VEC, R, NW, EDGE, XL, YL, false, EXTRA, false>::early(d, w, early);
     const bool odd = stage_multi_tables<POL, NW>(d);
     clock = (int64_t)__builtin_amdgcn_readfirstlane((int)(clock >> 32)) << 32 |
             (uint32_t)__builtin_amdgcn_readfirstlane((int)clock);
@@ -1085,20 +1097,20 @@ __device__ __forceinline__ void run_window(const yee2d_desc& d, const Window& w,
     if constexpr (EXTRA && POL == YEE_EZ) {
         if (window_pole(d, w, 64 * VEC)) {
             if (full) {
-                MultiWindow<POL, VEC, R, NW, EDGE, XL, true, true, true> window(d, w);
+                MultiWindow<POL, VEC, R, NW, EDGE, XL, YL, true, true, true> window(d, w);
                 run(window);
             } else {
-                MultiWindow<POL, VEC, R, NW, EDGE, XL, false, true, true> window(d, w);
+                MultiWindow<POL, VEC, R, NW, EDGE, XL, YL, false, true, true> window(d, w);
                 run(window);
             }
             return;
         }
     }
     if (full) {
-        MultiWindow<POL, VEC, R, NW, EDGE, XL, true, EXTRA, false> window(d, w);
+        MultiWindow<POL, VEC, R, NW, EDGE, XL, YL, true, EXTRA, false> window(d, w);
         run(window);
     } else {
-        MultiWindow<POL, VEC, R, NW, EDGE, XL, false, EXTRA, false> window(d, w);
+        MultiWindow<POL, VEC, R, NW, EDGE, XL, YL, false, EXTRA, false> window(d, w);
         run(window);
     }
 }
@@ -1128,18 +1140,25 @@ __device__ __forceinline__ void multi_block(const yee2d_desc& d, const yee2d_mul
     w.k0 = w.c0 - yee2d_multi_halo(t, tall ? TV : VEC);
     if constexpr (TR > 0) {
         if (tall) {
-            run_window<POL, TV, TR, NW, false, false, EXTRA>(d, w, clock, offset, launch, steps);
+            run_window<POL, TV, TR, NW, false, false, false, EXTRA>(d, w, clock, offset, launch, steps);
             return;
         }
     }
+    // layers of an axis without psi rows have none to step
+    const bool x_layers = d.cpml[0].n_rows > 0 && (w.w0 < d.layer_x_lo || w.w0 + w.rows > d.layer_x_hi);
+    const bool y_layers = d.cpml[1].n_rows > 0 && (w.k0 < d.layer_y_lo || w.k0 + columns > d.layer_y_hi);
     const bool lean = w.w0 >= 0 && w.w0 >= d.layer_x_lo && w.w0 + w.rows < d.nx && w.w0 + w.rows <= d.layer_x_hi &&
                       w.k0 >= 0 && w.k0 >= d.layer_y_lo && w.k0 + columns < d.ny && w.k0 + columns <= d.layer_y_hi;
     if (lean)
-        run_window<POL, VEC, R, NW, false, false, EXTRA>(d, w, clock, offset, launch, steps);
-    else if (d.cpml[0].n_rows == 0 || (w.w0 >= d.layer_x_lo && w.w0 + w.rows <= d.layer_x_hi))
-        run_window<POL, VEC, R, NW, true, false, EXTRA>(d, w, clock, offset, launch, steps);
+        run_window<POL, VEC, R, NW, false, false, false, EXTRA>(d, w, clock, offset, launch, steps);
+    else if (x_layers && y_layers)
+        run_window<POL, VEC, R, NW, true, true, true, EXTRA>(d, w, clock, offset, launch, steps);
+    else if (x_layers)
+        run_window<POL, VEC, R, NW, true, true, false, EXTRA>(d, w, clock, offset, launch, steps);
+    else if (y_layers)
+        run_window<POL, VEC, R, NW, true, false, true, EXTRA>(d, w, clock, offset, launch, steps);
     else
-        run_window<POL, VEC, R, NW, true, true, EXTRA>(d, w, clock, offset, launch, steps);
+        run_window<POL, VEC, R, NW, true, false, false, EXTRA>(d, w, clock, offset, launch, steps);
 }
 
 }  // namespace yee
