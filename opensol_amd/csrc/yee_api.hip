@@ -467,6 +467,8 @@ bool multi_ok(const yee2d_desc& d, bool extra)
     const int ids = d.polarization == YEE_EZ ? kMultiIds : kMultiIds / 2;   // H_z keeps two entries an id
     if (d.n_tfsf != 0 || has_walls(d) || d.n_materials >= ids) return false;
     if (d.periodic_x && d.cpml[0].n_rows > 0) return false;   // the windows do not wrap the x layers' rows
+    // without CPML rows along x the windows take the bulk spacing everywhere, the one-step kernels the arrays in the layer bounds
+    if (d.cpml[0].n_rows == 0 && (d.layer_x_lo > 0 || d.layer_x_hi < d.nx)) return false;
     if (!extra) return d.n_poles == 0 && d.n_dft == 0 && d.probes.n_probes == 0;
     if (d.n_poles > 1 || d.probes.n_probes > kMultiProbes) return false;
     if (d.n_poles == 1 && (d.polarization != YEE_EZ || d.pole[0].kind != YEE_DRUDE || !d.pole[0].state[1])) return false;

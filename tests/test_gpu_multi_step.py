@@ -293,3 +293,27 @@ def test_periodic_axis_with_layers(gpu, pol, axis):
     a, b = (arrays(sim, 20) for sim in sims)
     for name in a:
         assert bool((a[name] == b[name]).all()), name
+
+
+@pytest.mark.parametrize('pol', ['ez', 'hz'])
+@pytest.mark.parametrize('axis', ['x', 'y'])
+def test_uneven_spacings_without_layers(gpu, pol, axis):
+    """A descriptor whose layer bounds leave no bulk along an axis takes its spacings from the arrays, with or without CPML."""
+    import ctypes
+    from opensol_amd import _lib
+    sims = [build(pol, 129, 130, 'periodic', 'lossy') for _ in range(2)]
+    for sim in sims:
+        d = sim.engine.descriptor()
+        n = getattr(d, f'n{axis}')
+        torch = sim.engine.torch
+        stretch = torch.linspace(0.7, 1.0, n, device=sim.engine.device)
+        sim.spacings = [t * stretch for t in sim.engine.inv[0 if axis == 'x' else 2:][:2]]
+        for name, t in zip(('e', 'h'), sim.spacings):
+            setattr(d, f'inv_d{axis}_{name}', t.data_ptr())
+        setattr(d, f'layer_{axis}_lo', n)
+        _lib.check(sim.engine.lib.yee2d_update(sim.engine._ctx, ctypes.byref(d)), 'yee2d_update')
+    sims[0].engine.step(20)
+    sims[1].engine.step_timed(20)
+    a, b = (arrays(sim, 20) for sim in sims)
+    for name in a:
+        assert bool((a[name] == b[name]).all()), name

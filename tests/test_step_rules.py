@@ -69,6 +69,17 @@ def test_layers_of_a_periodic_x_axis_are_stepped_one_launch_at_a_time(lib):
     assert steps_per_launch(lib, d, 100) > 3
 
 
+def test_spacings_of_layer_bounds_without_cpml_are_stepped_one_launch_at_a_time(lib):
+    d = descriptor(300, 257)
+    d.layer_y_lo = 257
+    assert steps_per_launch(lib, d, 100) > 3
+    for lo, hi in ((300, 300), (0, 0), (5, 300)):
+        d.layer_x_lo, d.layer_x_hi = lo, hi
+        assert steps_per_launch(lib, d, 100) == 1
+    layers(d, 0, 16)
+    assert steps_per_launch(lib, d, 100) > 3
+
+
 @pytest.mark.parametrize('nx,ny,several', [(2, 2_000_000_000, False), (2, 300_000_000, True), (100_000, 100_000, True)])
 @pytest.mark.parametrize('pol', ['ez', 'hz'])
 def test_grids_with_more_windows_than_a_launch_holds_step_one_launch_at_a_time(lib, pol, nx, ny, several):
