@@ -418,7 +418,7 @@ def run_3d(args, torch):
     sim = build_3d_workload(graph_steps=args.graph_steps, planes_per_tile=args.planes_per_tile)
     sim.finalize()
     engine = sim.engine
-    rows_per_tile, planes_per_tile = engine.launch_geometry()
+    planes_per_tile = engine.launch_geometry()[1]
     cells = sim.model.cell_count
     print(f'# workload ready: {sim.model.shape}, {len(sim.model.materials.materials)} materials, '
           f'm = {sim.model.sample_interval}', file=sys.stderr, flush=True)
@@ -452,8 +452,7 @@ def run_3d(args, torch):
               **_common_fields(args, value, per_step),
               'data': 'synthetic (seeded boxes, Gaussian point dipole, two flux planes)',
               'config': {'workload': workload, 'grid': list(sim.model.shape), 'cpml': 12, 'dx_m': 25e-9, 'boxes': 200,
-                         'seed': SEED, 'graph_steps': args.graph_steps, 'rows_per_tile': rows_per_tile,
-                         'planes_per_tile': planes_per_tile, 'sample_interval': sim.model.sample_interval},
+                         'seed': SEED, 'graph_steps': args.graph_steps, 'planes_per_tile': planes_per_tile, 'sample_interval': sim.model.sample_interval},
               'roofline': roofline, 'cpu_baseline': baseline}
     return result
 
